@@ -18,43 +18,63 @@ struct BlockDesc {
     double epsm1_plate;  // ε(iξ)-1 of the plate (+inf: perfect reflector)
     double epsm1_sphere; // ε(iξ)-1 of the sphere
     double LbyR;
-    int m, lmin, ldim, N;   // N = 2 ldim, window l in [lmin, lmin+ldim)
+    int m, lmin, ldim;      // window l in [lmin, lmin+ldim)
+    int N;                  // dimension of the matrix to factor (k_wave_window
+                            // sets it for the dense form of a Gram matrix)
     int is_pr;              // plate is a perfect reflector: I_TE = -|I_TM|
-    // K_ν table: ν in [mu, nu_max]
-    int mu, nu_max, nK;
-    // I table: l in [lo, lo+nl)
-    int lo, nl;
-    // quadrature grid of the K integrals: v_k = v0 + k h, k < n_nodes,
-    // x(v) = 1 + A² softplus(v)²
+    // quadrature grid: v_k = v0 + k h, k < n_nodes, x(v) = 1 + A² softplus(v)²
+    // (of the wave-number factor, or of the K integrals of the tables)
     double v0, h, A;
-    int n_nodes, n_waves;
-    // matrix
-    int lda;
-    int pad_;
-    // byte offsets into the arena
-    int64_t off_mie;    // 4 * ldim doubles: log|a_l|, log|b_l|, then the mantissas
-                        // of e^{ea(l)}, e^{eb(l)}; then 2 * ldim int exponents;
-                        // then nl + (2 nl - 1) doubles: parts of log a0 of I
+    int n_nodes, n_waves;   // n_waves: wavefronts of 64 nodes
+    int n_chunks;           // runs of 16 degrees of the window
+    int mie_L;              // degrees 1 .. mie_L of the block's Mie table
+    // K and I tables (caps_integrate_init): ν in [mu, nu_max], l in [lo, lo+nl)
+    int mu, nu_max, nK;
+    int lo, nl;
+    int lda;                // leading dimension of the matrix, if there is one
+    // byte offsets into the arena; nP = 64 n_waves
+    int64_t off_mie;    // the block's MieDesc table
+    int64_t off_node;   // 3 nP doubles: x, √r_TM, √|r_TE|
+    int64_t off_ck;     // n_chunks nP double2: S_l, S_{l-1} at each chunk's start, then
+                        // n_chunks nP ints: their exponents
+    int64_t off_norm;   // n_chunks nP doubles: squared norms of the rows' chunks
+    int64_t off_act;    // n_chunks nP/8 ints: exponent of a tile's largest of them
+    int64_t off_dn;     // nP doubles: squared norms of the rows
+    int64_t off_rows;   // F: 32 n_chunks rows (degree; a_l, b_l) of 2 nP doubles
+    int64_t off_band;   // nP/8 columns of BAND_TILES tiles of 16 x 16: -G
+    int64_t off_part;   // GRAM_SPLIT such bands: partial sums
+    int64_t off_a0;     // nl + (2 nl - 1) doubles: parts of log a0 of I
     int64_t off_kpart;  // n_waves * nK * KPart
     int64_t off_k;      // 2 pols * nK * KEnt (K = m * 2^e), then 2 pols * nK
                         // doubles log|K|
     int64_t off_i;      // I = mant * 2^exp: 2 pols * nl*nl signed double mantissas,
                         // then 2 pols * nl*nl int exponents
     int64_t off_mat;    // lda * N doubles (column-major)
-    int64_t off_diag;   // N doubles: diagonal of M
-    int64_t off_piv;    // N ints: LU pivots
+    int64_t off_diag;   // N doubles: diagonal of M (or G)
     int64_t off_cpart;  // n_rtiles x N doubles: per row tile, the column sums
                         // of |M_ij| over i != j (written with the matrix)
     int n_rtiles;       // row tiles of off_cpart (0: none)
-    int pad2_;
+    int pad_;
 };
 
-// Blocks whose I tables share the coefficients a_q: same m, ℓ-window and
-// polarizations (the blocks of one m at several frequencies).
-constexpr int IG_MAX = 8;
-struct IGroup {
-    int count;
-    int blk[IG_MAX];
+// The band of G: tiles on and below the diagonal per column of 16 x 16 tiles
+// (8 nodes each).  Rows of F fall off like e^{-δ²/16} in the distance δ = h
+// times the node distance, and G_ij enters the determinant squared: what lies
+// more than 48 nodes (δ = 24) apart changes it by less than 1e-16 of its
+// value, the tail of x -> 1 of the smallest m included (scanned over R/L
+// 0.1 .. 1000, ξ 1e-3 .. 300, both materials: no difference to the full
+// matrix above 1e-15).
+constexpr int BAND_TILES = 7;
+constexpr int GRAM_SPLIT = 8;    // runs of chunks summed apart (k_gram)
+constexpr int MAX_CHUNKS = 768;  // ldim <= 12288
+
+// One Mie table: degrees 1 .. L at one ξ of one object; at off: L doubles each
+// of log|a_l|, log|b_l| and the mantissas of √(a_l g_l), √(b_l g_l), g_l =
+// (2l+1)/(l(l+1)), over a common power of two, then L ints: its exponent.
+struct MieDesc {
+    double xi_, LbyR, epsm1;
+    int64_t off;
+    int L, pad_;
 };
 
 // Partial K sums of one wave of quadrature nodes for one ν.
@@ -89,6 +109,9 @@ struct BlockOut {
                         // runs without pivot search on u = 1 + d, summing
                         // log1p(d); 0: the matrix holds 1 - M (or a user
                         // matrix), LU with partial pivoting
+    int tile0, tiles;   // the nodes that matter: tiles of 8 nodes (G has
+                        // 16 tiles rows)
+    int etr, emin;      // exponent of the trace; of the smallest row chunk kept
     int pad_;
 };
 

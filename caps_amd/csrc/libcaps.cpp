@@ -3,8 +3,9 @@
 // One device context per caps_t (stream, events, a growable HBM arena,
 // pinned staging buffers), created on the first GPU call.  A batch of
 // (ξ, m) blocks is laid out in the arena (BlockDesc offsets), the pipeline
-// Mie -> K -> I -> assemble(1-M) -> trace -> LU runs asynchronously on the
-// context's stream, and only the per-block scalars come back.  The
+// Mie and nodes -> row norms -> trace and window -> rows -> Gram matrix -> LU
+// runs asynchronously on the context's stream, and only the per-block scalars
+// come back.  The
 // determinant shortcuts of the reference (src/matrix.c:78-82, 144-145,
 // 494-505) are applied to those scalars on the host.
 #include <dlfcn.h>
@@ -29,17 +30,22 @@
 using capsd::BlockDesc;
 using capsd::BlockOut;
 using capsd::KPart;
-using capsd::IG_MAX;
-using capsd::IGroup;
+using capsd::MieDesc;
 
 struct capsx_mlp;
 extern "C" {
 void capsx_mlp_predict(capsx_mlp* h, const float* X, int n, float* Y);
-void capsd_launch_mie(const BlockDesc*, char*, const double*, int, int, hipStream_t);
-void capsd_launch_K(const BlockDesc*, char*, const double*, int, int, int, int, int*, hipStream_t);
-void capsd_launch_I(const BlockDesc*, char*, const void*, const int*, const double*, int64_t, int*, const BlockOut*,
-                    int, int, hipStream_t);
-void capsd_launch_assemble(const BlockDesc*, char*, const double*, int, int, int, const BlockOut*, int, hipStream_t);
+void capsd_launch_wave_start(const void*, int, int, const BlockDesc*, char*, int, int, int*, hipStream_t);
+void capsd_launch_wave_norms(const BlockDesc*, char*, const BlockOut*, int, int, hipStream_t);
+void capsd_launch_wave_window(BlockDesc*, char*, BlockOut*, const int*, int, int, int, hipStream_t);
+void capsd_launch_wave_rows(const BlockDesc*, char*, const BlockOut*, int, int, int, hipStream_t);
+void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, hipStream_t);
+void capsd_launch_band_ldl(const BlockDesc*, char*, BlockOut*, int, int, hipStream_t);
+void capsd_launch_band_dense(const BlockDesc*, char*, const BlockOut*, int, int, int, hipStream_t);
+void capsd_launch_wave_matrix(const BlockDesc*, char*, const BlockOut*, int, int, int, int, hipStream_t);
+void capsd_launch_a0(const BlockDesc*, char*, const double*, int, hipStream_t);
+void capsd_launch_K(const BlockDesc*, char*, const double*, int, int, int, int*, hipStream_t);
+void capsd_launch_I(const BlockDesc*, char*, int, int, int*, hipStream_t);
 void capsd_launch_trace(const BlockDesc*, char*, BlockOut*, int, int, hipStream_t);
 void capsd_launch_dominance(const BlockDesc*, char*, BlockOut*, int, int, int, hipStream_t);
 void capsd_launch_frobenius(const BlockDesc*, char*, BlockOut*, int, int, hipStream_t);
@@ -109,7 +115,6 @@ void device_init()
 }
 
 constexpr int MAX_LU_STREAMS = 4;
-constexpr int MAX_PARTS = MAX_LU_STREAMS;   // parts of a batch (BatchPlan)
 
 struct Ctx {
     hipStream_t stream = nullptr;
@@ -118,20 +123,19 @@ struct Ctx {
     // that one group's panel factorizations overlap another's updates
     hipStream_t lu_stream[MAX_LU_STREAMS];
     hipEvent_t lu_done[MAX_LU_STREAMS];
-    hipEvent_t part_i_done[MAX_PARTS];   // part g's I finished
-    hipEvent_t lu_ready = nullptr;        // a one-part batch's matrices assembled
-    hipEvent_t head_fork = nullptr;       // a batch's start, for the Mie kernel's stream
-    hipEvent_t mie_done = nullptr;        // the batch's Mie coefficients written
+    hipEvent_t lu_ready = nullptr;        // a batch's dense matrices written
     char* arena = nullptr;
     size_t arena_size = 0;
-    BlockDesc* d_desc = nullptr;
+    // what a batch uploads, in one copy: the status word (zero), the block
+    // descriptors and right behind those in use the Mie tables' descriptors
+    char* d_up = nullptr;
+    char* h_up = nullptr;         // pinned
+    int* d_status = nullptr;      // = d_up
+    BlockDesc* d_desc = nullptr;  // in d_up
     LuSide* d_side = nullptr;
     BlockOut* d_out = nullptr;
-    int* d_status = nullptr;
-    IGroup* d_groups = nullptr;
-    IGroup* h_groups = nullptr;
     int cap_blocks = 0;
-    BlockDesc* h_desc = nullptr;  // pinned
+    BlockDesc* h_desc = nullptr;  // in h_up
     LuSide* h_side = nullptr;
     BlockOut* h_out = nullptr;
     int* h_status = nullptr;
@@ -140,7 +144,7 @@ struct Ctx {
     size_t pts_bytes = 0;
     double timing[6] = {0, 0, 0, 0, 0, 0};
     // accumulated since capsx_stats_reset: stage ms [0..5], blocks, blocks
-    // factored (not skipped), algorithmic LU flops, batches, I pairs, and
+    // factored (not skipped), LU flops, batches, I pairs of tables, and
     // with profiling on the trailing update's ms, flops, launches, bytes
     double acc[16] = {};
     // per-launch timing of the LU's trailing-update kernel (capsx_profile)
@@ -182,11 +186,7 @@ Ctx* ctx_of(caps_t* self)
             HIPCHECK(hipStreamCreateWithFlags(&c->lu_stream[g], hipStreamNonBlocking));
             HIPCHECK(hipEventCreateWithFlags(&c->lu_done[g], hipEventDisableTiming));
         }
-        for (auto& e : c->part_i_done) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         HIPCHECK(hipEventCreateWithFlags(&c->lu_ready, hipEventDisableTiming));
-        HIPCHECK(hipEventCreateWithFlags(&c->head_fork, hipEventDisableTiming));
-        HIPCHECK(hipEventCreateWithFlags(&c->mie_done, hipEventDisableTiming));
-        HIPCHECK(hipMalloc(&c->d_status, sizeof(int)));
         HIPCHECK(hipHostMalloc((void**)&c->h_status, sizeof(int), hipHostMallocDefault));
         self->priv = c;
     }
@@ -198,16 +198,13 @@ void ctx_free(Ctx* c)
     if (!c) return;
     hipStreamSynchronize(c->stream);
     if (c->arena) hipFree(c->arena);
-    if (c->d_desc) hipFree(c->d_desc);
+    if (c->d_up) hipFree(c->d_up);
     if (c->d_side) hipFree(c->d_side);
     if (c->d_out) hipFree(c->d_out);
-    if (c->d_status) hipFree(c->d_status);
-    if (c->h_desc) hipHostFree(c->h_desc);
+    if (c->h_up) hipHostFree(c->h_up);
     if (c->h_side) hipHostFree(c->h_side);
     if (c->h_out) hipHostFree(c->h_out);
     if (c->h_status) hipHostFree(c->h_status);
-    if (c->d_groups) hipFree(c->d_groups);
-    if (c->h_groups) hipHostFree(c->h_groups);
     if (c->pts) hipFree(c->pts);
     for (auto& e : c->ev) hipEventDestroy(e);
     for (auto& e : c->gemm_ev) hipEventDestroy(e);
@@ -216,35 +213,35 @@ void ctx_free(Ctx* c)
         hipStreamDestroy(c->lu_stream[g]);
         hipEventDestroy(c->lu_done[g]);
     }
-    for (auto& e : c->part_i_done) hipEventDestroy(e);
     hipEventDestroy(c->lu_ready);
-    hipEventDestroy(c->head_fork);
-    hipEventDestroy(c->mie_done);
     hipStreamDestroy(c->stream);
     delete c;
 }
+
+constexpr size_t UP_HEAD = 256;   // the status word's share of d_up
 
 void ensure_blocks(Ctx* c, int n)
 {
     if (n <= c->cap_blocks) return;
     const int cap = std::max(n, 2 * c->cap_blocks);
-    if (c->d_desc) {
+    if (c->d_up) {
         HIPCHECK(hipStreamSynchronize(c->stream));
-        hipFree(c->d_desc);
+        hipFree(c->d_up);
         hipFree(c->d_side);
         hipFree(c->d_out);
-        hipHostFree(c->h_desc);
+        hipHostFree(c->h_up);
         hipHostFree(c->h_side);
         hipHostFree(c->h_out);
-        hipFree(c->d_groups);
-        hipHostFree(c->h_groups);
     }
-    HIPCHECK(hipMalloc(&c->d_desc, cap * sizeof(BlockDesc)));
-    HIPCHECK(hipMalloc(&c->d_groups, cap * sizeof(IGroup)));
-    HIPCHECK(hipHostMalloc((void**)&c->h_groups, cap * sizeof(IGroup), hipHostMallocDefault));
+    const size_t up = UP_HEAD + cap * (sizeof(BlockDesc) + sizeof(MieDesc));
+    HIPCHECK(hipMalloc(&c->d_up, up));
+    HIPCHECK(hipHostMalloc((void**)&c->h_up, up, hipHostMallocDefault));
+    memset(c->h_up, 0, UP_HEAD);
+    c->d_status = (int*)c->d_up;
+    c->d_desc = (BlockDesc*)(c->d_up + UP_HEAD);
+    c->h_desc = (BlockDesc*)(c->h_up + UP_HEAD);
     HIPCHECK(hipMalloc(&c->d_side, cap * sizeof(LuSide)));
     HIPCHECK(hipMalloc(&c->d_out, cap * sizeof(BlockOut)));
-    HIPCHECK(hipHostMalloc((void**)&c->h_desc, cap * sizeof(BlockDesc), hipHostMallocDefault));
     HIPCHECK(hipHostMalloc((void**)&c->h_side, cap * sizeof(LuSide), hipHostMallocDefault));
     HIPCHECK(hipHostMalloc((void**)&c->h_out, cap * sizeof(BlockOut), hipHostMallocDefault));
     c->cap_blocks = cap;
@@ -510,200 +507,208 @@ void grid_for(BlockDesc& d)
     d.n_waves = (d.n_nodes + 63) / 64;
 }
 
-// A batch runs as `parts` parts, contiguous block ranges [part_b[g],
-// part_b[g+1]) (the LU stream groups): part g's I, assembly and LU run in
-// order on stream g, and part g's I starts when part g-1's I is done, so
-// the I of one part runs beside the assembly and LU of the part before it
-// (measured on the C2 batch: 2 parts 0.295 s per step, against 0.302 s
-// with the parts' I run together; one stream computing every part's I
-// while a second factored the parts in turn was slower, 0.31-0.44 s for
-// 2-8 parts).
-struct BatchPlan {
-    int n = 0, maxN = 0, minN = 0, max_ldim = 0, max_waves = 0, max_nK = 0, max_nl = 0;
-    int sum_waves = 0;   // K quadrature waves over the batch's blocks
-    int64_t max_ntri = 0;
-    size_t bytes = 0;
-    std::vector<IGroup> groups;   // per part, ordered by class (see build_igroups)
-    int parts = 1;
-    int part_b[MAX_PARTS + 1] = {};
-    int part_goff[MAX_PARTS] = {};      // first I group of each part
-    int part_cls[MAX_PARTS][8] = {};    // I groups per class of each part
-    // determinant forms the LU launches kernels for (capsd_launch_lu kinds):
-    // 2 = delta form only (round-trip blocks; one that turns out not column
-    // dominant is left unfactored and run again with 1 = pivoted), 6 = the
-    // same in the symmetric form (1 - M of a round trip is symmetric: the
-    // reference factors it as such, sym_spd in src/libcaps.c:954)
-    int lu_kinds = 2;
-};
-
-// Groups of blocks [b0, b1) that share the I coefficients a_q: same caps
-// object, m, ℓ-window and polarizations, at most IG_MAX per group; appended
-// to p.groups by class, the class sizes in cls.
-void build_igroups(caps_t* const* objs, const BlockDesc* desc, int b0, int b1, BatchPlan& p, int* cls_count)
+// Quadrature grid of the wave-number factor (k_wave_start): the same map with
+// step 0.5, at which the determinants agree with those of a much finer grid
+// to 2e-14 (scanned over R/L 0.1 .. 1000, ξ 1e-3 .. 300, small and large m,
+// both materials; 0.45: 2.0e-14, 0.55: 5.6e-14, 0.6: 1.0e-12), up to where the
+// integrand of the largest degree has fallen by e^{-50} from its peak.
+void wave_grid_for(BlockDesc& d)
 {
-    const int n = b1 - b0;
-    std::vector<int> idx(n);
-    for (int i = 0; i < n; i++) idx[i] = b0 + i;
-    auto key = [&](int i) {
-        const BlockDesc& d = desc[i];
-        return std::make_tuple(1 - d.is_pr, (uintptr_t)objs[i], d.m, d.lmin, d.ldim);
-    };
-    std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return key(x) < key(y); });
-    // classes: perfect reflector (TM only) or both polarizations, times at
-    // most 1, 2, 4 or 8 blocks; the kernel is instantiated per class
-    std::vector<IGroup> cls[8];
-    // at most 8 blocks per group (k_I keeps a chunk of a_q and every sum in
-    // registers: 125 VGPRs for 8 blocks with both polarizations, 4 waves
-    // per SIMD); a run of r blocks with one key is cut into ceil(r/8) groups
-    // of near-equal size, consecutive in the input order (in a free energy
-    // neighbouring frequencies, whose sums take similar numbers of terms).
-    // CAPS_AMD_IGROUP_MAX lowers the maximum.
-    static const int genv = (int)env_double("CAPS_AMD_IGROUP_MAX", 0);
-    const int gmax = std::max(1, std::min(IG_MAX, genv > 0 ? genv : IG_MAX));
-    for (int i = 0; i < n;) {
-        int r = 1;
-        while (i + r < n && key(idx[i + r]) == key(idx[i])) r++;
-        const int ng = (r + gmax - 1) / gmax;
-        for (int k = 0, at = i; k < ng; k++) {
-            IGroup g;
-            memset(&g, 0, sizeof(g));
-            g.count = r / ng + (k < r % ng ? 1 : 0);
-            for (int t = 0; t < g.count; t++) g.blk[t] = idx[at + t];
-            at += g.count;
-            const int sc = g.count <= 1 ? 0 : g.count <= 2 ? 1 : g.count <= 4 ? 2 : 3;
-            cls[(desc[idx[i]].is_pr ? 0 : 4) + sc].push_back(g);
-        }
-        i += r;
+    const double alpha = d.alpha, nu = 2.0 * (d.lmin + d.ldim) - 1;
+    const double xp = hypot(1, nu / alpha);
+    auto g = [&](double x) { return nu * acosh(x) - alpha * x; };
+    const double target = g(xp) - 50;
+    double step = 8 * sqrt((xp * xp - 1) / (alpha * xp)) + 1 / alpha, lo = xp, hi = xp + step;
+    for (int i = 0; i < 200 && g(hi) > target; i++) {
+        lo = hi;
+        step *= 1.5;
+        hi = xp + step;
     }
-    for (int k = 0; k < 8; k++) {
-        cls_count[k] = (int)cls[k].size();
-        p.groups.insert(p.groups.end(), cls[k].begin(), cls[k].end());
+    for (int i = 0; i < 4; i++) {
+        const double mid = 0.5 * (lo + hi);
+        (g(mid) > target ? lo : hi) = mid;
     }
+    d.h = 0.5;
+    d.v0 = -19;
+    d.A = 0.5 / sqrt(alpha);
+    const double s = sqrt(std::max(hi - 1, 60 / alpha)) / d.A;
+    const double vhi = s > 30 ? s : log(expm1(s));
+    d.n_nodes = (int)ceil((vhi - d.v0) / d.h) + 1;
+    d.n_waves = (d.n_nodes + 63) / 64;
 }
 
-// Fill descriptors for blocks [0, n) and their arena offsets.
-BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const int* m, int n, int with_lu)
+// What a batch computes.  JOB_PIVOTED: determinants by the pivoted LU, of
+// blocks that a JOB_LOGDET batch left unfactored.
+enum Job { JOB_LOGDET, JOB_PIVOTED, JOB_MATRIX, JOB_TABLES };
+
+// The matrix that a determinant is taken of: the band of the Gram matrix
+// (one kernel per block); the Gram matrix dense, for the LU's kernels
+// (pivoted LU, a schedule fixed by capsx_lu_config, per-launch profiling,
+// CAPS_AMD_LU_SYM=0); M itself, dense (caps_M_init, and CHOLESKY, whose
+// shortcut rule looks at the lower triangle of M).
+enum Form { FORM_BAND, FORM_GRAM, FORM_M };
+
+struct BatchPlan {
+    int n = 0, ntab = 0, maxN = 0, minN = 0, max_ldim = 0, max_waves = 0, max_wq = 0, max_mie = 0;
+    size_t bytes = 0;
+    Job job = JOB_LOGDET;
+    Form form = FORM_BAND;
+    int dmode = 0;      // dense_mode of the determinant
+    int split = 0;      // k_gram's runs of chunks in workgroups of their own
+    // determinant forms the LU launches kernels for (capsd_launch_lu kinds):
+    // 1 = pivoted, 2 = delta form, 6 = delta form of a symmetric matrix
+    int lu_kinds = 6;
+    // K and I tables: waves of the quadrature, entries
+    int sum_waves = 0, max_nK = 0, max_nl = 0;
+};
+
+bool schedule_fixed()
+{
+    std::lock_guard<std::mutex> lock(g_cfg_mu);
+    return g_have_override;
+}
+
+// Descriptors and arena offsets of blocks [0, n), or of the first of them that
+// fit the HBM budget together (p.n, at least one).
+BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const int* m, int n, Job job, int dmode)
 {
     BatchPlan p;
-    p.n = n;
-    // CAPS_AMD_LU_SYM=0: the general (non-symmetric) delta form
-    p.lu_kinds = env_double("CAPS_AMD_LU_SYM", 1) != 0 ? 6 : 2;
-    const int nb = capsd_lu_nb();
+    p.job = job;
+    p.dmode = dmode;
+    p.lu_kinds = job == JOB_PIVOTED ? 1 : env_double("CAPS_AMD_LU_SYM", 1) != 0 ? 6 : 2;
+    const bool det = job == JOB_LOGDET || job == JOB_PIVOTED;
+    p.form = job == JOB_MATRIX || dmode == 2                                            ? FORM_M
+             : job == JOB_PIVOTED || c->prof || p.lu_kinds != 6 || schedule_fixed() ? FORM_GRAM
+                                                                                         : FORM_BAND;
+    const size_t budget = arena_budget();
     int64_t off = 0;
-    double last_xi = NAN, ep = 0, es = 0;
-    caps_t* last_obj = nullptr;
+    auto take = [&](int64_t bytes) {
+        const int64_t o = off;
+        off = align256(off + bytes);
+        return o;
+    };
+    // one Mie table per object and ξ (ε of both bodies evaluated once)
+    struct Key {
+        caps_t* obj;
+        double xi;
+        bool operator==(const Key& o) const { return obj == o.obj && xi == o.xi; }
+    };
+    struct Hash {
+        size_t operator()(const Key& k) const { return std::hash<void*>()(k.obj) * 31 + std::hash<double>()(k.xi); }
+    };
+    struct Tab {
+        double ep, es;
+        int L;
+        int64_t off;
+    };
+    std::unordered_map<Key, int, Hash> index;
+    std::vector<Tab> tabs;
+    std::vector<MieDesc> mds;
+    std::vector<int> tab_of;
+    int64_t strips = 0;
     for (int b = 0; b < n; b++) {
+        const int64_t off0 = off;
         caps_t* self = objs[b];
         const int ldim = self->ldim;
-        const int N = 2 * ldim;
-        const int lda = (N + 15) & ~15;
         BlockDesc& d = c->h_desc[b];
         memset(&d, 0, sizeof(d));
         d.xi_ = xi_[b];
         d.alpha = 2 * xi_[b];
-        if (!(xi_[b] == last_xi) || self != last_obj) {
-            ep = caps_epsilonm1_plate(self, xi_[b]);
-            es = caps_epsilonm1_sphere(self, xi_[b]);
-            last_xi = xi_[b];
-            last_obj = self;
-        }
-        d.epsm1_plate = ep;
-        d.epsm1_sphere = es;
         d.LbyR = self->LbyR;
         d.m = m[b];
         size_t lmin, lmax;
         caps_estimate_lminmax(self, m[b], &lmin, &lmax);
         d.lmin = (int)lmin;
         d.ldim = ldim;
-        d.N = N;
-        d.lda = lda;
-        d.is_pr = std::isinf(caps_epsilonm1_plate(self, INFINITY)) ? 1 : 0;
-        d.mu = m[b] > 0 ? 2 * m[b] : 2;
-        d.lo = d.lmin - 1;
-        d.nl = ldim + 2;
-        d.nu_max = 2 * (d.lo + d.nl - 1);
-        d.nK = d.nu_max - d.mu + 1;
-        grid_for(d);
-        d.off_mie = off;
-        off = align256(off + (5 * (int64_t)ldim + 3 * (int64_t)(ldim + 2)) * 8);
-        d.off_kpart = off;
-        off = align256(off + (int64_t)d.n_waves * d.nK * sizeof(KPart));
-        // K table after a zeroed guard of capsd::K_GUARD entries (k_K_combine):
-        // the I recurrence's chunks read up to 2 (chunk - 1) entries below
-        // index 0 for steps past qmax, whose coefficients are 0
-        d.off_k = off + 256;
-        off = align256(d.off_k + 2 * (int64_t)d.nK * (sizeof(capsd::KEnt) + 8));
-        d.off_i = off;
-        off = align256(off + 2 * (int64_t)d.nl * d.nl * 12);
-        d.off_mat = off;
-        off = align256(off + (int64_t)lda * N * 8);
-        d.off_diag = off;
-        off = align256(off + (int64_t)N * 8);
-        d.off_piv = off;
-        off = align256(off + (int64_t)N * 4);
-        // column sums of |M| per 32-row tile of the assembly (k_assemble),
-        // for the column dominance test of the LU's delta form
-        d.n_rtiles = with_lu ? (ldim + 15) / 16 : 0;
-        d.off_cpart = off;
-        off = align256(off + (int64_t)d.n_rtiles * N * 8);
-        LuSide& s = c->h_side[b];
-        if (with_lu) {
-            off = lu_side_layout(s, off, N, lda);
-        } else
-            s.off_panel = s.off_logs = s.off_moved = s.off_ut = s.off_inv = 0;
-        p.maxN = std::max(p.maxN, N);
-        p.minN = b == 0 ? N : std::min(p.minN, N);
+        const auto at = index.emplace(Key{self, xi_[b]}, (int)tabs.size());
+        if (at.second) {
+            tabs.push_back({caps_epsilonm1_plate(self, xi_[b]), caps_epsilonm1_sphere(self, xi_[b]), 0, 0});
+            MieDesc md;
+            memset(&md, 0, sizeof(md));
+            md.xi_ = xi_[b];
+            md.LbyR = self->LbyR;
+            md.epsm1 = tabs.back().es;
+            mds.push_back(md);
+        }
+        Tab& tab = tabs[at.first->second];
+        d.epsm1_plate = tab.ep;
+        d.epsm1_sphere = tab.es;
+        tab_of.push_back(at.first->second);
+        d.n_chunks = (ldim + 15) / 16;
+        if (job == JOB_TABLES) {
+            d.is_pr = std::isinf(caps_epsilonm1_plate(self, INFINITY)) ? 1 : 0;
+            d.mu = m[b] > 0 ? 2 * m[b] : 2;
+            d.lo = d.lmin - 1;
+            d.nl = ldim + 2;
+            d.nu_max = 2 * (d.lo + d.nl - 1);
+            d.nK = d.nu_max - d.mu + 1;
+            grid_for(d);
+            d.off_a0 = take(3 * (int64_t)d.nl * 8);
+            d.off_kpart = take((int64_t)d.n_waves * d.nK * sizeof(KPart));
+            // K table after a zeroed guard of capsd::K_GUARD entries (k_K_combine):
+            // the I recurrence's chunks read up to 2 (chunk - 1) entries below
+            // index 0 for steps past qmax, whose coefficients are 0
+            d.off_k = take(256 + 2 * (int64_t)d.nK * (sizeof(capsd::KEnt) + 8)) + 256;
+            d.off_i = take(2 * (int64_t)d.nl * d.nl * 12);
+        } else {
+            tab.L = std::max(tab.L, d.lmin + ldim - 1);
+            wave_grid_for(d);
+            const int64_t nP = 64 * (int64_t)d.n_waves, nc = d.n_chunks;
+            d.off_node = take(3 * nP * 8);
+            d.off_ck = take(nc * nP * 20);
+            d.off_norm = take(nc * nP * 8);
+            d.off_act = take(nc * (nP / 8) * 4);
+            d.off_dn = take(nP * 8);
+            d.off_rows = take(32 * nc * 2 * nP * 8);
+            if (p.form != FORM_M) d.off_band = take(nP / 8 * (capsd::BAND_TILES * 256) * 8);
+            // nodes of a block that matter: about 0.8 of them, 32 per strip
+            strips += (d.n_nodes + 39) / 40;
+            d.N = p.form == FORM_M ? 2 * ldim : (int)(2 * nP);
+            d.lda = ((d.N + 15) & ~15) + (p.form == FORM_GRAM ? 16 : 0);
+            if (p.form != FORM_BAND) {
+                d.off_mat = take((int64_t)d.lda * d.N * 8);
+                d.off_diag = take((int64_t)d.N * 8);
+                if (det) off = lu_side_layout(c->h_side[b], off, d.N, d.lda);
+            }
+        }
+        if (b > 0 && (size_t)off > budget) {
+            off = off0;
+            tab_of.pop_back();
+            break;
+        }
+        p.n = b + 1;
+        p.minN = b == 0 ? d.N : std::min(p.minN, d.N);
+        p.maxN = std::max(p.maxN, d.N);
         p.max_ldim = std::max(p.max_ldim, ldim);
         p.max_waves = std::max(p.max_waves, d.n_waves);
+        p.max_wq = std::max(p.max_wq, d.n_waves * ((d.n_chunks + 3) / 4));
         p.sum_waves += d.n_waves;
         p.max_nK = std::max(p.max_nK, d.nK);
-        p.max_ntri = std::max(p.max_ntri, (int64_t)d.nl * (d.nl + 1) / 2);
         p.max_nl = std::max(p.max_nl, d.nl);
     }
+    // a batch whose strips of the band leave the GPU idle (fewer than 1.5 per
+    // CU) splits each into GRAM_SPLIT workgroups (one block, R/L = 200: 7)
+    p.split = det && p.form != FORM_M && strips < 384;
+    if (p.split)
+        for (int b = 0; b < p.n; b++)
+            c->h_desc[b].off_part = take((int64_t)capsd::GRAM_SPLIT * (c->h_desc[b].n_waves * 8) *
+                                         (capsd::BAND_TILES * 256) * 8);
+    if (job != JOB_TABLES) {
+        p.ntab = (int)tabs.size();
+        for (int t = 0; t < p.ntab; t++) {
+            mds[t].L = tabs[t].L;
+            mds[t].off = tabs[t].off = take((int64_t)tabs[t].L * 36);
+            p.max_mie = std::max(p.max_mie, tabs[t].L);
+        }
+        // the tables' descriptors right behind the blocks'
+        memcpy((void*)(c->h_desc + p.n), mds.data(), p.ntab * sizeof(MieDesc));
+        for (int b = 0; b < p.n; b++) {
+            c->h_desc[b].off_mie = tabs[tab_of[b]].off;
+            c->h_desc[b].mie_L = tabs[tab_of[b]].L;
+        }
+    }
     p.bytes = (size_t)off;
-    // parts = LU stream groups of the tuned schedule, at most
-    // CAPS_AMD_PARTS (default 1; one without an LU, and in profiled runs,
-    // which time each update launch alone).  Since the I, K and assembly
-    // kernels and the LU's own kernels got faster, running the I of one
-    // part beside the LU of another no longer pays: C2 step 164.5 ms with
-    // one part, 165.4 ms with two, 165.9 ms with three (the kernels slow
-    // each other down as much as they overlap)
-    p.parts = 1;
-    if (with_lu && !c->prof) {
-        const int cap = std::max(1, (int)env_double("CAPS_AMD_PARTS", 1));
-        p.parts = std::max(1, std::min(std::min(lu_config(p.maxN, n).streams, cap), std::min(MAX_PARTS, n / 4)));
-    }
-    p.groups.clear();
-    // part 0 takes the fraction f0 of the blocks (its I runs alone, before
-    // any LU can start), the others share the rest equally
-    // (CAPS_AMD_PART0_FRAC; default: equal parts)
-    const double f0 = p.parts > 1 ? env_double("CAPS_AMD_PART0_FRAC", 1.0 / p.parts) : 1.0;
-    p.part_b[0] = 0;
-    p.part_b[1] = std::max(1, std::min(n - (p.parts - 1), (int)std::lround(n * f0)));
-    for (int g = 2; g <= p.parts; g++)
-        p.part_b[g] = p.part_b[1] + (int)((int64_t)(n - p.part_b[1]) * (g - 1) / (p.parts - 1));
-    for (int g = 0; g < p.parts; g++) {
-        p.part_goff[g] = (int)p.groups.size();
-        build_igroups(objs, c->h_desc, p.part_b[g], p.part_b[g + 1], p, p.part_cls[g]);
-    }
     return p;
-}
-
-BatchPlan plan_batch(caps_t* self, Ctx* c, const double* xi_, const int* m, int n, int with_lu)
-{
-    std::vector<caps_t*> objs(n, self);
-    return plan_batch_multi(objs.data(), c, xi_, m, n, with_lu);
-}
-
-size_t block_bytes_estimate(caps_t* self, int m)
-{
-    const int ldim = self->ldim, N = 2 * ldim;
-    const size_t lda = (N + 15) & ~15;
-    size_t lmin, lmax;
-    caps_estimate_lminmax(self, m, &lmin, &lmax);
-    const size_t nK = 2 * (lmin + ldim) + 4;
-    return (size_t)2 * (ldim + 2) * (ldim + 2) * 12 + 256 + lda * N * 8 + lda * (size_t)(2 * capsd_lu_npanels() * capsd_lu_nb() + 2 * capsd_lu_nb()) * 8 + nK * (24 * 2 + 24 * 64) +
-           (size_t)N * 32 + (size_t)((ldim + 15) / 16) * N * 8 + 65536;
 }
 
 // The LU of blocks [0, n) (descriptors already on the device) after event
@@ -764,22 +769,15 @@ int launch_lu_groups(Ctx* c, int n, int maxN, const LuCfg& cfg, hipEvent_t ready
     return launched;
 }
 
-// LU schedule of a planned one-part batch.  Blocks of unequal N run in
+// LU schedule of a planned batch of dense matrices.  Blocks of unequal N run in
 // MAX_LU_STREAMS groups of about equal cost, whose chains of dependent panel
 // steps then overlap, each with the schedule of its share of n_eff =
-// sum N^3 / maxN^3 blocks of the largest N (mixed-aspect batch of 64 blocks,
-// N 614-5462: LU 15.9 ms in one group with the table's schedule for 64
-// blocks, 12.4 ms this way).  One group when profiled: HIP events time the
-// launches of one group.
+// sum N^3 / maxN^3 blocks of the largest N.  One group when profiled: HIP
+// events time the launches of one group.
 LuCfg batch_lu_config(const Ctx* c, const BatchPlan& p, bool prof)
 {
     LuCfg cfg = lu_config(p.maxN, p.n);
-    bool fixed;
-    {
-        std::lock_guard<std::mutex> lock(g_cfg_mu);
-        fixed = g_have_override;   // a schedule fixed by capsx_lu_config applies as it is
-    }
-    if (p.parts == 1 && p.minN < p.maxN && !fixed) {
+    if (p.minN < p.maxN && !schedule_fixed()) {   // a schedule fixed by capsx_lu_config applies as it is
         double w = 0;
         for (int b = 0; b < p.n; b++) w += std::pow((double)c->h_desc[b].N / p.maxN, 3);
         cfg = lu_config(p.maxN, std::max(1, (int)lround(w / MAX_LU_STREAMS)));
@@ -801,141 +799,123 @@ int k_segments(const BatchPlan& p)
     return std::min(8, (target + p.sum_waves - 1) / p.sum_waves);
 }
 
-// Run the pipeline for n blocks already planned; mode 0: LU path, 1: M only.
 // The kernels of one planned batch on the library's stream (and the LU
 // streams); stage events between the stages when `events`.  Returns the
 // number of trailing-update launches of the first LU group.
-int enqueue_batch(Ctx* c, const BatchPlan& p, int mode, int lu_mode_shortcuts, bool events)
+int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
 {
     const int n = p.n;
     hipStream_t s = c->stream;
-    if (events) HIPCHECK(hipEventRecord(c->ev[0], s));
-    // the Mie coefficients beside the K quadrature (independent; the I
-    // tables need both), on the LU stream that no LU group or part uses:
-    // the K stage's time is then what it adds after the Mie kernel
-    hipStream_t sm = c->lu_stream[MAX_LU_STREAMS - 1];
-    HIPCHECK(hipEventRecord(c->head_fork, s));
-    HIPCHECK(hipStreamWaitEvent(sm, c->head_fork, 0));
-    capsd_launch_mie(c->d_desc, c->arena, g_lfac_dev, n, p.max_ldim, sm);
-    if (events) HIPCHECK(hipEventRecord(c->ev[1], sm));
-    HIPCHECK(hipEventRecord(c->mie_done, sm));
-    capsd_launch_K(c->d_desc, c->arena, g_lfac_dev, n, p.max_waves, p.max_nK, k_segments(p), c->d_status, s);
-    HIPCHECK(hipStreamWaitEvent(s, c->mie_done, 0));
-    if (events) HIPCHECK(hipEventRecord(c->ev[2], s));
-    int nlaunched = 0;
-    // part g on stream g (part 0 on the library's stream); its I waits for
-    // part g-1's I; stage events: I and assembly end with the last part's,
-    // the LU with the join of all parts
-    for (int g = 0; g < p.parts; g++) {
-        hipStream_t sg = g == 0 ? s : c->lu_stream[g - 1];
-        const int b0 = p.part_b[g], nb = p.part_b[g + 1] - b0;
-        const bool last = g == p.parts - 1;
-        if (g > 0) HIPCHECK(hipStreamWaitEvent(sg, c->part_i_done[g - 1], 0));
-        const IGroup* gr = c->d_groups + p.part_goff[g];
-        if (mode == 0) {
-            // trace pass: the I pairs of the diagonal band, the diagonal of M,
-            // the trace and its shortcut; the full I and matrix then only
-            // for the blocks that need an LU
-            capsd_launch_I(c->d_desc, c->arena, gr, p.part_cls[g], g_lfac_dev, p.max_nl, c->d_status, c->d_out, 1, 0,
-                           sg);
-            capsd_launch_assemble(c->d_desc + b0, c->arena, g_lfac_dev, nb, p.max_ldim, mode, c->d_out + b0, 1, sg);
-            capsd_launch_trace(c->d_desc + b0, c->arena, c->d_out + b0, nb, 0, sg);
-        }
-        capsd_launch_I(c->d_desc, c->arena, gr, p.part_cls[g], g_lfac_dev, p.max_ntri, c->d_status, c->d_out,
-                       0, mode == 0, sg);
-        if (!last) HIPCHECK(hipEventRecord(c->part_i_done[g], sg));
-        if (events && last) HIPCHECK(hipEventRecord(c->ev[3], sg));
-        // the symmetric delta-form LU reads nothing above the diagonal outside
-        // its 64 x 64 diagonal blocks: those mirror tiles are not assembled
-        const bool sym_only = mode == 0 && !lu_mode_shortcuts && (p.lu_kinds & 4) && !(p.lu_kinds & 1);
-        capsd_launch_assemble(c->d_desc + b0, c->arena, g_lfac_dev, nb, p.max_ldim, mode, c->d_out + b0,
-                              (mode == 0 ? 2 : 0) | (sym_only ? 4 : 0), sg);
-        if (mode == 0) capsd_launch_dominance(c->d_desc + b0, c->arena, c->d_out + b0, nb, p.maxN, g_delta_mode, sg);
-        if (mode == 0 && lu_mode_shortcuts)
-            capsd_launch_frobenius(c->d_desc + b0, c->arena, c->d_out + b0, nb, lu_mode_shortcuts == 2, sg);
-        if (events && last) HIPCHECK(hipEventRecord(c->ev[4], sg));
-        if (mode != 0) continue;
-        const bool prof = c->prof && p.parts == 1;
-        const LuCfg cfg = batch_lu_config(c, p, prof);
-        if (p.parts == 1) {
-            // one part: the LU in the schedule's stream groups
-            HIPCHECK(hipEventRecord(c->lu_ready, s));
-            nlaunched = launch_lu_groups(c, n, p.maxN, cfg, c->lu_ready, prof, p.lu_kinds);
-            continue;
-        }
-        const int k = capsd_launch_lu(c->d_desc + b0, c->arena, c->d_side + b0, c->d_out + b0, nb, p.maxN, sg,
-                                      cfg.levels, cfg.xcd, cfg.tile, prof ? c->gemm_ev.data() : nullptr,
-                                      prof ? c->gemm_info.data() : nullptr, p.lu_kinds);
-        if (g == 0) nlaunched = k;
+    auto mark = [&](int i) {
+        if (events) HIPCHECK(hipEventRecord(c->ev[i], s));
+    };
+    mark(0);
+    if (p.job == JOB_TABLES) {
+        capsd_launch_a0(c->d_desc, c->arena, g_lfac_dev, p.max_nl, s);
+        mark(1);
+        capsd_launch_K(c->d_desc, c->arena, g_lfac_dev, p.max_waves, p.max_nK, k_segments(p), c->d_status, s);
+        mark(2);
+        capsd_launch_I(c->d_desc, c->arena, c->h_desc[0].is_pr, p.max_nl, c->d_status, s);
+        mark(3);
+        mark(4);
+        return 0;
     }
-    for (int g = 1; g < p.parts; g++) {
-        HIPCHECK(hipEventRecord(c->lu_done[g], c->lu_stream[g - 1]));
-        HIPCHECK(hipStreamWaitEvent(s, c->lu_done[g], 0));
+    const bool det = p.job != JOB_MATRIX, piv = p.job == JOB_PIVOTED;
+    capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.max_waves, c->d_status, s);
+    mark(1);
+    if (det) {
+        capsd_launch_wave_norms(c->d_desc, c->arena, c->d_out, n, p.max_wq, s);
+        capsd_launch_wave_window(c->d_desc, c->arena, c->d_out, c->d_status, n, piv ? 0 : g_delta_mode,
+                                 p.form == FORM_GRAM, s);
     }
-    return nlaunched;
+    mark(2);
+    capsd_launch_wave_rows(c->d_desc, c->arena, c->d_out, n, p.max_wq, p.form == FORM_M, s);
+    mark(3);
+    if (p.form == FORM_M)
+        capsd_launch_wave_matrix(c->d_desc, c->arena, c->d_out, n, p.max_ldim, det ? 0 : 1,
+                                 det && !piv && p.lu_kinds == 6, s);
+    else
+        capsd_launch_gram(c->d_desc, c->arena, c->d_out, n, p.max_waves, p.split, p.form == FORM_BAND, s);
+    // the symmetric delta-form LU reads nothing above the diagonal outside its
+    // 64 x 64 diagonal blocks; k_frobenius (LU mode) reads all of the matrix
+    if (p.form == FORM_GRAM)
+        capsd_launch_band_dense(c->d_desc, c->arena, c->d_out, n, p.max_waves, p.lu_kinds != 6 || p.dmode, s);
+    if (det && p.dmode && p.form != FORM_BAND)
+        capsd_launch_frobenius(c->d_desc, c->arena, c->d_out, n, p.dmode == 2, s);
+    mark(4);
+    if (!det) return 0;
+    if (p.form == FORM_BAND) {
+        capsd_launch_band_ldl(c->d_desc, c->arena, c->d_out, n, p.dmode != 0, s);
+        return 0;
+    }
+    HIPCHECK(hipEventRecord(c->lu_ready, s));
+    return launch_lu_groups(c, n, p.maxN, batch_lu_config(c, p, c->prof), c->lu_ready, c->prof, p.lu_kinds);
 }
 
 // Identity of a captured batch: everything the launch sequence depends on
 // (grid shapes, group classes, LU schedule, buffers).  Descriptor contents
 // are read by the kernels at run time and are not part of it.
-std::vector<char> graph_key(Ctx* c, const BatchPlan& p, int mode, int lu_mode_shortcuts)
+std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
 {
-    const LuCfg cfg = batch_lu_config(c, p, c->prof && p.parts == 1);
     struct {
-        int n, maxN, max_ldim, max_waves, max_nK, kseg, mode, shortcuts, lu_kinds, delta_mode;
-        int64_t max_ntri;
-        int parts, part_b[MAX_PARTS + 1], part_goff[MAX_PARTS], cls[MAX_PARTS][8];
+        int n, ntab, maxN, max_ldim, max_waves, max_wq, max_mie, max_nK, max_nl, kseg, job, form, dmode, split;
+        int is_pr, lu_kinds, delta_mode;
         int levels, streams, xcd, tile;
         int lu_bnd[MAX_LU_STREAMS + 1], lu_gN[MAX_LU_STREAMS];   // the LU's stream groups (lu_groups)
         int lu_kernels[3], grid_panel_rows;   // LU kernel variants (capsx_lu_kernels, capsx_lu_grid_panel_rows)
-        const void *arena, *desc, *side, *out, *groups;
+        const void *arena, *desc, *side, *out;
     } k;
     memset(&k, 0, sizeof(k));
     k.n = p.n;
+    k.ntab = p.ntab;
     k.maxN = p.maxN;
     k.max_ldim = p.max_ldim;
     k.max_waves = p.max_waves;
-    k.kseg = k_segments(p);
+    k.max_wq = p.max_wq;
+    k.max_mie = p.max_mie;
     k.max_nK = p.max_nK;
-    k.mode = mode;
-    k.shortcuts = lu_mode_shortcuts;
+    k.max_nl = p.max_nl;
+    k.job = p.job;
+    k.form = p.form;
+    k.dmode = p.dmode;
+    k.split = p.split;
+    if (p.job == JOB_TABLES) {
+        k.kseg = k_segments(p);
+        k.is_pr = c->h_desc[0].is_pr;
+    }
     k.lu_kinds = p.lu_kinds;
     k.delta_mode = g_delta_mode;
-    k.max_ntri = p.max_ntri;
-    k.parts = p.parts;
-    memcpy(k.part_b, p.part_b, sizeof(k.part_b));
-    memcpy(k.part_goff, p.part_goff, sizeof(k.part_goff));
-    memcpy(k.cls, p.part_cls, sizeof(k.cls));
-    k.levels = cfg.levels;
-    k.streams = cfg.streams;
-    k.xcd = cfg.xcd;
-    k.tile = cfg.tile;
-    if (p.parts == 1 && mode == 0) lu_groups(c, p.n, p.maxN, cfg.streams, k.lu_bnd, k.lu_gN);
+    if (p.form != FORM_BAND) {
+        const LuCfg cfg = batch_lu_config(c, p, c->prof);
+        k.levels = cfg.levels;
+        k.streams = cfg.streams;
+        k.xcd = cfg.xcd;
+        k.tile = cfg.tile;
+        lu_groups(c, p.n, p.maxN, cfg.streams, k.lu_bnd, k.lu_gN);
+    }
     capsd_lu_kernels(-1, -1, -1, k.lu_kernels);
     k.grid_panel_rows = capsd_lu_grid_panel_rows(0);
     k.arena = c->arena;
     k.desc = c->d_desc;
     k.side = c->d_side;
     k.out = c->d_out;
-    k.groups = c->d_groups;
     const char* b = reinterpret_cast<const char*>(&k);
     return std::vector<char>(b, b + sizeof(k));
 }
 
-// Run the pipeline for n blocks already planned; mode 0: LU path, 1: M only.
-// With graph mode on, each batch shape is captured once into a HIP graph and
-// replayed; descriptor uploads and the status reset stay outside the graph.
-void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_shortcuts)
+// Run the pipeline for the blocks already planned.  With graph mode on, each
+// batch shape is captured once into a HIP graph and replayed; the descriptor
+// upload (with the status word's reset) stays outside the graph.
+void run_batch(caps_t* self, Ctx* c, const BatchPlan& p)
 {
     const int n = p.n;
+    const bool det = p.job == JOB_LOGDET || p.job == JOB_PIVOTED;
     hipStream_t s = c->stream;
     ensure_arena(c, p.bytes);
-    HIPCHECK(hipMemcpyAsync(c->d_desc, c->h_desc, n * sizeof(BlockDesc), hipMemcpyHostToDevice, s));
-    HIPCHECK(hipMemcpyAsync(c->d_side, c->h_side, n * sizeof(LuSide), hipMemcpyHostToDevice, s));
-    const int ng = (int)p.groups.size();
-    memcpy(c->h_groups, p.groups.data(), ng * sizeof(IGroup));
-    HIPCHECK(hipMemcpyAsync(c->d_groups, c->h_groups, ng * sizeof(IGroup), hipMemcpyHostToDevice, s));
-    HIPCHECK(hipMemsetAsync(c->d_status, 0, sizeof(int), s));
+    HIPCHECK(hipMemcpyAsync(c->d_up, c->h_up, UP_HEAD + n * sizeof(BlockDesc) + p.ntab * sizeof(MieDesc),
+                            hipMemcpyHostToDevice, s));
+    if (det && p.form != FORM_BAND)
+        HIPCHECK(hipMemcpyAsync(c->d_side, c->h_side, n * sizeof(LuSide), hipMemcpyHostToDevice, s));
     const int nupd = capsd_lu_max_updates(p.maxN);
     if (c->prof && (int)c->gemm_ev.size() < 2 * nupd) {
         const size_t old = c->gemm_ev.size();
@@ -946,14 +926,14 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_s
     int nlaunched = 0;
     const bool use_graph = c->graph && !c->prof;
     if (use_graph) {
-        const std::vector<char> key = graph_key(c, p, mode, lu_mode_shortcuts);
+        const std::vector<char> key = graph_key(c, p);
         hipGraphExec_t exec = nullptr;
         for (auto& g : c->graphs)
             if (g.first == key) exec = g.second;
         if (!exec) {
             hipGraph_t graph;
             HIPCHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            enqueue_batch(c, p, mode, lu_mode_shortcuts, false);
+            enqueue_batch(c, p, false);
             HIPCHECK(hipStreamEndCapture(s, &graph));
             HIPCHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
             HIPCHECK(hipGraphDestroy(graph));
@@ -966,12 +946,13 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_s
         HIPCHECK(hipEventRecord(c->ev[0], s));
         HIPCHECK(hipGraphLaunch(exec, s));
     } else {
-        nlaunched = enqueue_batch(c, p, mode, lu_mode_shortcuts, true);
+        nlaunched = enqueue_batch(c, p, true);
     }
     HIPCHECK(hipEventRecord(c->ev[5], s));
     HIPCHECK(hipGetLastError());
-    if (mode == 0) HIPCHECK(hipMemcpyAsync(c->h_out, c->d_out, n * sizeof(BlockOut), hipMemcpyDeviceToHost, s));
-    HIPCHECK(hipMemcpyAsync(c->h_status, c->d_status, sizeof(int), hipMemcpyDeviceToHost, s));
+    // a determinant's status comes with its results
+    if (det) HIPCHECK(hipMemcpyAsync(c->h_out, c->d_out, n * sizeof(BlockOut), hipMemcpyDeviceToHost, s));
+    else HIPCHECK(hipMemcpyAsync(c->h_status, c->d_status, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     float ms;
     if (use_graph) {
@@ -985,10 +966,13 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_s
     }
     HIPCHECK(hipEventElapsedTime(&ms, c->ev[0], c->ev[5]));
     c->timing[5] = ms;
-    TERMINATE(*c->h_status != 0, "non-finite k-integral (flags %d) in a batch of %d blocks (xi_=%g, m=%d ...)",
-              *c->h_status, n, c->h_desc[0].xi_, c->h_desc[0].m);
+    const int status = det ? c->h_out[0].status : *c->h_status;
+    TERMINATE(status != 0, "non-finite k-integral (flags %d) in a batch of %d blocks (xi_=%g, m=%d ...)", status, n,
+              c->h_desc[0].xi_, c->h_desc[0].m);
     for (int i = 0; i < 6; i++) c->acc[i] += c->timing[i];
-    if (c->prof && mode == 0) {
+    // dimension of a factored block's matrix
+    auto dim_of = [&](int b) { return p.form == FORM_M ? (double)c->h_desc[b].N : 16.0 * c->h_out[b].tiles; };
+    if (c->prof && det) {
         // algorithmic flops of each k_lu_gemm_dma launch: 2 x rows x columns
         // x depth; the time of the other update launches (k_lu_gemm tiles)
         for (int pi = 0; pi < nlaunched; pi++) {
@@ -1003,7 +987,7 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_s
             const bool sym = p.lu_kinds & 4;
             for (int b = 0; b < n; b++) {
                 if (c->h_out[b].skip) continue;
-                const double N = c->h_desc[b].N;
+                const double N = dim_of(b);
                 const double r0 = g[0] + g[1], c0 = g[0] + g[3];
                 // region rows x cols, depth kk: flops 2 x elements x kk; HBM
                 // bytes: C read and written once, L and U read once.  The
@@ -1037,14 +1021,16 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p, int mode, int lu_mode_s
     c->acc[9] += 1;
     for (int b = 0; b < n; b++) {
         const BlockDesc& d = c->h_desc[b];
-        c->acc[10] += (double)d.nl * (d.nl + 1) / 2 * (d.is_pr ? 1 : 2);
-        if (mode == 0 && c->h_out[b].skip == 0) {
-            const double N = d.N;
+        if (p.job == JOB_TABLES) c->acc[10] += (double)d.nl * (d.nl + 1) / 2 * (d.is_pr ? 1 : 2);
+        if (det && c->h_out[b].skip == 0) {
+            const double N = dim_of(b);
             c->acc[7] += 1;
-            // LU: 2/3 N^3 - 1/2 N^2 + 5/6 N flops; the symmetric (LDL^T)
-            // form of a dominant block: 1/3 N^3 + 1/2 N^2 - 5/6 N
+            // LU: 2/3 N^3 - 1/2 N^2 + 5/6 N flops; LDL^T of a symmetric matrix:
+            // 1/3 N^3 + 1/2 N^2 - 5/6 N; of a band of half-width w: w (w + 2)
+            // per column but for the last w, which are dense
+            const double w = std::min(N, p.form == FORM_BAND ? 16.0 * (capsd::BAND_TILES - 1) : N);
             if ((p.lu_kinds & 4) && c->h_out[b].delta)
-                c->acc[8] += 1.0 / 3 * N * N * N + 0.5 * N * N - 5.0 / 6 * N;
+                c->acc[8] += (N - w) * w * (w + 2) + 1.0 / 3 * w * w * w + 0.5 * w * w - 5.0 / 6 * w;
             else
                 c->acc[8] += 2.0 / 3 * N * N * N - 0.5 * N * N + 5.0 / 6 * N;
         }
@@ -1100,19 +1086,6 @@ double finish_block(const BlockOut& o, int lu_mode)
 // diagonal only, so its Mercator test sees the lower triangle).
 int dense_mode(detalg_t a) { return a == DETALG_HODLR ? 0 : a == DETALG_CHOLESKY ? 2 : 1; }
 bool is_lu_mode(detalg_t a) { return dense_mode(a) != 0; }
-
-// Largest number of blocks per launch sequence that fits the HBM budget.
-int chunk_blocks_multi(caps_t* const* objs, const int* m, int n)
-{
-    const size_t budget = arena_budget();
-    size_t acc = 0;
-    int k = 0;
-    for (; k < n; k++) {
-        acc += block_bytes_estimate(objs[k], m[k]);
-        if (acc > budget && k > 0) break;
-    }
-    return std::max(k, 1);
-}
 
 }  // namespace
 
@@ -1558,21 +1531,21 @@ static int logdetD_multi_ordered(caps_t* host, caps_t* const* objs, const double
     std::lock_guard<std::mutex> lock(c->mu);
     const int lu_mode = dense_mode(objs[0]->detalg);
     double tot[6] = {0, 0, 0, 0, 0, 0};
-    // a batch of several launch sequences takes the whole budget at once:
-    // HIP kept a freed arena's memory from the next allocation (device memory
-    // free after growing a 92.6 GB arena to 100 GB: 115 of 309 GB), so an
-    // arena grown between sequences held both
-    if (chunk_blocks_multi(objs, m, n) < n) ensure_arena(c, arena_budget());
     // CAPS_AMD_PROGRESS=1: one line on stderr per launch sequence
     static const bool progress = env_double("CAPS_AMD_PROGRESS", 0) > 0;
     for (int b0 = 0; b0 < n;) {
         const double t_seq = progress ? wall_seconds() : 0;
-        const int k = chunk_blocks_multi(objs + b0, m + b0, n - b0);
-        ensure_blocks(c, k);
-        BatchPlan p = plan_batch_multi(objs + b0, c, xi_ + b0, m + b0, k, 1);
-        run_batch(host, c, p, 0, lu_mode);
-        // blocks whose 1 - M is not column dominant were left unfactored by
-        // the delta-form LU: run them again with the pivoted LU
+        ensure_blocks(c, n - b0);
+        const BatchPlan p = plan_batch_multi(objs + b0, c, xi_ + b0, m + b0, n - b0, JOB_LOGDET, lu_mode);
+        const int k = p.n;
+        // a batch of several launch sequences takes the whole budget at once:
+        // HIP kept a freed arena's memory from the next allocation (device memory
+        // free after growing a 92.6 GB arena to 100 GB: 115 of 309 GB), so an
+        // arena grown between sequences held both
+        if (k < n) ensure_arena(c, arena_budget());
+        run_batch(host, c, p);
+        // blocks left unfactored (the delta form ruled out by
+        // capsx_lu_delta_mode): run them again with the pivoted LU
         std::vector<int> again;
         for (int i = 0; i < k; i++)
             if (c->h_out[i].skip == 0 && !c->h_out[i].delta) again.push_back(b0 + i);
@@ -1596,11 +1569,14 @@ static int logdetD_multi_ordered(caps_t* host, caps_t* const* objs, const double
                 rx.push_back(xi_[i]);
                 rm.push_back(m[i]);
             }
-            BatchPlan q = plan_batch_multi(ro.data(), c, rx.data(), rm.data(), (int)again.size(), 1);
-            q.lu_kinds = 1;
-            run_batch(host, c, q, 0, lu_mode);
-            for (size_t j = 0; j < again.size(); j++) take(c->h_out[j], again[j]);
-            for (int i = 0; i < 6; i++) tot[i] += c->timing[i];
+            for (int a0 = 0; a0 < (int)again.size();) {
+                const BatchPlan q = plan_batch_multi(ro.data() + a0, c, rx.data() + a0, rm.data() + a0,
+                                                     (int)again.size() - a0, JOB_PIVOTED, lu_mode);
+                run_batch(host, c, q);
+                for (int j = 0; j < q.n; j++) take(c->h_out[j], again[a0 + j]);
+                for (int i = 0; i < 6; i++) tot[i] += c->timing[i];
+                a0 += q.n;
+            }
         }
         if (progress)
             fprintf(stderr, "capsx: blocks %d..%d of %d (dimension <= %d, %zu pivoted) in %.2f s\n", b0, b0 + k - 1,
@@ -1678,8 +1654,8 @@ caps_M_t* caps_M_init(caps_t* caps, int m, double xi_)
     Ctx* c = ctx_of(caps);
     std::lock_guard<std::mutex> lock(c->mu);
     ensure_blocks(c, 1);
-    BatchPlan p = plan_batch(caps, c, &xi_, &m, 1, 0);
-    run_batch(caps, c, p, 1, 0);
+    const BatchPlan p = plan_batch_multi(&caps, c, &xi_, &m, 1, JOB_MATRIX, 0);
+    run_batch(caps, c, p);
     const BlockDesc& d = c->h_desc[0];
     caps_M_t* self = (caps_M_t*)calloc(1, sizeof(caps_M_t));
     self->caps = caps;
@@ -1695,8 +1671,9 @@ caps_M_t* caps_M_init(caps_t* caps, int m, double xi_)
                          d.N * sizeof(double), d.N, hipMemcpyDeviceToHost));
     self->al = (double*)malloc(d.ldim * sizeof(double));
     self->bl = (double*)malloc(d.ldim * sizeof(double));
-    HIPCHECK(hipMemcpy(self->al, c->arena + d.off_mie, d.ldim * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHECK(hipMemcpy(self->bl, c->arena + d.off_mie + d.ldim * 8, d.ldim * sizeof(double), hipMemcpyDeviceToHost));
+    HIPCHECK(hipMemcpy(self->al, c->arena + d.off_mie + (d.lmin - 1) * 8, d.ldim * sizeof(double),
+                       hipMemcpyDeviceToHost));
+    HIPCHECK(hipMemcpy(self->bl, c->arena + d.off_mie + ((int64_t)d.mie_L + d.lmin - 1) * 8, d.ldim * sizeof(double), hipMemcpyDeviceToHost));
     self->integration = st;
     return self;
 }
@@ -3276,8 +3253,8 @@ static void block_tables_host(caps_t* self, double xi_, int m, IntegTables& t)
     Ctx* c = ctx_of(self);
     std::lock_guard<std::mutex> lock(c->mu);
     ensure_blocks(c, 1);
-    BatchPlan p = plan_batch(self, c, &xi_, &m, 1, 0);
-    run_batch(self, c, p, 1, 0);
+    const BatchPlan p = plan_batch_multi(&self, c, &xi_, &m, 1, JOB_TABLES, 0);
+    run_batch(self, c, p);
     const BlockDesc& d = c->h_desc[0];
     t.m = m;
     t.is_pr = d.is_pr != 0;
@@ -3601,7 +3578,6 @@ int capsx_block_nodes(caps_t* self, double xi_, int m)
     size_t lmin, lmax;
     caps_estimate_lminmax(self, m, &lmin, &lmax);
     d.alpha = 2 * xi_;
-    d.mu = m > 0 ? 2 * m : 2;
     d.lo = (int)lmin - 1;
     d.nl = self->ldim + 2;
     d.nu_max = 2 * (d.lo + d.nl - 1);

@@ -1,9 +1,8 @@
-// Round-trip matrix of (ξ, m) blocks on gfx950: Mie coefficients, the
-// k-integrals K_ν, the integrals I_{l1 l2} and the matrix 1 - M.
-//
-// Every kernel is batched: blockIdx.y (or .z) selects the (ξ, m) block, the
-// remaining grid dimensions cover the work of one block, lanes beyond a
-// block's own extent idle.  All arithmetic is FP64.
+// The k-integrals K_ν and I_{l1 l2} of one block as tables (the reference's
+// integration.h; determinants are taken from the wave-number factor,
+// waves.hip), point functions, and what dense matrices need beside the LU:
+// trace, dominance, the LU-mode shortcut, the ξ = 0 blocks.  All arithmetic
+// is FP64.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -19,54 +18,26 @@ template <typename T>
 __device__ __forceinline__ T* at(char* base, int64_t off) { return reinterpret_cast<T*>(base + off); }
 
 // ---------------------------------------------------------------------------
-// Mie coefficients: one lane per l of the block's window.
-// Reference: src/libcaps.c:557-602 (caps_mie), cached per block as in
-// src/libcaps.c:690-694 and 766-770.
-//
-// Besides log|a_l|, log|b_l| it stores the per-l halves of the element
-// prefactors: log Λ_{l1 l2} = (g(l1) + g(l2))/2 with
-// g(l) = log(2l+1) - log l - log(l+1) + log(l-m)! - log(l+m)! (the
-// separable form of src/libcaps.c:45-48), so ea(l) = (log|a_l| + g(l))/2 and
-// eb(l) = (log|b_l| + g(l))/2 give every element prefactor as a product of
-// two factors e^{ea}, e^{eb}, stored as mantissa × 2^exponent.
-__global__ void __launch_bounds__(256) k_mie(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                             const double* __restrict__ lfac_tab)
+// Separable parts of log a0 of the I integrals:
+//   log a0(l1, l2) = g1(l1) + g1(l2) + g2(l1 + l2),
+//   g1(l) = log(2l)! - log l! - log(l-m)!,
+//   g2(s) = log s! - log(2s)! + log(s-2m)!      (m -> max(m, 1))
+__global__ void __launch_bounds__(256) k_a0(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                            const double* __restrict__ lfac_tab)
 {
-    const BlockDesc& d = desc[blockIdx.y];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double* al = at<double>(arena, d.off_mie);   // [a | b | ea | eb], ldim each
-    {
-        // separable parts of log a0 of the I integrals:
-        //   log a0(l1, l2) = g1(l1) + g1(l2) + g2(l1 + l2),
-        //   g1(l) = log(2l)! - log l! - log(l-m)!,
-        //   g2(s) = log s! - log(2s)! + log(s-2m)!      (m -> max(m, 1))
-        const int m_ = d.m > 0 ? d.m : 1;
-        double* g1 = al + 5 * d.ldim;
-        double* g2 = g1 + d.nl;
-        if (i < d.nl) {
-            const int l = d.lo + i;
-            g1[i] = l >= m_ ? lfac(lfac_tab, 2 * l) - lfac(lfac_tab, l) - lfac(lfac_tab, l - m_) : 0.0;
-        }
-        if (i < 2 * d.nl - 1) {
-            const int sl = 2 * d.lo + i;
-            g2[i] = sl >= 2 * m_ ? lfac(lfac_tab, sl) - lfac(lfac_tab, 2 * sl) + lfac(lfac_tab, sl - 2 * m_) : 0.0;
-        }
+    const BlockDesc& d = desc[0];
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int m_ = d.m > 0 ? d.m : 1;
+    double* g1 = at<double>(arena, d.off_a0);
+    double* g2 = g1 + d.nl;
+    if (i < d.nl) {
+        const int l = d.lo + i;
+        g1[i] = l >= m_ ? lfac(lfac_tab, 2 * l) - lfac(lfac_tab, l) - lfac(lfac_tab, l - m_) : 0.0;
     }
-    if (i >= d.ldim) return;
-    double lna, lnb;
-    const int l = d.lmin + i, m = d.m;
-    mie(d.xi_, d.LbyR, d.epsm1_sphere, l, lna, lnb);
-    const double g = logi(2 * l + 1) - logi(l) - logi(l + 1) + lfac(lfac_tab, l - m) - lfac(lfac_tab, l + m);
-    al[i] = lna;
-    al[d.ldim + i] = lnb;
-    int* ex = reinterpret_cast<int*>(al + 4 * d.ldim);
-    // e^{ea}, e^{eb} as mantissa in [1, 2) times 2^exponent
-    const double xa = (lna + g) / 2 * (1 / LOG2), xb = (lnb + g) / 2 * (1 / LOG2);
-    const double fa = floor(xa), fb = floor(xb);
-    al[2 * d.ldim + i] = exp2(xa - fa);
-    al[3 * d.ldim + i] = exp2(xb - fb);
-    ex[i] = (int)fa;
-    ex[d.ldim + i] = (int)fb;
+    if (i < 2 * d.nl - 1) {
+        const int sl = 2 * d.lo + i;
+        g2[i] = sl >= 2 * m_ ? lfac(lfac_tab, sl) - lfac(lfac_tab, 2 * sl) + lfac(lfac_tab, sl - 2 * m_) : 0.0;
+    }
 }
 
 // Mie coefficients at arbitrary (ξ, l) points (scalar API caps_mie).
@@ -368,50 +339,26 @@ __device__ __forceinline__ AlphaND alpha_nd(double p, double s2, double d2)
     return {(p2 - s2) * (p2 - d2), 4 * p2 - 1};
 }
 
-// One group: up to GM blocks that share (m, ℓ-window, polarizations) — in
-// a free energy the blocks of one m at different frequencies — so the a_q of
-// a pair are computed once and applied to every block's K table.
-// band != 0: only the pairs with i1 - i2 <= 2, which the diagonal of M
-// needs (the trace pass); use_skip != 0: blocks whose trace shortcut is
-// already decided (out[b].skip) take no part.
-// C: steps of the a_q recurrence per chunk (see below)
-template <int NPOL, int GM, int C>
+// The full lower triangle of block 0, C steps of the a_q recurrence per chunk
+// (see below).
+template <int NPOL>
 __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                           const IGroup* __restrict__ groups, const double* __restrict__ lfac_tab,
-                                           int* __restrict__ status, const BlockOut* __restrict__ out, int band,
-                                           int use_skip)
+                                           int* __restrict__ status)
 {
+    constexpr int C = 4;
     static_assert(C >= 3, "the convergence test looks at a chunk's last three terms");
     static_assert(2 * (C - 1) <= K_GUARD, "a chunk reads at most 2 (C - 1) entries below the K table");
-    const IGroup& grp = groups[blockIdx.y];
-    const int G = grp.count;
-    // the group's blocks that take part (uniform over the workgroup)
-    bool act[GM];
-    bool any = false;
-#pragma unroll
-    for (int g = 0; g < GM; g++) {
-        act[g] = g < G && !(use_skip && out[grp.blk[g]].skip);
-        any = any || act[g];
-    }
-    if (!any) return;
-    const BlockDesc& d = desc[grp.blk[0]];
+    const BlockDesc& d = desc[0];
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int nl = d.nl;
     int i1, i2;
-    if (band) {
-        if (t >= 3 * (int64_t)nl) return;
-        i1 = (int)(t / 3);
-        i2 = i1 - (int)(t % 3);
-        if (i2 < 0) return;
-    } else {
-        const int64_t ntri = (int64_t)nl * (nl + 1) / 2;
-        if (t >= ntri) return;
-        // triangular index -> (i1 >= i2)
-        i1 = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-        while ((int64_t)i1 * (i1 + 1) / 2 > t) i1--;
-        while ((int64_t)(i1 + 1) * (i1 + 2) / 2 <= t) i1++;
-        i2 = (int)(t - (int64_t)i1 * (i1 + 1) / 2);
-    }
+    const int64_t ntri = (int64_t)nl * (nl + 1) / 2;
+    if (t >= ntri) return;
+    // triangular index -> (i1 >= i2)
+    i1 = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+    while ((int64_t)i1 * (i1 + 1) / 2 > t) i1--;
+    while ((int64_t)(i1 + 1) * (i1 + 2) / 2 <= t) i1++;
+    i2 = (int)(t - (int64_t)i1 * (i1 + 1) / 2);
     const int l1 = d.lo + i1, l2 = d.lo + i2;
     // the table keeps the lower triangle only (row i1 >= column i2, row
     // major): a wave's stores are contiguous, and readers take I(l1, l2) at
@@ -420,16 +367,12 @@ __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, c
     const int64_t nl2 = (int64_t)nl * nl;
 
     const int m_ = d.m > 0 ? d.m : 1;
+    double* Im = at<double>(arena, d.off_i);         // [2][nl*nl]
+    int* Ie = at<int>(arena, d.off_i + 16 * nl2);    // [2][nl*nl]
     if (l2 < m_ || l2 < d.m) {
-        for (int g = 0; g < G; g++) {
-            if (!act[g]) continue;
-            const BlockDesc& dg = desc[grp.blk[g]];
-            double* Im = at<double>(arena, dg.off_i);
-            int* Ie = at<int>(arena, dg.off_i + 16 * nl2);
-            for (int pol = 0; pol < 2; pol++) {
-                Im[pol * nl2 + a] = 0;
-                Ie[pol * nl2 + a] = 0;
-            }
+        for (int pol = 0; pol < 2; pol++) {
+            Im[pol * nl2 + a] = 0;
+            Ie[pol * nl2 + a] = 0;
         }
         return;
     }
@@ -442,50 +385,33 @@ __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, c
     int qmax = (l12 - 2 * m_) / 2;
     qmax = min(qmax, min(l1, l2));
     const double Ap = -2 * m * (n - nu) * (n + nu + 1);
-    const double* g1 = at<double>(arena, d.off_mie) + 5 * d.ldim;   // separable parts of log a0 (k_mie)
+    const double* g1 = at<double>(arena, d.off_a0);   // separable parts of log a0
     const double* g2 = g1 + nl;
     const double log_a0 = g1[i1] + g1[i2] + g2[i1 + i2];
 
-    // per block and polarization: running sum (exponent-aligned to the q = 0
-    // term) and its shift S - E0 (a_q = aq 2^S, E0 the exponent of the q = 0
-    // term)
-    // the group's K tables (same nK: same m and ℓ-window); polarization pol
-    // of block g at kb[g] + pol nK
-    const KEnt* kb[GM];
+    // per polarization: running sum (exponent-aligned to the q = 0 term) and
+    // its shift S - E0 (a_q = aq 2^S, E0 the exponent of the q = 0 term)
+    const KEnt* kb = at<KEnt>(arena, d.off_k);   // polarization pol at kb + pol nK
     const int nK = d.nK;
-    double sum[GM][NPOL];
-    int sh[GM][NPOL];
-    // bit g NPOL + pp: that sum has converged (absent blocks count as such)
-    unsigned done = 0;
+    double sum[NPOL];
+    int sh[NPOL];
+    unsigned done = 0;   // bit pp: that sum has converged
 #pragma unroll
-    for (int g = 0; g < GM; g++) {
-        kb[g] = act[g] ? at<KEnt>(arena, desc[grp.blk[g]].off_k) : nullptr;
-#pragma unroll
-        for (int pp = 0; pp < NPOL; pp++) {
-            sh[g][pp] = 0;
-            sum[g][pp] = 0;
-            if (act[g]) {
-                const KEnt k0 = kb[g][(POL0 + pp) * nK + l12 - mu];
-                sh[g][pp] = -k0.e;   // S - E0, S = 0
-                sum[g][pp] = k0.m;
-            } else {
-                done |= 1u << (g * NPOL + pp);
-            }
-        }
+    for (int pp = 0; pp < NPOL; pp++) {
+        const KEnt k0 = kb[(POL0 + pp) * nK + l12 - mu];
+        sh[pp] = -k0.e;   // S - E0, S = 0
+        sum[pp] = k0.m;
     }
-    constexpr unsigned ALL = NPOL * GM >= 32 ? ~0u : (1u << (NPOL * GM)) - 1;
+    constexpr unsigned ALL = (1u << NPOL) - 1;
 
     // q = 1, 2: eqs. (26)-(30), added to every sum
     auto add_term = [&](int q, double aq) {
         const int j = l12 - 2 * q - mu;
 #pragma unroll
-        for (int g = 0; g < GM; g++)
-#pragma unroll
-            for (int pp = 0; pp < NPOL; pp++)
-                if (act[g]) {
-                    const KEnt kv = kb[g][(POL0 + pp) * nK + j];
-                    sum[g][pp] += ldexp(aq * kv.m, kv.e + sh[g][pp]);
-                }
+        for (int pp = 0; pp < NPOL; pp++) {
+            const KEnt kv = kb[(POL0 + pp) * nK + j];
+            sum[pp] += ldexp(aq * kv.m, kv.e + sh[pp]);
+        }
     };
     double aqm2 = 1, aqm1 = 1, aq = 1;  // a_{q-2}, a_{q-1}, a_q
     double tn = 0, tv = 0, r3 = 0, rn1 = 0, rv1 = 0;
@@ -537,9 +463,7 @@ __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, c
                 aqm1 = ldexp(aqm1, -e);
                 S += e;
 #pragma unroll
-                for (int g = 0; g < GM; g++)
-#pragma unroll
-                    for (int pp = 0; pp < NPOL; pp++) sh[g][pp] += e;
+                for (int pp = 0; pp < NPOL; pp++) sh[pp] += e;
             }
         }
         double ac[C];
@@ -574,28 +498,24 @@ __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, c
         }
         const int jb = l12 - 2 * q0 - mu;   // K index of the chunk's first step
 #pragma unroll
-        for (int g = 0; g < GM; g++) {
-            if (!act[g]) continue;
+        for (int pp = 0; pp < NPOL; pp++) {
+            const unsigned bit = 1u << pp;
+            if (!__any(!(done & bit))) continue;   // uniform: converged in every lane
+            // index jb - 2t; steps past qmax (coefficient 0) may reach
+            // 2 (C - 1) entries below the table: the zeroed guard there
+            // (polarization 0) or the other polarization's last entries
+            const KEnt* kp = kb + (POL0 + pp) * nK + jb;
+            KEnt kv[C];
 #pragma unroll
-            for (int pp = 0; pp < NPOL; pp++) {
-                const unsigned bit = 1u << (g * NPOL + pp);
-                if (!__any(!(done & bit))) continue;   // uniform: converged in every lane
-                // index jb - 2t; steps past qmax (coefficient 0) may reach
-                // 2 (C - 1) entries below the table: the zeroed guard there
-                // (polarization 0) or the other polarization's last entries
-                const KEnt* kp = kb[g] + (POL0 + pp) * nK + jb;
-                KEnt kv[C];
+            for (int t = 0; t < C; t++) kv[t] = kp[-2 * t];
+            double tm[C];
 #pragma unroll
-                for (int t = 0; t < C; t++) kv[t] = kp[-2 * t];
-                double tm[C];
-#pragma unroll
-                for (int t = 0; t < C; t++) {
-                    tm[t] = ldexp(ac[t] * kv[t].m, kv[t].e + sh[g][pp]);
-                    sum[g][pp] += tm[t];
-                }
-                const double lim = fabs(sum[g][pp]) * 0x1p-56;
-                if (fabs(tm[C - 1]) < lim && fabs(tm[C - 2]) < lim && fabs(tm[C - 3]) < lim) done |= bit;
+            for (int t = 0; t < C; t++) {
+                tm[t] = ldexp(ac[t] * kv[t].m, kv[t].e + sh[pp]);
+                sum[pp] += tm[t];
             }
+            const double lim = fabs(sum[pp]) * 0x1p-56;
+            if (fabs(tm[C - 1]) < lim && fabs(tm[C - 2]) < lim && fabs(tm[C - 3]) < lim) done |= bit;
         }
     }
 
@@ -606,287 +526,23 @@ __global__ void __launch_bounds__(256) k_I(const BlockDesc* __restrict__ desc, c
     const double a0m = exp2(la2 - fl);
     const int a0e = (int)fl;
 #pragma unroll
-    for (int g = 0; g < GM; g++) {
-        if (!act[g]) continue;
-        const BlockDesc& dg = desc[grp.blk[g]];
-        double* Im = at<double>(arena, dg.off_i);                 // [2][nl*nl]
-        int* Ie = at<int>(arena, dg.off_i + 16 * nl2);            // [2][nl*nl]
-#pragma unroll
-        for (int pp = 0; pp < NPOL; pp++) {
-            const int pol = POL0 + pp;
-            const double sv = sum[g][pp];
-            if (!(sv != 0) || !isfinite(sv)) atomicOr(status, 2);
-            int e2;
-            const double mt = frexp(sv * a0m, &e2);
-            const int ex = e2 + a0e + S - sh[g][pp];
-            // (plain stores: non-temporal ones leave the waves' partial lines
-            // unmerged in L2, 10 % more bytes written to HBM)
-            Im[pol * nl2 + a] = mt;
-            Ie[pol * nl2 + a] = ex;
-            if (NPOL == 1) {
-                Im[a] = -fabs(mt);
-                Ie[a] = ex;
-            }
+    for (int pp = 0; pp < NPOL; pp++) {
+        const int pol = POL0 + pp;
+        const double sv = sum[pp];
+        if (!(sv != 0) || !isfinite(sv)) atomicOr(status, 2);
+        int e2;
+        const double mt = frexp(sv * a0m, &e2);
+        const int ex = e2 + a0e + S - sh[pp];
+        Im[pol * nl2 + a] = mt;
+        Ie[pol * nl2 + a] = ex;
+        if (NPOL == 1) {
+            Im[a] = -fabs(mt);
+            Ie[a] = ex;
         }
     }
 }
 
 // ---------------------------------------------------------------------------
-// Matrix assembly: one lane per 2x2 (E,M) tile (l1, l2), 16 x 16 tiles per
-// workgroup.  Writes
-// mode 0: 1 - M (the matrix the LU factors), mode 1: M, column-major with
-// leading dimension lda; row i = 2(l1-lmin) + p1, column j = 2(l2-lmin) + p2
-// (the interleaved index map of src/libcaps.c:717-743).  Elements follow
-// src/libcaps.c:761-831 and A/B/C/D src/integration.c:762-888.
-
-// Element contributions in linear form: with the prefactor e^p = pm · 2^pe
-// (Mie and Λ factors), X·e^p is summed directly from the I values (stored as
-// mantissa × 2^exponent),
-//   A·e^p = m² I e^p,
-//   B·e^p = Σ_k c_k I_k e^p   (4 terms; m = 0: I itself),
-//   C·e^p = m [-(l2+1)(l2+m)/(2l2+1) I_1 e^p + l2(l2-m+1)/(2l2+1) I_2 e^p],
-// the same quantities as src/integration.c:762-888 followed by the exp of
-// src/libcaps.c:784-829, without the intermediate log: each term is a
-// product of mantissas and one ldexp.  Terms below the smallest double
-// vanish, as they do there.
-
-// Coefficients of B and C, separable in l1 and l2:
-//   u(l) = (l+1)(l+m)/(2l+1),  v(l) = l(l-m+1)/(2l+1).
-struct UV {
-    double u, v;
-};
-
-typedef double nt_double2 __attribute__((ext_vector_type(2)));   // 16-byte non-temporal stores
-
-__device__ __forceinline__ UV uv(int l, int m)
-{
-    const double r = 1.0 / (2 * l + 1);
-    return {(l + 1.) * (l + m) * r, l * (l - m + 1.) * r};
-}
-
-// flags bit 0: the trace pass: only the diagonal tiles and only the
-// diagonal of M (from I pairs with |l1 - l2| <= 2); bit 1: leave out the
-// blocks with out[b].skip set; bit 2: the symmetric delta-form LU follows,
-// so a mirror tile outside the 64 x 64 diagonal blocks (tile pairs 2k, 2k+1)
-// is not written, only its column partial sums (from the lower tile's rows).
-// Full pass: workgroup blockIdx.x takes the tile pair (bx, by), bx >= by
-// (linear index over the lower triangle of 16 x 16 tiles of (l1, l2)): the
-// tile at rows of bx and columns of by and its mirror at rows of by and
-// columns of bx, both from one I window (I is symmetric), so every I value
-// is read about once.  Trace pass: blockIdx.x = bx = by.
-// mode 0 (LU path) writes -M, i.e. 1 - M without its unit diagonal (the LU's
-// delta form; k_dominance puts the unit diagonal back where the LU needs
-// partial pivoting), and for every column of a tile's 32 rows the sum of
-// |M_ij| over its rows i != j into off_cpart (at the tile's row tile);
-// mode 1 writes M.
-__global__ void __launch_bounds__(256) k_assemble(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                  const double* __restrict__ lfac_tab, int mode,
-                                                  const BlockOut* __restrict__ out, int flags)
-{
-    const BlockDesc& d = desc[blockIdx.z];
-    if ((flags & 2) && out[blockIdx.z].skip) return;
-    const bool diag_only = flags & 1;
-    int bx, by;
-    if (diag_only) {
-        bx = by = blockIdx.x;
-    } else {
-        const int64_t t = blockIdx.x;
-        bx = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
-        while ((int64_t)bx * (bx + 1) / 2 > t) bx--;
-        while ((int64_t)(bx + 1) * (bx + 2) / 2 <= t) bx++;
-        by = (int)(t - (int64_t)bx * (bx + 1) / 2);
-    }
-    const int L1 = d.lmin + bx * 16, L2 = d.lmin + by * 16;
-    if (L1 >= d.lmin + d.ldim) return;   // uniform over the workgroup (L2 <= L1)
-    const int m = d.m;
-    // the I values of the workgroup's 16 x 16 tile and its ±1 halo, both
-    // polarizations, loaded once into LDS; the window holds I(l1, l2) at
-    // [pol][l2 - L2 + 1][l1 - L1 + 1] (rows padded to 19: conflict-free
-    // column accesses).  The table keeps I(l1, l2) = I(l2, l1) once, at row
-    // max(l1, l2), column min(l1, l2) (row major): below the diagonal
-    // (L1 > L2) consecutive lanes take consecutive l2, so that the reads are
-    // contiguous
-    __shared__ double wm[2][18][19];
-    __shared__ int we[2][18][19];
-    __shared__ double csum[16][2][16];   // [column pair][parity][row pair]: |M| of the lane's 2 rows
-    __shared__ double rsum[16][2][16];   // [row pair][parity][column pair]: |M| of the lane's 2 columns
-    {
-        const double* Im = at<double>(arena, d.off_i);
-        const int* Ie = at<int>(arena, d.off_i + 16 * (int64_t)d.nl * d.nl);
-        const int64_t nl2 = (int64_t)d.nl * d.nl;
-        const bool below = L1 > L2;
-        for (int t = threadIdx.x; t < 2 * 18 * 18; t += 256) {
-            const int pol = t / 324, u = (t / 18) % 18, v = t % 18;
-            const int r = below ? v : u, c = below ? u : v;
-            const int l1 = L1 - 1 + c, l2 = L2 - 1 + r;
-            const bool ok = l1 >= d.lo && l2 >= d.lo && l1 < d.lo + d.nl && l2 < d.lo + d.nl && l1 >= m && l2 >= m;
-            const int hi = max(l1, l2), lw = min(l1, l2);
-            const int64_t idx = pol * nl2 + (int64_t)(hi - d.lo) * d.nl + (lw - d.lo);
-            wm[pol][r][c] = ok ? Im[idx] : 0.0;
-            we[pol][r][c] = ok ? Ie[idx] : 0;
-        }
-    }
-    __syncthreads();
-    const int c0 = threadIdx.x & 15, r0 = threadIdx.x >> 4;
-    const bool partials = mode == 0 && !diag_only && d.n_rtiles > 0;
-    // flags bit 2: its columns' partial sums are the lower tile's row sums
-    // (|M_ij| = |M_ji|)
-    const bool skip_mirror = (flags & 4) && !diag_only && bx != by && (bx >> 1) != (by >> 1);
-    const bool rows_too = partials && skip_mirror;
-    const double* ma = at<double>(arena, d.off_mie) + 2 * d.ldim;   // mantissas of e^{ea}, e^{eb}
-    const double* mb = ma + d.ldim;
-    const int* xa = reinterpret_cast<const int*>(ma + 2 * d.ldim);  // their exponents
-    const int* xb = xa + d.ldim;
-    double* Am = at<double>(arena, d.off_mat);
-    const int64_t lda = d.lda;
-    const double sg = mode == 0 ? -1.0 : 1.0;
-
-    // The 2 x 2 block of matrix rows 2 i2, 2 i2 + 1 and columns 2 j2,
-    // 2 j2 + 1 (l1 = lmin + i2, l2 = lmin + j2), written, and for the
-    // partial column sums its |M| over its two rows per column (i2 == j2:
-    // without the diagonal) into csum[cp][.][rp].  I(l1 + a, l2 + b) is
-    // wm[pol][wr + b][wc + a] (tr = 0) or wm[pol][wr + a][wc + b] (tr = 1,
-    // the mirror tile: the window of (l2, l1)).
-    auto block = [&](int i2, int j2, int wr, int wc, bool tr, int cp, int rp) {
-        const int l1 = d.lmin + i2, l2 = d.lmin + j2;
-        // I(l1 + a, l2 + b) of polarization pol times the prefactor pm 2^pe
-        auto X = [&](int pol, int a, int b, double pm, int pe) {
-            const int rr = tr ? wr + a : wr + b, cc = tr ? wc + b : wc + a;
-            return ldexp(wm[pol][rr][cc] * pm, we[pol][rr][cc] + pe);
-        };
-        const double ma1 = ma[i2], mb1 = mb[i2], ma2 = ma[j2], mb2 = mb[j2];
-        const int xa1 = xa[i2], xb1 = xb[i2], xa2 = xa[j2], xb2 = xb[j2];
-        const int TE = 0, TM = 1;
-        const UV c1 = uv(l1, m), c2 = uv(l2, m);
-        // A = m² I;  B = u1 u2 I(-1,-1) - v1 u2 I(+1,-1) - u1 v2 I(-1,+1) + v1 v2 I(+1,+1)
-        // (m = 0: B = I);  C(l1,l2) = m [-u2 I(0,-1) + v2 I(0,+1)];
-        // D(l1,l2) = C(l2,l1) = m [-u1 I(-1,0) + v1 I(+1,0)]   (I symmetric)
-        auto A = [&](int pol, double pm, int pe) { return m == 0 ? 0.0 : (double)m * m * X(pol, 0, 0, pm, pe); };
-        auto B = [&](int pol, double pm, int pe) {
-            if (m == 0) return X(pol, 0, 0, pm, pe);
-            return c1.u * c2.u * X(pol, -1, -1, pm, pe) - c1.v * c2.u * X(pol, 1, -1, pm, pe)
-                 - c1.u * c2.v * X(pol, -1, 1, pm, pe) + c1.v * c2.v * X(pol, 1, 1, pm, pe);
-        };
-        auto C = [&](int pol, double pm, int pe) {
-            return m * (-c2.u * X(pol, 0, -1, pm, pe) + c2.v * X(pol, 0, 1, pm, pe));
-        };
-        auto D = [&](int pol, double pm, int pe) {
-            return m * (-c1.u * X(pol, -1, 0, pm, pe) + c1.v * X(pol, 1, 0, pm, pe));
-        };
-        // EE: √(a_l1 a_l2) Λ (B_TM - A_TE);  MM: √(b_l1 b_l2) Λ (A_TM - B_TE)
-        const double pEE = ma1 * ma2, pMM = mb1 * mb2;
-        const int eEE = xa1 + xa2, eMM = xb1 + xb2;
-        const double EE = B(TM, pEE, eEE) - A(TE, pEE, eEE);
-        const double MM = A(TM, pMM, eMM) - B(TE, pMM, eMM);
-        if (diag_only) {
-            double* dg = at<double>(arena, d.off_diag);
-            dg[2 * i2] = EE;
-            dg[2 * i2 + 1] = MM;
-            return;
-        }
-        double EM = 0, ME = 0;
-        if (m != 0) {
-            // EM: D_TM - C_TE with (a_l1 + b_l2)/2;  ME: C_TM - D_TE with (b_l1 + a_l2)/2
-            const double pEM = ma1 * mb2, pME = mb1 * ma2;
-            const int eEM = xa1 + xb2, eME = xb1 + xa2;
-            EM = D(TM, pEM, eEM) - C(TE, pEM, eEM);
-            ME = C(TM, pME, eME) - D(TE, pME, eME);
-        }
-        const int64_t r = 2 * i2, c = 2 * j2;
-        // rows r, r+1 of a column are adjacent: one 16-byte store per column
-        // (r and lda even, the matrix 256-byte aligned)
-        // (non-temporal: the matrices of a batch are far larger than the
-        // caches, and these lines would only evict the I windows)
-        __builtin_nontemporal_store((nt_double2){sg * EE, sg * ME}, reinterpret_cast<nt_double2*>(Am + r + c * lda));
-        __builtin_nontemporal_store((nt_double2){sg * EM, sg * MM},
-                                    reinterpret_cast<nt_double2*>(Am + r + (c + 1) * lda));
-        if (i2 == j2) {
-            double* dg = at<double>(arena, d.off_diag);
-            dg[r] = EE;
-            dg[r + 1] = MM;
-        }
-        if (partials) {
-            // column c: EE (row r, the diagonal when i2 = j2) and ME (row r+1);
-            // column c+1: EM (row r) and MM (row r+1, the diagonal when i2 = j2)
-            csum[cp][0][rp] = (i2 == j2 ? 0.0 : fabs(EE)) + fabs(ME);
-            csum[cp][1][rp] = fabs(EM) + (i2 == j2 ? 0.0 : fabs(MM));
-            if (rows_too) {
-                // row r: EE, EM; row r+1: ME, MM (no diagonal in such a tile)
-                rsum[rp][0][cp] = fabs(EE) + fabs(EM);
-                rsum[rp][1][cp] = fabs(ME) + fabs(MM);
-            }
-        }
-    };
-    // the 32 columns of a tile at column tile ct, row tile rt: the sum over
-    // its 32 rows in row order
-    auto column_sums = [&](int rt, int ct) {
-        if (threadIdx.x < 32) {
-            const int jp = threadIdx.x >> 1, par = threadIdx.x & 1;
-            const int col = 2 * (ct * 16 + jp) + par;
-            if (col < d.N) {
-                double sum = 0;
-#pragma unroll
-                for (int q = 0; q < 16; q++) sum += csum[jp][par][q];
-                at<double>(arena, d.off_cpart)[(int64_t)rt * d.N + col] = sum;
-            }
-        }
-    };
-
-    // the tile (rows of bx, columns of by): lane (c0, r0) takes i2 = 16 bx + c0,
-    // j2 = 16 by + r0
-    {
-        const int i2 = bx * 16 + c0, j2 = by * 16 + r0;
-        const bool in = i2 < d.ldim && j2 < d.ldim && (!diag_only || i2 == j2);
-        if (in) block(i2, j2, r0 + 1, c0 + 1, false, r0, c0);
-        else if (partials) {
-            csum[r0][0][c0] = 0.0;
-            csum[r0][1][c0] = 0.0;
-            if (rows_too) {
-                rsum[c0][0][r0] = 0.0;
-                rsum[c0][1][r0] = 0.0;
-            }
-        }
-        if (diag_only) return;   // no barrier follows in the trace pass
-        if (partials) {
-            __syncthreads();
-            column_sums(bx, by);
-        }
-    }
-    if (bx == by) return;   // uniform: a diagonal tile is its own mirror
-    if (skip_mirror) {
-        // the mirror's 32 columns (rows of bx) over the 32 rows of by: the
-        // lower tile's row sums in column order
-        if (rows_too && threadIdx.x >= 32 && threadIdx.x < 64) {
-            const int ip = (threadIdx.x - 32) >> 1, par = threadIdx.x & 1;
-            const int col = 2 * (bx * 16 + ip) + par;
-            if (col < d.N) {
-                double sum = 0;
-#pragma unroll
-                for (int q = 0; q < 16; q++) sum += rsum[ip][par][q];
-                at<double>(arena, d.off_cpart)[(int64_t)by * d.N + col] = sum;
-            }
-        }
-        return;
-    }
-    // the mirror (rows of by, columns of bx): lane (c0, r0) takes
-    // i2 = 16 by + c0, j2 = 16 bx + r0, whose I(l1 + a, l2 + b) is the
-    // window's I(l2 + b, l1 + a)
-    {
-        if (partials) __syncthreads();   // csum is reused
-        const int i2 = by * 16 + c0, j2 = bx * 16 + r0;
-        const bool in = i2 < d.ldim && j2 < d.ldim;
-        if (in) block(i2, j2, c0 + 1, r0 + 1, true, r0, c0);
-        else if (partials) {
-            csum[r0][0][c0] = 0.0;
-            csum[r0][1][c0] = 0.0;
-        }
-        if (partials) {
-            __syncthreads();
-            column_sums(by, bx);
-        }
-    }
-}
-
 // Column diagonal dominance of 1 - M (the matrix holds -M, the column sums
 // of |M_ij|, i != j, per row tile are in off_cpart): column j is dominant if
 // Σ_{i≠j} |M_ij| < |1 - M_jj|.  A matrix whose columns are all strictly
@@ -1061,59 +717,25 @@ using namespace capsd;
 
 extern "C" {
 
-void capsd_launch_mie(const BlockDesc* desc, char* arena, const double* lfac_tab, int nblocks, int max_ldim,
-                      hipStream_t s)
+// The K and I tables of one block (desc[0]).
+void capsd_launch_a0(const BlockDesc* desc, char* arena, const double* lfac_tab, int nl, hipStream_t s)
 {
-    dim3 g((2 * (max_ldim + 2) + 255) / 256, nblocks);
-    hipLaunchKernelGGL(k_mie, g, dim3(256), 0, s, desc, arena, lfac_tab);
+    hipLaunchKernelGGL(k_a0, dim3((2 * nl + 255) / 256), dim3(256), 0, s, desc, arena, lfac_tab);
 }
 
-void capsd_launch_K(const BlockDesc* desc, char* arena, const double* lfac_tab, int nblocks, int max_waves,
-                    int max_nK, int nseg, int* status, hipStream_t s)
+void capsd_launch_K(const BlockDesc* desc, char* arena, const double* lfac_tab, int waves, int nK, int nseg,
+                    int* status, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_K_partial, dim3(max_waves * nseg, nblocks), dim3(64), 0, s, desc, arena, lfac_tab, nseg);
-    hipLaunchKernelGGL(k_K_combine, dim3((max_nK + 255) / 256, nblocks), dim3(256), 0, s, desc, arena, status);
+    hipLaunchKernelGGL(k_K_partial, dim3(waves * nseg), dim3(64), 0, s, desc, arena, lfac_tab, nseg);
+    hipLaunchKernelGGL(k_K_combine, dim3((nK + 255) / 256), dim3(256), 0, s, desc, arena, status);
 }
 
-// I tables of the batch's groups, ordered by class: perfect reflectors
-// (TM only) with at most 1, 2, 4, 8 blocks per group, then both
-// polarizations likewise; counts[8] holds the groups per class.
-// band: only the pairs the diagonal of M needs (max_ntri is then the
-// largest nl); use_skip: leave out the blocks with out[b].skip set.
-void capsd_launch_I(const BlockDesc* desc, char* arena, const void* groups, const int* counts,
-                    const double* lfac_tab, int64_t max_ntri, int* status, const BlockOut* out, int band,
-                    int use_skip, hipStream_t s)
+// is_pr: TM only (perfect reflector: I_TE = -|I_TM|)
+void capsd_launch_I(const BlockDesc* desc, char* arena, int is_pr, int nl, int* status, hipStream_t s)
 {
-    const IGroup* gr = (const IGroup*)groups;
-    const unsigned gx = (unsigned)(((band ? 3 * max_ntri : max_ntri) + 255) / 256);
-    // recurrence steps per chunk: 4 (default) or 8 (CAPS_AMD_I_CHUNK=8)
-    static const int chunk = [] {
-        const char* e = getenv("CAPS_AMD_I_CHUNK");
-        return e && atoi(e) == 8 ? 8 : 4;
-    }();
-    int off = 0;
-#define KI(NP, GMV, CLS)                                                                                       \
-    if (counts[CLS] > 0) {                                                                                    \
-        if (chunk == 8)                                                                                       \
-            hipLaunchKernelGGL((k_I<NP, GMV, 8>), dim3(gx, counts[CLS]), dim3(256), 0, s, desc, arena,       \
-                               gr + off, lfac_tab, status, out, band, use_skip);                              \
-        else                                                                                                  \
-            hipLaunchKernelGGL((k_I<NP, GMV, 4>), dim3(gx, counts[CLS]), dim3(256), 0, s, desc, arena,       \
-                               gr + off, lfac_tab, status, out, band, use_skip);                              \
-    }                                                                                                         \
-    off += counts[CLS];
-    KI(1, 1, 0) KI(1, 2, 1) KI(1, 4, 2) KI(1, 8, 3)
-    KI(2, 1, 4) KI(2, 2, 5) KI(2, 4, 6) KI(2, 8, 7)
-#undef KI
-}
-
-// flags: see k_assemble (1 = diagonal only, 2 = leave out skipped blocks)
-void capsd_launch_assemble(const BlockDesc* desc, char* arena, const double* lfac_tab, int nblocks, int max_ldim,
-                           int mode, const BlockOut* out, int flags, hipStream_t s)
-{
-    const unsigned T = (unsigned)((max_ldim + 15) / 16);
-    dim3 g((flags & 1) ? T : T * (T + 1) / 2, 1, nblocks);
-    hipLaunchKernelGGL(k_assemble, g, dim3(256), 0, s, desc, arena, lfac_tab, mode, out, flags);
+    const dim3 g((unsigned)(((int64_t)nl * (nl + 1) / 2 + 255) / 256));
+    if (is_pr) hipLaunchKernelGGL(k_I<1>, g, dim3(256), 0, s, desc, arena, status);
+    else hipLaunchKernelGGL(k_I<2>, g, dim3(256), 0, s, desc, arena, status);
 }
 
 void capsd_launch_frobenius(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int lower, hipStream_t s)

@@ -1,0 +1,802 @@
+// Determinants of (ξ, m) blocks from their wave-number factor on gfx950.
+//
+// Every element of the round-trip matrix is an integral over x = cosh θ in
+// [1, ∞) of products of two one-degree functions (the A, B, C, D of the
+// reference, src/integration.c:762-888, with I_{l1 l2} = ∫ r_p e^{-αx}
+// P_l1^m P_l2^m/(x²-1) dx written under one integral sign):
+//   p_l = m P_l^m/√(x²-1),  t_l = √(x²-1) dP_l^m/dx  (m = 0: p_l = 0, t_l = P_l^1),
+//   EE = √(a a') Λ Σ_x w (r_TM t t' + |r_TE| p p'),
+//   MM = √(b b') Λ Σ_x w (r_TM p p' + |r_TE| t t'),
+//   EM = √(a b') Λ Σ_x w (r_TM t p' + |r_TE| p t'),
+// all terms positive.  On the nodes of one quadrature grid that is M = FᵀF,
+// one row of F per node and polarization, and det(1 - FᵀF) = det(1 - F Fᵀ):
+// the determinant of the smaller Gram matrix G = F Fᵀ, whose dimension is
+// twice the number of nodes that matter (some 2.2 √(2 lmax) + 30) instead of
+// 2 ldim.  A row of F is a ridge of a few standard deviations around the
+// degree whose saddle point is the node, so rows of distant nodes do not
+// overlap: G is banded, and each of its tiles needs a fraction of the degrees.
+// R/L = 200, ldim = 1200: 2400 rows become about 400 with a half-bandwidth
+// of 96; R/L = 2000, ldim = 12000: 24000 become about 1300.
+//
+// Kernels (blockIdx.y, or .x of the last, selects the block):
+//   k_wave_start   the Mie coefficients of each (object, ξ), and beside them
+//                  the nodes with the degree recurrence of P_l^m over all l,
+//                  whose state is kept at the start of every 16 degrees;
+//   k_wave_rows    F of 16 degrees x 64 nodes from such a state: first only
+//                  the squared norms (trace, window, activity), then the
+//                  rows of the blocks that need a determinant;
+//   k_wave_window  trace, trace shortcut, the nodes that matter;
+//   k_gram         the band of -G on FP64 MFMA;
+//   k_band_ldl     log det(1 - G): banded LDLᵀ, one workgroup per block;
+//   k_band_dense   -G as a dense matrix (schedules fixed by the caller, the
+//                  pivoted LU);
+//   k_wave_matrix  M = FᵀF itself (caps_M_init, CHOLESKY mode).
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+
+#include "blocks.h"
+#include "device_math.h"
+#include "wave.h"
+
+namespace capsd {
+
+template <typename T>
+__device__ __forceinline__ T* at(char* base, int64_t off) { return reinterpret_cast<T*>(base + off); }
+
+typedef double double4_t __attribute__((ext_vector_type(4)));
+
+// Row of node k and polarization p (0 TM, 1 TE) in F: tiles of 8 nodes, 8 TM
+// rows then 8 TE rows, so that a tile of 16 rows is the unit of the band.
+__device__ __forceinline__ int row_of(int k, int p) { return (k >> 3) * 16 + p * 8 + (k & 7); }
+
+// Exponent of what is zero whatever it is added to: 2^NO_EXP 2^E = 0.
+constexpr int NO_EXP = -(1 << 28);
+
+// x^(-1) from the hardware estimate and two Newton steps (normal x).
+__device__ __forceinline__ double rcp_nr(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(fma(-x, r, 1.0), r, r);
+    return fma(fma(-x, r, 1.0), r, r);
+}
+
+// One step of S_l = √((l-m)!/(l+m)!) P_l^m upward in the degree (DLMF
+// 14.10.3), c1 = (2l+1)/√((l+1)²-m²), c2 = √(l²-m²)/√((l+1)²-m²).
+__device__ __forceinline__ void degree_step(double c1, double c2, double x, double& p, double& pp)
+{
+    const double pn = fma(c1 * x, p, -(c2 * pp));
+    pp = p;
+    p = pn;
+}
+
+// Powers of two moved from S into its exponent E (every fourth step: a step
+// multiplies by less than 2x + 1).
+__device__ __forceinline__ void rescale(double& p, double& pp, int& E)
+{
+    if (p > 0x1p300) {
+        p *= 0x1p-300;
+        pp *= 0x1p-300;
+        E += 300;
+    }
+}
+
+// log(C(2m, m)/4^m): a product for small m, else the asymptotic series of
+// log Γ(m+½)/Γ(m+1) (DLMF 5.11.13), whose first neglected term is below 1e-16
+// from m = 16.
+__device__ __forceinline__ double log_central_binomial(int m)
+{
+    if (m < 16) {
+        double r = 1;
+        for (int k = 1; k <= m; k++) r *= (2 * k - 1) / (2.0 * k);
+        return log(r);
+    }
+    const double i = 1.0 / m, i2 = i * i;
+    return -0.5 * log(M_PI * m)
+         + i * (-1. / 8 + i2 * (1. / 192 + i2 * (-1. / 640 + i2 * (17. / 14336 - i2 * (31. / 18432)))));
+}
+
+__device__ void mie_entry(const MieDesc& t, char* __restrict__ arena, int l)
+{
+    if (l > t.L) return;
+    double lna, lnb;
+    mie(t.xi_, t.LbyR, t.epsm1, l, lna, lnb);
+    double* a = at<double>(arena, t.off) + (l - 1);
+    a[0] = lna;
+    a[t.L] = lnb;
+    // √a_l and √b_l times √((2l+1)/(l(l+1))) as mantissas of one power of two
+    const double g = log((2.0 * l + 1) / ((double)l * (l + 1.0)));
+    const double xa = (lna + g) / 2 * (1 / LOG2), xb = (lnb + g) / 2 * (1 / LOG2);
+    const double fa = floor(xa);
+    a[2 * t.L] = exp2(xa - fa);
+    a[3 * t.L] = exp2(xb - fa);
+    at<int>(arena, t.off + 32 * (int64_t)t.L)[l - 1] = (int)fa;
+}
+
+// blockIdx.y < ntab: Mie coefficients of table blockIdx.y, one lane per l.
+// Else block blockIdx.y - ntab: 64 nodes per wavefront, one lane each; a
+// chain of one FMA per degree, 17 cycles a step (R/L = 200: 9 µs of a single
+// block), so the rest of F's work is left to k_wave_rows, which starts from
+// the states kept here and runs all degrees at once.
+__global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ tabs, int ntab,
+                                                   const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                   int* __restrict__ status)
+{
+    if ((int)blockIdx.y < ntab) {
+        mie_entry(tabs[blockIdx.y], arena, blockIdx.x * 64 + threadIdx.x + 1);
+        return;
+    }
+    const BlockDesc& d = desc[blockIdx.y - ntab];
+    const int wave = blockIdx.x, lane = threadIdx.x;
+    if (wave >= d.n_waves) return;
+    const int k = wave * 64 + lane, nP = d.n_waves * 64;
+    const int mm = d.m > 0 ? d.m : 1;
+    double x = 1, p = 0, pp = 0, stm = 0, ste = 0;
+    int E = NO_EXP;   // lanes without a node: 0 times a power of two that is 0
+    if (k < d.n_nodes) {
+        const double v = d.v0 + k * d.h;
+        const double L = v > 40 ? v : log1p(exp(v));
+        const double sg = 1 / (1 + exp(-v));
+        const double xm1 = d.A * d.A * L * L;
+        x = 1 + xm1;
+        const double x2m1 = xm1 * (x + 1);
+        const double dx = 2 * d.A * d.A * L * sg;
+        // S_mm = √(C(2mm,mm)/4^mm) (x²-1)^{mm/2}, times e^{-ξx} √(h dx) and, for
+        // m > 0, the 1/√(x²-1) of p_l and t_l
+        const double lb = 0.5 * (log_central_binomial(mm) + (d.m > 0 ? mm - 1 : mm) * log(x2m1) + log(d.h * dx))
+                        - d.xi_ * x;
+        const double lb2 = lb * (1 / LOG2), fl = floor(lb2);
+        E = (int)fl;
+        p = exp((lb2 - fl) * LOG2);
+        double rte, rtm;
+        fresnel(d.epsm1_plate, d.xi_, d.xi_ * sqrt(x2m1), rte, rtm);
+        stm = sqrt(fabs(rtm));
+        ste = sqrt(fabs(rte));
+        if (!(stm > 0 && ste > 0 && isfinite(stm) && isfinite(ste) && isfinite(lb))) atomicOr(status, 1);
+    }
+    double* nd = at<double>(arena, d.off_node);
+    nd[k] = x;
+    nd[nP + k] = stm;
+    nd[2 * nP + k] = ste;
+
+    __shared__ double c1s[64], c2s[64];
+    auto coefficients = [&](int l0) {
+        const double l = l0 + lane;
+        const double den = 1 / sqrt((l + 1 - mm) * (l + 1 + mm));
+        c1s[lane] = (2 * l + 1) * den;
+        c2s[lane] = sqrt((l - mm) * (l + mm)) * den;
+        __syncthreads();
+    };
+    for (int l0 = mm; l0 < d.lmin; l0 += 64) {   // below the window
+        coefficients(l0);
+        const int n = min(64, d.lmin - l0);
+        int j = 0;
+        for (; j + 4 <= n; j += 4) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) degree_step(c1s[j + q], c2s[j + q], x, p, pp);
+            rescale(p, pp, E);
+        }
+        for (; j < n; j++) degree_step(c1s[j], c2s[j], x, p, pp);
+        rescale(p, pp, E);
+        __syncthreads();
+    }
+    double2* cp = at<double2>(arena, d.off_ck);
+    int* ce = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP);
+    for (int c0 = 0; c0 < d.n_chunks; c0 += 4) {
+        coefficients(d.lmin + 16 * c0);
+        const int nc = min(4, d.n_chunks - c0);
+        for (int c = 0; c < nc; c++) {
+            const int64_t i = (int64_t)(c0 + c) * nP + k;
+            cp[i] = make_double2(p, pp);
+            ce[i] = E;
+#pragma unroll
+            for (int j = 0; j < 16; j += 4) {
+#pragma unroll
+                for (int q = 0; q < 4; q++) degree_step(c1s[16 * c + j + q], c2s[16 * c + j + q], x, p, pp);
+                rescale(p, pp, E);
+            }
+        }
+        __syncthreads();
+    }
+}
+
+// F of degrees lmin + 16 c .. + 15 at 64 nodes (one lane each), four chunks c
+// per workgroup.  STORE = false: the nodes' squared norms over the chunk and
+// per tile of 8 nodes the exponent of the largest (c_k < 2^e).  STORE = true:
+// the rows themselves, F[2(l-lmin) + (0: a_l, 1: b_l)][row], of the blocks
+// without a trace shortcut; tiles that k_gram reads as zero (a chunk norm
+// below 2^emin, or outside the window) are not written.  all != 0: every
+// entry (k_wave_matrix).  Degrees past the window are zero.
+// VALU-bound: about 20 FP64 instructions per degree and lane.
+template <bool STORE>
+__global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                   const BlockOut* __restrict__ out, int all)
+{
+    const int b = blockIdx.y;
+    const BlockDesc& d = desc[b];
+    const int nq = (d.n_chunks + 3) / 4;
+    if ((int)blockIdx.x >= d.n_waves * nq) return;
+    if (STORE && !all && (out[b].skip || out[b].tiles <= 0)) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wave = blockIdx.x % d.n_waves, c = (blockIdx.x / d.n_waves) * 4 + wv;
+    const int nP = d.n_waves * 64, nT = nP >> 3, k = wave * 64 + lane;
+    const int m = d.m, mm = m > 0 ? m : 1;
+    struct Deg {
+        double c1, c2, l, rt, ma, mb;
+        int e, pad_;
+        double tf;
+    };
+    __shared__ Deg degs[4][16];
+    const bool in = c < d.n_chunks;
+    if (in && lane < 16) {
+        const int l = d.lmin + 16 * c + lane;
+        const double den = 1 / sqrt((l + 1.0 - mm) * (l + 1.0 + mm));
+        Deg g;
+        g.l = l;
+        g.rt = sqrt(((double)l - mm) * ((double)l + mm));
+        g.c1 = (2.0 * l + 1) * den;
+        g.c2 = g.rt * den;
+        const double* a = at<double>(arena, d.off_mie) + (l - 1);
+        const bool ok = l < d.lmin + d.ldim;
+        g.ma = ok ? a[2 * (int64_t)d.mie_L] : 0.0;
+        g.mb = ok ? a[3 * (int64_t)d.mie_L] : 0.0;
+        g.e = ok ? at<int>(arena, d.off_mie + 32 * (int64_t)d.mie_L)[l - 1] : NO_EXP;
+        g.tf = sqrt((double)l * (l + 1.0));   // m = 0: t_l = P_l^1 = √(l(l+1)) S_l
+        degs[wv][lane] = g;
+    }
+    __syncthreads();
+    if (!in) return;
+    const int64_t ci = (int64_t)c * nP + k;
+    const int tile = k >> 3;
+    int* act = at<int>(arena, d.off_act) + (int64_t)c * nT + tile;
+    bool st = true;
+    if (STORE && !all) {
+        const int t0 = out[b].tile0;
+        st = tile >= t0 && tile < t0 + out[b].tiles && *act >= out[b].emin;
+        if (!__any(st)) return;
+    }
+    const double* nd = at<double>(arena, d.off_node);
+    const double x = nd[k], stm = nd[nP + k], ste = nd[2 * nP + k];
+    const double2 s = at<double2>(arena, d.off_ck)[ci];
+    double p = s.x, pp = s.y;
+    int E = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[ci];
+    const int64_t ldf = 2 * (int64_t)nP;
+    double* F = STORE ? at<double>(arena, d.off_rows) + 32 * (int64_t)c * ldf + row_of(k, 0) : nullptr;
+    double norm = 0;
+#pragma unroll 4
+    for (int j = 0; j < 16; j++) {
+        const Deg& g = degs[wv][j];
+        const double t = m > 0 ? fma(g.l * x, p, -(g.rt * pp)) : g.tf * p;
+        const double u = ldexp(1.0, E + g.e);
+        const double utm = u * stm, ute = u * ste, mp = d.m * p;
+        const double f0 = t * utm * g.ma, f1 = mp * utm * g.mb;   // TM row: a_l, b_l
+        const double f2 = mp * ute * g.ma, f3 = t * ute * g.mb;   // TE row
+        if (STORE) {
+            if (st) {
+                F[0] = f0;
+                F[8] = f2;
+                F[ldf] = f1;
+                F[ldf + 8] = f3;
+            }
+            F += 2 * ldf;
+        } else {
+            norm = fma(f0, f0, fma(f1, f1, fma(f2, f2, fma(f3, f3, norm))));
+        }
+        degree_step(g.c1, g.c2, x, p, pp);
+        if ((j & 3) == 3) rescale(p, pp, E);
+    }
+    if (!STORE) {
+        at<double>(arena, d.off_norm)[ci] = norm;
+        int e = norm > 0 ? ilogb(norm) + 1 : NO_EXP;   // a NaN norm: the trace is NaN
+        e = max(e, dpp_i<DPP_QUAD_X1>(e));
+        e = max(e, dpp_i<DPP_QUAD_X2>(e));
+        e = max(e, dpp_i<DPP_HALF_MIRROR>(e));
+        if ((lane & 7) == 0) *act = e;
+    }
+}
+
+// Trace of M = the sum of all rows' squared norms (per node in chunk order,
+// then over the nodes with compensated sums in a fixed order), the trace
+// shortcut |tr M| < 1e-8 (src/matrix.c:78-82), and the window: tiles of 8
+// nodes from the first to the last node whose rows carry more than 2^-60 of
+// the trace (together the others change the determinant by less than a few
+// 1e-17 of it; R/L = 20 .. 2000: 10-60 % of the nodes of large m).  dense:
+// the matrix dimension for the LU's kernels goes to desc[b].N.
+__global__ void __launch_bounds__(256) k_wave_window(BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                     BlockOut* __restrict__ out, const int* __restrict__ status,
+                                                     int allow, int dense)
+{
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const BlockDesc& d = desc[b];
+    const int nP = d.n_waves * 64;
+    const double* cn = at<double>(arena, d.off_norm);
+    double* dn = at<double>(arena, d.off_dn);
+    double s = 0, comp = 0;
+    for (int k = tid; k < nP; k += 256) {
+        double v = 0;
+#pragma unroll 8
+        for (int c = 0; c < d.n_chunks; c++) v += cn[(int64_t)c * nP + k];
+        dn[k] = v;
+        double t, e;
+        two_sum(s, v, t, e);
+        s = t;
+        comp += e;
+    }
+    __shared__ double hs[256], cs[256];
+    __shared__ int lo_s, hi_s;
+    hs[tid] = s;
+    cs[tid] = comp;
+    if (tid == 0) {
+        lo_s = nP;
+        hi_s = -1;
+    }
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+        if (tid < o) {
+            double t, e;
+            two_sum(hs[tid], hs[tid + o], t, e);
+            hs[tid] = t;
+            cs[tid] = (cs[tid] + cs[tid + o]) + e;
+        }
+        __syncthreads();
+    }
+    const double trace = hs[0] + cs[0], thr = trace * 0x1p-60;
+    for (int k = tid; k < nP; k += 256)
+        if (dn[k] > thr) {
+            atomicMin(&lo_s, k);
+            atomicMax(&hi_s, k);
+        }
+    __syncthreads();
+    if (tid != 0) return;
+    BlockOut& o = out[b];
+    const bool fin = isfinite(trace);
+    o.trace = trace;
+    // skip 1: trace shortcut; 3: non-finite trace (no LU, NaN result)
+    o.skip = fabs(trace) < 1e-8 ? 1 : (fin ? 0 : 3);
+    o.logdet = NAN;
+    o.frob2 = o.tr2 = 0;
+    o.status = *status;   // of the whole batch: it comes back with the results
+    o.delta = allow;
+    o.tile0 = lo_s >> 3;
+    o.tiles = o.skip || hi_s < 0 ? 0 : (hi_s >> 3) - (lo_s >> 3) + 1;
+    o.etr = fin && trace > 0 ? ilogb(trace) : 0;
+    // a chunk of a row is left out where √c < 2^-68 √tr: with any other row
+    // it adds less than 2^-68 tr to an element of G
+    o.emin = o.etr - 137;
+    if (dense) desc[b].N = 16 * o.tiles;
+}
+
+// The band of -G = -F Fᵀ on FP64 MFMA (v_mfma_f64_16x16x4f64): a workgroup takes
+// the four column tiles 4 s .. 4 s + 3 and for each its BAND_TILES tiles on
+// and below the diagonal (one column per wavefront, seven accumulators, the
+// column's own tile being both operands of the diagonal one); the rows of all
+// ten tiles go through LDS, 16 of F's columns per double-buffered stage.
+// Only chunks of 16 degrees in which some pair of the workgroup's rows has a
+// product of norms above 2^-68 tr are read (R/L = 200: a third of them).
+// The chunks left are cut into GRAM_SPLIT equal runs, each summed from zero
+// and added in order; a batch too small to fill the GPU gives each run its
+// own workgroup (partial sums added by k_gram_sum in the same order, so the
+// bits do not depend on the batch).
+__global__ void __launch_bounds__(256) k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                              const BlockOut* __restrict__ out, int split, int delta_only)
+{
+    constexpr int NR = BAND_TILES + 3, RW = 16 * NR, PITCH = RW + 16, KS = 16;
+    constexpr int LD2 = RW / 2, PER = KS * LD2 / 256;   // 16-byte loads per lane and stage
+    static_assert(KS * LD2 % 256 == 0, "whole loads");
+    __shared__ double S[2][KS][PITCH];
+    __shared__ int list[MAX_CHUNKS];
+    __shared__ int nlist;
+    const int b = blockIdx.y;
+    const BlockDesc& d = desc[b];
+    const BlockOut& o = out[b];
+    const int T = o.tiles, J0 = 4 * ((int)blockIdx.x / split), run = blockIdx.x % split;
+    if (o.skip || J0 >= T || (delta_only && !o.delta)) return;
+    const int nP = d.n_waves * 64, nT = nP >> 3, nt = min(NR, T - J0), ncol = min(4, T - J0);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
+    // the chunks that count, with the mask of the tiles that are not zero
+    if (wv == 0) {
+        const int* act = at<int>(arena, d.off_act) + o.tile0 + J0;
+        int n = 0;
+        for (int c0 = 0; c0 < d.n_chunks; c0 += 64) {
+            const int c = c0 + lane;
+            int er = NO_EXP, ec = NO_EXP, mask = 0;
+            if (c < d.n_chunks)
+                for (int t = 0; t < nt; t++) {
+                    const int e = act[(int64_t)c * nT + t];
+                    er = max(er, e);
+                    if (t < ncol) ec = max(ec, e);
+                    if (e >= o.emin) mask |= 1 << t;
+                }
+            const bool ok = er + ec >= 2 * o.etr - 136;
+            const unsigned long long bal = __ballot(ok);
+            if (ok) list[n + __popcll(bal & ((1ull << lane) - 1))] = c | (mask << 16);
+            n += __popcll(bal);
+        }
+        if (lane == 0) nlist = n;
+    }
+    __syncthreads();
+    const int64_t ldf = 2 * (int64_t)nP;
+    const double* F = at<double>(arena, d.off_rows) + 16 * (int64_t)(o.tile0 + J0);
+    double4_t tot[BAND_TILES];
+#pragma unroll
+    for (int r = 0; r < BAND_TILES; r++) tot[r] = (double4_t){0, 0, 0, 0};
+    typedef double double2_t __attribute__((ext_vector_type(2)));
+    double2_t pf[PER];
+    const int g0 = split > 1 ? run : 0, g1 = split > 1 ? run + 1 : GRAM_SPLIT;
+    for (int g = g0; g < g1; g++) {
+        const int s0 = 2 * (nlist * g / GRAM_SPLIT), s1 = 2 * (nlist * (g + 1) / GRAM_SPLIT);
+        double4_t acc[BAND_TILES];
+#pragma unroll
+        for (int r = 0; r < BAND_TILES; r++) acc[r] = (double4_t){0, 0, 0, 0};
+        auto fetch = [&](int s) {
+            const int en = list[s >> 1];
+            const double* Fs = F + (int64_t)(32 * (en & 0xffff) + 16 * (s & 1)) * ldf;
+#pragma unroll
+            for (int t = 0; t < PER; t++) {
+                const int i = tid + 256 * t, kk = i / LD2, q = i % LD2;
+                pf[t] = (en >> (16 + (q >> 3))) & 1 ? *reinterpret_cast<const double2_t*>(Fs + kk * ldf + 2 * q)
+                                                    : (double2_t){0, 0};
+            }
+        };
+        if (s0 < s1) fetch(s0);
+        for (int s = s0; s < s1; s++) {
+            double(*W)[PITCH] = S[s & 1];
+#pragma unroll
+            for (int t = 0; t < PER; t++) {
+                const int i = tid + 256 * t;
+                *reinterpret_cast<double2_t*>(&W[i / LD2][2 * (i % LD2)]) = pf[t];
+            }
+            __syncthreads();   // the other buffer's readers have passed the barrier before this one
+            if (s + 1 < s1) fetch(s + 1);
+            if (wv < ncol) {
+#pragma unroll
+                for (int kk = 0; kk < KS; kk += 4) {
+                    const double* w = &W[kk + lk][16 * wv + li];
+                    const double cv = w[0];
+#pragma unroll
+                    for (int r = 0; r < BAND_TILES; r++)
+                        acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv, w[16 * r], acc[r], 0, 0, 0);
+                }
+            }
+        }
+        // the stage buffers are free for the next run's first stage only when
+        // all wavefronts are done with this run's last one
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < BAND_TILES; r++) tot[r] += acc[r];
+    }
+    if (wv >= ncol) return;
+    // lane l, register q: column l/16 + 4q of the column tile, row l%16; tiles
+    // are kept column by column
+    double* B = at<double>(arena, split > 1 ? d.off_part + (int64_t)run * nT * (BAND_TILES * 256 * 8) : d.off_band)
+              + (int64_t)(J0 + wv) * (BAND_TILES * 256);
+#pragma unroll
+    for (int r = 0; r < BAND_TILES; r++)
+        if (J0 + wv + r < T) {
+#pragma unroll
+            for (int q = 0; q < 4; q++) B[r * 256 + 64 * q + lane] = split > 1 ? tot[r][q] : -tot[r][q];
+        }
+}
+
+__global__ void __launch_bounds__(256) k_gram_sum(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                  const BlockOut* __restrict__ out, int delta_only)
+{
+    const int b = blockIdx.y;
+    const BlockDesc& d = desc[b];
+    const BlockOut& o = out[b];
+    const int J = blockIdx.x / BAND_TILES, r = blockIdx.x % BAND_TILES;
+    if (o.skip || J + r >= o.tiles || (delta_only && !o.delta)) return;
+    const int64_t per = (int64_t)(d.n_waves * 8) * (BAND_TILES * 256);
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const double* P = at<double>(arena, d.off_part) + i;
+    double s = 0;
+#pragma unroll
+    for (int g = 0; g < GRAM_SPLIT; g++) s += P[g * per];
+    at<double>(arena, d.off_band)[i] = -s;
+}
+
+// log det(1 - G) of one block by LDLᵀ without pivoting (1 - G is symmetric
+// positive definite, so the elimination is stable in any order), in the
+// delta form: the matrix holds -G, pivots are u = 1 + d with d the stored
+// diagonal, and log u = log1p(d) keeps the accuracy of small blocks.  One
+// workgroup of eight wavefronts; the seven tile columns of the active band
+// live in LDS (100 KB), the next one is loaded while a column is eliminated.
+// Per tile column: wavefronts 0 and 1 factor its 16 columns, one lane per
+// row (the 16 diagonal rows in both, so that no other exchange is needed
+// than lane broadcasts), wavefront 2 takes the logs of the column before;
+// then all update the up to 21 tiles behind it on MFMA.  Bound by the chain
+// of 16 pivots per column.
+// mercator: the LU-mode rule of src/matrix.c:489-505 first (||M||_F² = tr M² =
+// Σ G_ij²; skip = 2: the host returns the two-term series).
+__global__ void __launch_bounds__(512) k_band_ldl(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                  BlockOut* __restrict__ out, int mercator)
+{
+    constexpr int NW = 8, NTH = 64 * NW, BT = BAND_TILES, COL = BT * 256;
+    __shared__ double S[BT * COL];
+    __shared__ double us[2][16], ds[2][16];
+    __shared__ double red[NTH];
+    const int b = blockIdx.x;
+    const BlockDesc& d = desc[b];
+    BlockOut& o = out[b];
+    const int T = o.tiles;
+    if (o.skip || !o.delta || T <= 0) return;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
+    const double* __restrict__ B = at<double>(arena, d.off_band);
+    if (mercator) {
+        double f = 0;
+        for (int64_t i = tid; i < (int64_t)T * COL; i += NTH) {
+            const int r = (int)(i % COL) >> 8, J = (int)(i / COL);
+            if (J + r < T) f += (r ? 2.0 : 1.0) * (B[i] * B[i]);
+        }
+        red[tid] = f;
+        __syncthreads();
+        for (int s = NTH / 2; s > 0; s >>= 1) {
+            if (tid < s) red[tid] += red[tid + s];
+            __syncthreads();
+        }
+        const double f2 = red[0], norm = sqrt(f2);
+        bool take = false;
+        if (norm < 1) {
+            const double merc = -o.trace - f2 / 2, err = fabs(norm * norm / 2 + norm + log1p(-norm));
+            take = fabs(err / merc) < 1e-8;
+        }
+        __syncthreads();
+        if (tid == 0) {
+            o.frob2 = o.tr2 = f2;
+            if (take) o.skip = 2;
+        }
+        if (take) return;
+    }
+    for (int K = 0; K < BT && K < T; K++)
+        for (int i = tid; i < COL; i += NTH) S[K * COL + i] = B[(int64_t)K * COL + i];
+    __syncthreads();
+    double ls = 0, lc = 0;   // wavefront 2, lanes 0 .. 15: Σ log u in double-double
+    auto add_log = [&](int J) {
+        const double dv = ds[J & 1][li];
+        const double v = dv > -0.5 ? log1p(dv) : log(fabs(1.0 + dv));
+        double t, e;
+        two_sum(ls, v, t, e);
+        ls = t;
+        lc += e;
+    };
+    constexpr int PFN = (COL + NTH - 1) / NTH;
+    double pf[PFN];
+    for (int J = 0; J < T; J++) {
+        const int nb = min(BT - 1, T - 1 - J), sj = J % BT;
+        const bool more = J + BT < T;
+        if (more) {
+#pragma unroll
+            for (int s = 0; s < PFN; s++)
+                if (tid + s * NTH < COL) pf[s] = B[(int64_t)(J + BT) * COL + tid + s * NTH];
+        }
+        if (wv < 2) {
+            const int pr = wv * 48 + lane - 16;
+            const bool dg = lane < 16, on = dg || pr < nb * 16;
+            double* tp = S + sj * COL + (dg ? lane : (1 + (pr >> 4)) * 256 + (pr & 15));
+            double a[16];
+#pragma unroll
+            for (int t = 0; t < 16; t++) a[t] = on ? tp[16 * t] : 0.0;
+#pragma unroll
+            for (int t = 0; t < 16; t++) {
+                const double ru = rcp_nr(1.0 + lane_d(a[t], t));
+                const double l = lane > t ? a[t] * ru : 0.0;
+#pragma unroll
+                for (int j = t + 1; j < 16; j++) a[j] = fma(-l, lane_d(a[j], t), a[j]);
+                a[t] = lane > t ? l : a[t];
+            }
+            if (!dg && on) {
+#pragma unroll
+                for (int t = 0; t < 16; t++) tp[16 * t] = a[t];
+            }
+            if (wv == 0 && dg) {
+                double dv = a[0];
+#pragma unroll
+                for (int t = 1; t < 16; t++) dv = lane == t ? a[t] : dv;
+                us[J & 1][lane] = 1.0 + dv;
+                ds[J & 1][lane] = dv;
+            }
+        } else if (wv == 2 && J > 0 && lane < 16) {
+            add_log(J - 1);
+        }
+        __syncthreads();
+        // tile (I, K) of the columns behind: -= L_I u L_Kᵀ
+        const double* Lc = S + sj * COL;
+        for (int i = wv; i < nb * (nb + 1) / 2; i += NW) {
+            int I = 1, K = i;
+            while (K >= I) K -= I++;
+            K++;
+            double* C = S + ((J + K) % BT) * COL + (I - K) * 256;
+            double4_t acc;
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[q] = C[64 * q + lane];
+#pragma unroll
+            for (int kk = 0; kk < 16; kk += 4) {
+                const int e = 16 * (kk + lk) + li;
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Lc[K * 256 + e] * us[J & 1][kk + lk], -Lc[I * 256 + e], acc,
+                                                           0, 0, 0);
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) C[64 * q + lane] = acc[q];
+        }
+        __syncthreads();
+        if (more) {
+#pragma unroll
+            for (int s = 0; s < PFN; s++)
+                if (tid + s * NTH < COL) S[sj * COL + tid + s * NTH] = pf[s];
+        }
+    }
+    if (wv != 2) return;
+    if (lane < 16) add_log(T - 1);
+    else ls = lc = 0;
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) {
+        const double so = __shfl_xor(ls, off), co = __shfl_xor(lc, off);
+        double t, e;
+        two_sum(ls, so, t, e);
+        ls = t;
+        lc = (lc + co) + e;
+    }
+    if (lane == 0) o.logdet = ls + lc;
+}
+
+// -G dense, column-major (zero outside the band), for the LU's kernels:
+// 1 - G (the unit diagonal on it) for blocks of the pivoted LU; full = 0:
+// rows from the column's 64-row diagonal block on.  The diagonal of G goes
+// to off_diag.
+__global__ void __launch_bounds__(256) k_band_dense(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                    const BlockOut* __restrict__ out, int full)
+{
+    const int b = blockIdx.z;
+    const BlockDesc& d = desc[b];
+    const int N = d.N, j = blockIdx.y;
+    if (out[b].skip || j >= N) return;
+    const double* B = at<double>(arena, d.off_band);
+    double* A = at<double>(arena, d.off_mat) + (int64_t)j * d.lda;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= N || (!full && i < (j & ~63))) return;
+    const int I = i >> 4, J = j >> 4, r = I - J;
+    double v = 0;
+    if (r >= 0 && r < BAND_TILES) v = B[((int64_t)J * BAND_TILES + r) * 256 + (j & 15) * 16 + (i & 15)];
+    else if (r < 0 && -r < BAND_TILES) v = B[((int64_t)I * BAND_TILES - r) * 256 + (i & 15) * 16 + (j & 15)];
+    if (i == j) {
+        at<double>(arena, d.off_diag)[i] = -v;
+        if (!out[b].delta) v += 1.0;
+    }
+    A[i] = v;
+}
+
+// M = FᵀF (mode 1) or -M (mode 0), column-major, on FP64 MFMA: 64 x 64 tiles of
+// four wavefronts of 32 x 32, over all nodes; the operands are rows of F's
+// storage (a degree's values at consecutive nodes), turned in LDS.  Each
+// element sums the same products in the same order as its mirror.  lower:
+// tiles above the diagonal are not written.
+__global__ void __launch_bounds__(256) k_wave_matrix(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                     const BlockOut* __restrict__ out, int mode, int lower)
+{
+    constexpr int KS = 16, PITCH = 64 + 16;
+    __shared__ double SA[KS][PITCH], SB[KS][PITCH];
+    const int b = blockIdx.z;
+    const BlockDesc& d = desc[b];
+    const int N = 2 * d.ldim, m0 = 64 * blockIdx.x, n0 = 64 * blockIdx.y;
+    if (m0 >= N || n0 >= N || (lower && m0 < n0) || (mode == 0 && out[b].skip)) return;
+    const int64_t ldf = 2 * (int64_t)d.n_waves * 64;
+    const double* F = at<double>(arena, d.off_rows);
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
+    const int wr = 32 * (wv & 1), wc = 32 * (wv >> 1);
+    double4_t acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[i][j] = (double4_t){0, 0, 0, 0};
+    // F's storage holds 32 ceil(ldim/16) rows, so a row tile's last rows may
+    // lie past it: they are taken as zero
+    const int nrow = 32 * d.n_chunks;
+    for (int64_t s = 0; s < ldf; s += KS) {
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int i = tid + 256 * t, r = i >> 3, q = 2 * (i & 7);
+            const double2 z = make_double2(0, 0);
+            const double2 va = m0 + r < nrow ? *reinterpret_cast<const double2*>(F + (m0 + r) * ldf + s + q) : z;
+            const double2 vb = n0 + r < nrow ? *reinterpret_cast<const double2*>(F + (n0 + r) * ldf + s + q) : z;
+            SA[q][r] = va.x;
+            SA[q + 1][r] = va.y;
+            SB[q][r] = vb.x;
+            SB[q + 1][r] = vb.y;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < KS; kk += 4) {
+            double av[2], bv[2];
+#pragma unroll
+            for (int i = 0; i < 2; i++) av[i] = SA[kk + lk][wr + 16 * i + li];
+#pragma unroll
+            for (int j = 0; j < 2; j++) bv[j] = SB[kk + lk][wc + 16 * j + li];
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bv[j], av[i], acc[i][j], 0, 0, 0);
+        }
+    }
+    // swapped operands: lane l, register q: row wr + 16i + l%16, column wc + 16j + l/16 + 4q
+    double* A = at<double>(arena, d.off_mat);
+    double* dg = at<double>(arena, d.off_diag);
+#pragma unroll
+    for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int row = m0 + wr + 16 * i + li, col = n0 + wc + 16 * j + lk + 4 * q;
+                if (row >= N || col >= N) continue;
+                double v = acc[i][j][q];
+                if (row == col) dg[row] = v;
+                if (mode == 0) v = row == col && !out[b].delta ? 1.0 - v : -v;
+                A[row + (int64_t)col * d.lda] = v;
+            }
+}
+
+}  // namespace capsd
+
+using namespace capsd;
+
+extern "C" {
+
+void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const BlockDesc* desc, char* arena, int nblocks,
+                             int max_waves, int* status, hipStream_t s)
+{
+    const int gx = max_waves > (max_mie + 63) / 64 ? max_waves : (max_mie + 63) / 64;
+    hipLaunchKernelGGL(k_wave_start, dim3(gx, ntab + nblocks), dim3(64), 0, s, (const MieDesc*)tabs, ntab, desc,
+                       arena, status);
+}
+
+// max_wq: largest n_waves ceil(n_chunks/4) of the blocks
+void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_wq,
+                             hipStream_t s)
+{
+    hipLaunchKernelGGL(k_wave_rows<false>, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena, out, 0);
+}
+
+void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_wq, int all,
+                            hipStream_t s)
+{
+    hipLaunchKernelGGL(k_wave_rows<true>, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena, out, all);
+}
+
+void capsd_launch_wave_window(BlockDesc* desc, char* arena, BlockOut* out, const int* status, int nblocks, int allow,
+                              int dense, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_wave_window, dim3(nblocks), dim3(256), 0, s, desc, arena, out, status, allow, dense);
+}
+
+// The band of -G; split != 0: one workgroup per run of chunks and a sum
+void capsd_launch_gram(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves, int split,
+                       int delta_only, hipStream_t s)
+{
+    const int T = max_waves * 8, ns = split ? GRAM_SPLIT : 1;
+    hipLaunchKernelGGL(k_gram, dim3((T + 3) / 4 * ns, nblocks), dim3(256), 0, s, desc, arena, out, ns, delta_only);
+    if (split)
+        hipLaunchKernelGGL(k_gram_sum, dim3(T * BAND_TILES, nblocks), dim3(256), 0, s, desc, arena, out, delta_only);
+}
+
+void capsd_launch_band_ldl(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int mercator, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_band_ldl, dim3(nblocks), dim3(512), 0, s, desc, arena, out, mercator);
+}
+
+void capsd_launch_band_dense(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves,
+                             int full, hipStream_t s)
+{
+    const int N = max_waves * 128;
+    hipLaunchKernelGGL(k_band_dense, dim3((N + 255) / 256, N, nblocks), dim3(256), 0, s, desc, arena, out, full);
+}
+
+void capsd_launch_wave_matrix(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_ldim,
+                              int mode, int lower, hipStream_t s)
+{
+    const int t = (2 * max_ldim + 63) / 64;
+    hipLaunchKernelGGL(k_wave_matrix, dim3(t, t, nblocks), dim3(256), 0, s, desc, arena, out, mode, lower);
+}
+
+}  // extern "C"

@@ -149,7 +149,7 @@ void caps_fresnel(caps_t *self, double xi_, double k_, double *r_TE, double *r_T
 
 /* ---- round-trip matrix and determinant: src/include/libcaps.h:145-150 -- */
 
-/* Builds the whole block on the GPU (Mie, K, I, matrix) and keeps a host
+/* Builds the whole matrix on the GPU and keeps a host
  * copy.  Aborts if xi_ <= 0.  Reference: src/libcaps.c:673-697. */
 caps_M_t *caps_M_init(caps_t *self, int m, double xi_);
 /* Element M^{(m)}_{l1 l2}(p1,p2), p = 'E' or 'M', lmin <= l1,l2 < lmin+ldim.
@@ -233,7 +233,9 @@ int caps_logdetD_batch(caps_t *self, const double *xi_, const int *m, int n, dou
  * build one caps object per geometry, src/caps.c:869-957, at 913). */
 int capsx_logdetD_multi(caps_t *const *objs, const double *xi_, const int *m, int n, double *out);
 
-/* Extension: LU schedule of the determinant stage.  levels 1 = 64-column
+/* Extension: LU schedule of dense matrices (kernel_logdet, the ξ = 0 blocks,
+ * device matrices; and of blocks while a schedule is fixed by
+ * capsx_lu_config: their Gram matrix is then factored dense).  levels 1 = 64-column
  * steps, 2 = 128-column steps of two panels with one K = 128 trailing
  * update, 3 = 256-column steps of four panels with one K = 256 update;
  * streams = groups of blocks factored on separate HIP streams; xcd =
@@ -292,8 +294,10 @@ int capsx_lu_time(int dim, int n, int reps, int levels, int streams, int xcd, in
 int capsx_lu_logdet_batch_noalloc(double *dA, int dim, int lda, int n, double *d_logdet, void *stream);
 
 /* Extension: per-stage timing of the last batch on this caps object, in
- * milliseconds: [0] Mie, [1] K, [2] I, [3] assembly, [4] LU, [5] total
- * (HIP events on the library's stream). */
+ * milliseconds (HIP events on the library's stream): [0] Mie coefficients and
+ * quadrature nodes, [1] row norms, trace and window, [2] rows of the
+ * wave-number factor, [3] matrix, [4] LU, [5] total; of a block's K and I
+ * tables [0] prefactors, [1] K, [2] I. */
 void caps_last_timing(caps_t *self, double ms[6]);
 
 /* Extension: free energy of the plane-sphere system at temperature T (K),
@@ -470,17 +474,17 @@ int capsx_lu_time_form(int dim, int n, int reps, int levels, int streams, int xc
 /* Test hook: D = A(16x4) B(4x16) through one FP64 MFMA instruction (the
  * register layout check).  Returns 0 on success. */
 int capsx_mfma_probe(const double *A, const double *B, double *D);
-/* Diagnostics: HIP events around every trailing-update launch (on != 0). */
+/* Diagnostics: HIP events around every trailing-update launch (on != 0);
+ * blocks then take the LU's kernels on the dense Gram matrix. */
 void capsx_profile(caps_t *self, int on);
 /* Accumulated statistics since the last reset: out[0..5] stage milliseconds
- * (Mie, K, I, assembly, LU, total; the Mie kernel runs beside the K
- * quadrature, whose time is what it adds after the Mie kernel ends),
- * out[6] blocks, out[7] blocks factored,
- * out[8] algorithmic LU flops, out[9] batches, out[10] I integrals; with
- * capsx_profile on, out[11..14] the milliseconds, algorithmic flops,
- * launches and algorithmic bytes of the trailing updates run by
- * k_lu_gemm_dma, out[15] the milliseconds of the other trailing-update
- * launches (k_lu_gemm tiles for regions one panel wide or high). */
+ * (as caps_last_timing), out[6] blocks, out[7] blocks factored, out[8] flops
+ * of their factorizations (of the band of the Gram matrix, or dense), out[9]
+ * batches, out[10] I integrals of tables; with capsx_profile on, out[11..14]
+ * the milliseconds, algorithmic flops, launches and algorithmic bytes of the
+ * trailing updates run by k_lu_gemm_dma, out[15] the milliseconds of the
+ * other trailing-update launches (k_lu_gemm tiles for regions one panel wide
+ * or high). */
 void capsx_stats(caps_t *self, double out[16]);
 void capsx_stats_reset(caps_t *self);
 

@@ -1,0 +1,105 @@
+"""The wave-number factor of the round-trip matrix (M = FᵀF, log det(1 - FᵀF) =
+log det(1 - F Fᵀ)) on the GPU, through the C ABI: the banded Gram matrix
+against the matrix M itself and against the Gram matrix run dense through
+the LU's kernels, at the edges of its tiles, chunks and windows.
+
+Tolerance.  M comes from the same rows F.  numpy's eigenvalues of M carry an
+absolute error of about N eps ||M|| <= N eps tr M, so Σ log1p(-λ) carries N eps
+relative to tr M <= |log det|/1, times 1/(1 - λ_max) (below 20 here); the
+band's left-out elements, the window and the factorization add less than
+1e-13: 20 N eps + 1e-12.  Dense against banded Gram matrix: the same
+elements, factored in another order, D <= 600 rows: 1e-12.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+EPS = 2.2e-16
+
+
+@pytest.fixture(scope="module")
+def ca():
+    import caps_amd
+    caps_amd.lib()
+    return caps_amd
+
+
+def make(ca, rbyl, ldim, metal, detalg=None):
+    c = ca.Caps(rbyl * 1e-6, 1e-6, ldim=ldim, detalg=detalg)
+    if metal:
+        c.set_drude(9.0, 0.035)
+    return c
+
+
+# ldim 1 .. 17: fewer degrees than a chunk of 16, one more than one; 24 more
+# than 1.5 chunks; m above ldim and far from the window's start (lmin > m);
+# ξ = 900: e^{-ξ} is not a double; ξ = 1e-3: nodes up to x = 1e5; R/L = 0.5
+CASES = [(20, 120, 1.0, 0, 0), (20, 120, 1.0, 1, 1), (20, 121, 0.3, 3, 0), (1, 1, 0.1, 0, 0), (2, 2, 0.5, 1, 1),
+         (2, 16, 0.5, 0, 1), (2, 17, 0.5, 2, 0), (4, 24, 2.0, 5, 0), (0.5, 20, 0.2, 1, 0), (10, 60, 1e-3, 0, 1),
+         (10, 60, 1e-3, 2, 0), (300, 700, 2.0, 90, 0), (500, 300, 1.0, 60, 1), (500, 900, 900.0, 0, 0),
+         (500, 900, 900.0, 4, 1), (100, 503, 30.0, 12, 1), (60, 360, 0.01, 7, 0)]
+
+
+@pytest.mark.parametrize("rbyl,ldim,xi,m,metal", CASES)
+def test_band_matches_matrix(ca, rbyl, ldim, xi, m, metal):
+    c = make(ca, rbyl, ldim, metal)
+    v, tr, fl = c.logdetD_batch([xi], [m], info=True)
+    M, _, _ = c.matrix(xi, m)
+    assert np.array_equal(M, M.T)
+    t = np.trace(M)
+    assert abs(tr[0] / t - 1) < 1e-12, (tr[0], t)
+    if abs(t) < 1e-8:
+        assert (fl[0] & 3) == 1 and v[0] == -tr[0]
+        return
+    lam = np.linalg.eigvalsh(M)
+    assert lam[-1] < 0.95
+    ref = float(np.sum(np.log1p(-lam)))
+    assert fl[0] == 4 and abs(v[0] / ref - 1) < 20 * len(M) * EPS + 1e-12, (v[0], ref)
+
+
+def test_band_matches_dense_gram(ca):
+    """The same Gram matrix through the LU's kernels: a schedule fixed by
+    capsx_lu_config runs the symmetric delta form, CAPS_AMD_LU_SYM=0 the
+    general one (the whole matrix); LU mode with its Mercator rule."""
+    import os
+    from caps_amd import autotune as at
+    for rbyl, ldim, metal, detalg in ((20, 120, 0, None), (50, 251, 1, "LU"), (200, 1200, 1, None)):
+        c = make(ca, rbyl, ldim, metal, detalg)
+        ms = list(range(0, 40, 3))
+        xs = [0.8 * rbyl] * len(ms)
+        v, tr, fl = c.logdetD_batch(xs, ms, info=True)
+        try:
+            at.set_config(1, 1, 0, 128)
+            w, tw, fw = c.logdetD_batch(xs, ms, info=True)
+        finally:
+            at.set_config(0)
+        os.environ["CAPS_AMD_LU_SYM"] = "0"
+        try:
+            g, _, fg = c.logdetD_batch(xs, ms, info=True)
+        finally:
+            os.environ.pop("CAPS_AMD_LU_SYM")
+        assert np.array_equal(tr, tw) and np.array_equal(fl, fw) and np.array_equal(fl, fg)
+        assert np.max(np.abs(w / v - 1)) < 1e-12 and np.max(np.abs(g / v - 1)) < 1e-12
+
+
+def test_band_batch_equals_single(ca):
+    """Partial sums of a block run alone (its chunks spread over workgroups)
+    and of a large batch (one workgroup per strip) are the same bits, and so
+    are batches of mixed geometries."""
+    a, b = make(ca, 40, 240, 1), make(ca, 90, 470, 0)
+    objs = [a, b] * 40
+    xs = np.repeat(np.linspace(0.5, 60, 40), 2)
+    ms = np.arange(80) % 23
+    v = ca.logdetD_multi(objs, xs, ms)
+    for i in range(0, 80, 7):
+        assert objs[i].logdetD(xs[i], int(ms[i])) == v[i], i
+
+
+def test_cholesky_mode_takes_the_matrix(ca):
+    """CHOLESKY, whose shortcut rule looks at the lower triangle of M, factors
+    M itself; the same determinants as the Gram matrix (rounding of an LU of N
+    rows: 20 N eps + 1e-12)."""
+    c, h = make(ca, 30, 150, 1, "CHOLESKY"), make(ca, 30, 150, 1)
+    ms = [0, 1, 2, 5, 9]
+    v, w = c.logdetD_batch([1.5] * 5, ms), h.logdetD_batch([1.5] * 5, ms)
+    assert np.max(np.abs(v / w - 1)) < 20 * 300 * EPS + 1e-12
