@@ -40,9 +40,9 @@ struct BlockDesc {
     int64_t off_norm;   // n_chunks nP doubles: squared norms of the rows' chunks
     int64_t off_act;    // n_chunks nP/8 ints: exponent of a tile's largest of them
     int64_t off_dn;     // nP doubles: squared norms of the rows
+    int64_t off_deg;    // 16 n_chunks Deg: the degrees' constants
     int64_t off_rows;   // F: 32 n_chunks rows (degree; a_l, b_l) of 2 nP doubles
     int64_t off_band;   // nP/8 columns of BAND_TILES tiles of 16 x 16: -G
-    int64_t off_part;   // GRAM_SPLIT such bands: partial sums
     int64_t off_a0;     // nl + (2 nl - 1) doubles: parts of log a0 of I
     int64_t off_kpart;  // n_waves * nK * KPart
     int64_t off_k;      // 2 pols * nK * KEnt (K = m * 2^e), then 2 pols * nK
@@ -65,8 +65,12 @@ struct BlockDesc {
 // 0.1 .. 1000, ξ 1e-3 .. 300, both materials: no difference to the full
 // matrix above 1e-15).
 constexpr int BAND_TILES = 7;
-constexpr int GRAM_SPLIT = 8;    // runs of chunks summed apart (k_gram)
-constexpr int MAX_CHUNKS = 768;  // ldim <= 12288
+
+// Constants of one degree of a block's window (see degree() in waves.hip).
+struct Deg {
+    double c1, c2, l, t0, rt, ma, mb;
+    int e, pad_;
+};
 
 // One Mie table: degrees 1 .. L at one ξ of one object; at off: L doubles each
 // of log|a_l|, log|b_l| and the mantissas of √(a_l g_l), √(b_l g_l), g_l =
@@ -111,8 +115,7 @@ struct BlockOut {
                         // matrix), LU with partial pivoting
     int tile0, tiles;   // the nodes that matter: tiles of 8 nodes (G has
                         // 16 tiles rows)
-    int etr, emin;      // exponent of the trace; of the smallest row chunk kept
-    int pad_;
+    int etr;            // exponent of the trace
 };
 
 }  // namespace capsd

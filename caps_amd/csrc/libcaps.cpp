@@ -36,10 +36,10 @@ struct capsx_mlp;
 extern "C" {
 void capsx_mlp_predict(capsx_mlp* h, const float* X, int n, float* Y);
 void capsd_launch_wave_start(const void*, int, int, const BlockDesc*, char*, int, int, int*, hipStream_t);
-void capsd_launch_wave_norms(const BlockDesc*, char*, const BlockOut*, int, int, hipStream_t);
+void capsd_launch_wave_norms(const BlockDesc*, char*, int, int, hipStream_t);
 void capsd_launch_wave_window(BlockDesc*, char*, BlockOut*, const int*, int, int, int, hipStream_t);
-void capsd_launch_wave_rows(const BlockDesc*, char*, const BlockOut*, int, int, int, hipStream_t);
-void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, hipStream_t);
+void capsd_launch_wave_rows(const BlockDesc*, char*, int, int, hipStream_t);
+void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, int, hipStream_t);
 void capsd_launch_band_ldl(const BlockDesc*, char*, BlockOut*, int, int, hipStream_t);
 void capsd_launch_band_dense(const BlockDesc*, char*, const BlockOut*, int, int, int, hipStream_t);
 void capsd_launch_wave_matrix(const BlockDesc*, char*, const BlockOut*, int, int, int, int, hipStream_t);
@@ -554,7 +554,7 @@ struct BatchPlan {
     Job job = JOB_LOGDET;
     Form form = FORM_BAND;
     int dmode = 0;      // dense_mode of the determinant
-    int split = 0;      // k_gram's runs of chunks in workgroups of their own
+    int gram_cols = 4;  // k_gram's column tiles per workgroup
     // determinant forms the LU launches kernels for (capsd_launch_lu kinds):
     // 1 = pivoted, 2 = delta form, 6 = delta form of a symmetric matrix
     int lu_kinds = 6;
@@ -659,8 +659,9 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             d.off_norm = take(nc * nP * 8);
             d.off_act = take(nc * (nP / 8) * 4);
             d.off_dn = take(nP * 8);
-            d.off_rows = take(32 * nc * 2 * nP * 8);
-            if (p.form != FORM_M) d.off_band = take(nP / 8 * (capsd::BAND_TILES * 256) * 8);
+            d.off_deg = take(16 * nc * sizeof(capsd::Deg));
+            if (p.form == FORM_M) d.off_rows = take(32 * nc * 2 * nP * 8);
+            else d.off_band = take(nP / 8 * (capsd::BAND_TILES * 256) * 8);
             // nodes of a block that matter: about 0.8 of them, 32 per strip
             strips += (d.n_nodes + 39) / 40;
             d.N = p.form == FORM_M ? 2 * ldim : (int)(2 * nP);
@@ -686,13 +687,11 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
         p.max_nK = std::max(p.max_nK, d.nK);
         p.max_nl = std::max(p.max_nl, d.nl);
     }
-    // a batch whose strips of the band leave the GPU idle (fewer than 1.5 per
-    // CU) splits each into GRAM_SPLIT workgroups (one block, R/L = 200: 7)
-    p.split = det && p.form != FORM_M && strips < 384;
-    if (p.split)
-        for (int b = 0; b < p.n; b++)
-            c->h_desc[b].off_part = take((int64_t)capsd::GRAM_SPLIT * (c->h_desc[b].n_waves * 8) *
-                                         (capsd::BAND_TILES * 256) * 8);
+    // four columns per workgroup make 1.8 times as many rows as the band has,
+    // one column seven times in four times as many workgroups, which is faster
+    // as long as strips of four would be fewer than CUs (R/L = 200, four columns
+    // and one: 1 block 83 and 32 us, 32 blocks 89 and 87, 64 blocks 124 and 170)
+    if (strips < 256) p.gram_cols = 1;
     if (job != JOB_TABLES) {
         p.ntab = (int)tabs.size();
         for (int t = 0; t < p.ntab; t++) {
@@ -824,18 +823,19 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
     capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.max_waves, c->d_status, s);
     mark(1);
     if (det) {
-        capsd_launch_wave_norms(c->d_desc, c->arena, c->d_out, n, p.max_wq, s);
+        capsd_launch_wave_norms(c->d_desc, c->arena, n, p.max_wq, s);
         capsd_launch_wave_window(c->d_desc, c->arena, c->d_out, c->d_status, n, piv ? 0 : g_delta_mode,
                                  p.form == FORM_GRAM, s);
     }
     mark(2);
-    capsd_launch_wave_rows(c->d_desc, c->arena, c->d_out, n, p.max_wq, p.form == FORM_M, s);
+    if (p.form == FORM_M) capsd_launch_wave_rows(c->d_desc, c->arena, n, p.max_wq, s);
     mark(3);
     if (p.form == FORM_M)
         capsd_launch_wave_matrix(c->d_desc, c->arena, c->d_out, n, p.max_ldim, det ? 0 : 1,
                                  det && !piv && p.lu_kinds == 6, s);
     else
-        capsd_launch_gram(c->d_desc, c->arena, c->d_out, n, p.max_waves, p.split, p.form == FORM_BAND, s);
+        capsd_launch_gram(c->d_desc, c->arena, c->d_out, n, p.max_waves, (p.max_ldim + 15) / 16, p.gram_cols,
+                          p.form == FORM_BAND, s);
     // the symmetric delta-form LU reads nothing above the diagonal outside its
     // 64 x 64 diagonal blocks; k_frobenius (LU mode) reads all of the matrix
     if (p.form == FORM_GRAM)
@@ -858,7 +858,7 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
 std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
 {
     struct {
-        int n, ntab, maxN, max_ldim, max_waves, max_wq, max_mie, max_nK, max_nl, kseg, job, form, dmode, split;
+        int n, ntab, maxN, max_ldim, max_waves, max_wq, max_mie, max_nK, max_nl, kseg, job, form, dmode, gram_cols;
         int is_pr, lu_kinds, delta_mode;
         int levels, streams, xcd, tile;
         int lu_bnd[MAX_LU_STREAMS + 1], lu_gN[MAX_LU_STREAMS];   // the LU's stream groups (lu_groups)
@@ -878,7 +878,7 @@ std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
     k.job = p.job;
     k.form = p.form;
     k.dmode = p.dmode;
-    k.split = p.split;
+    k.gram_cols = p.gram_cols;
     if (p.job == JOB_TABLES) {
         k.kseg = k_segments(p);
         k.is_pr = c->h_desc[0].is_pr;

@@ -585,8 +585,8 @@ __global__ void __launch_bounds__(256) k_dominance_fix(const BlockDesc* __restri
 // ξ = 0 blocks (EE, MM, plasma MM; src/libcaps.c:860-941): elements
 // M_ij = exp(h_i + h_j + T_{i+j}) with per-row terms h (n doubles) and
 // per-(l1+l2) terms T (2n - 1 doubles), both at arena offset off_tab.
-// Writes -M column-major (leading dimension lda; the LU's delta form, see
-// k_assemble), the diagonal of M, and per 64-row tile (blockIdx.x) the
+// Writes -M column-major (leading dimension lda; the LU factors 1 + this
+// without forming it), the diagonal of M, and per 64-row tile (blockIdx.x) the
 // column sums of |M_ij|, i != j.  Lanes run down the columns (coalesced
 // stores), 64 x 4 per workgroup.
 __global__ void __launch_bounds__(256) k_fill_xi0(const BlockDesc* __restrict__ desc, char* __restrict__ arena,

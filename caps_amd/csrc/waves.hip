@@ -22,15 +22,13 @@
 //   k_wave_start   the Mie coefficients of each (object, ξ), and beside them
 //                  the nodes with the degree recurrence of P_l^m over all l,
 //                  whose state is kept at the start of every 16 degrees;
-//   k_wave_rows    F of 16 degrees x 64 nodes from such a state: first only
-//                  the squared norms (trace, window, activity), then the
-//                  rows of the blocks that need a determinant;
+//   k_wave_norms   the squared norms of F's rows per 16 degrees;
 //   k_wave_window  trace, trace shortcut, the nodes that matter;
-//   k_gram         the band of -G on FP64 MFMA;
+//   k_gram         the band of -G on FP64 MFMA, F's rows made on the spot;
 //   k_band_ldl     log det(1 - G): banded LDLᵀ, one workgroup per block;
 //   k_band_dense   -G as a dense matrix (schedules fixed by the caller, the
 //                  pivoted LU);
-//   k_wave_matrix  M = FᵀF itself (caps_M_init, CHOLESKY mode).
+//   k_wave_rows, k_wave_matrix  F, and M = FᵀF itself (caps_M_init, CHOLESKY mode).
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -46,9 +44,8 @@ __device__ __forceinline__ T* at(char* base, int64_t off) { return reinterpret_c
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
-// Row of node k and polarization p (0 TM, 1 TE) in F: tiles of 8 nodes, 8 TM
-// rows then 8 TE rows, so that a tile of 16 rows is the unit of the band.
-__device__ __forceinline__ int row_of(int k, int p) { return (k >> 3) * 16 + p * 8 + (k & 7); }
+// F's rows are ordered 2 k + p for node k and polarization p (0 TM, 1 TE): a
+// tile of 8 nodes is 16 rows, the unit of the band.
 
 // Exponent of what is zero whatever it is added to: 2^NO_EXP 2^E = 0.
 constexpr int NO_EXP = -(1 << 28);
@@ -116,8 +113,8 @@ __device__ void mie_entry(const MieDesc& t, char* __restrict__ arena, int l)
 // blockIdx.y < ntab: Mie coefficients of table blockIdx.y, one lane per l.
 // Else block blockIdx.y - ntab: 64 nodes per wavefront, one lane each; a
 // chain of one FMA per degree, 17 cycles a step (R/L = 200: 9 µs of a single
-// block), so the rest of F's work is left to k_wave_rows, which starts from
-// the states kept here and runs all degrees at once.
+// block), so the rest of F's work is left to the kernels that start from the
+// states kept here and take all chunks of degrees at once.
 __global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ tabs, int ntab,
                                                    const BlockDesc* __restrict__ desc, char* __restrict__ arena,
                                                    int* __restrict__ status)
@@ -200,98 +197,141 @@ __global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ t
     }
 }
 
-// F of degrees lmin + 16 c .. + 15 at 64 nodes (one lane each), four chunks c
-// per workgroup.  STORE = false: the nodes' squared norms over the chunk and
-// per tile of 8 nodes the exponent of the largest (c_k < 2^e).  STORE = true:
-// the rows themselves, F[2(l-lmin) + (0: a_l, 1: b_l)][row], of the blocks
-// without a trace shortcut; tiles that k_gram reads as zero (a chunk norm
-// below 2^emin, or outside the window) are not written.  all != 0: every
-// entry (k_wave_matrix).  Degrees past the window are zero.
-// VALU-bound: about 20 FP64 instructions per degree and lane.
-template <bool STORE>
-__global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                   const BlockOut* __restrict__ out, int all)
+// What one degree needs, the same for all nodes of a block: c1, c2 of
+// degree_step; t_l = (l x + t0) S_l - rt S_{l-1} (m = 0: t_l = P_l^1 = √(l(l+1)) S_l);
+// mantissas and exponent of the Mie factors (zero past the window).
+__device__ __forceinline__ Deg degree(const BlockDesc& d, char* arena, int l)
 {
-    const int b = blockIdx.y;
-    const BlockDesc& d = desc[b];
-    const int nq = (d.n_chunks + 3) / 4;
-    if ((int)blockIdx.x >= d.n_waves * nq) return;
-    if (STORE && !all && (out[b].skip || out[b].tiles <= 0)) return;
+    const int mm = d.m > 0 ? d.m : 1;
+    const double den = 1 / sqrt((l + 1.0 - mm) * (l + 1.0 + mm));
+    const double rt = sqrt(((double)l - mm) * ((double)l + mm));
+    Deg g;
+    g.c1 = (2.0 * l + 1) * den;
+    g.c2 = rt * den;
+    g.l = d.m > 0 ? l : 0;
+    g.t0 = d.m > 0 ? 0.0 : sqrt((double)l * (l + 1.0));
+    g.rt = d.m > 0 ? rt : 0.0;
+    const double* a = at<double>(arena, d.off_mie) + (l - 1);
+    const bool ok = l < d.lmin + d.ldim;
+    g.ma = ok ? a[2 * (int64_t)d.mie_L] : 0.0;
+    g.mb = ok ? a[3 * (int64_t)d.mie_L] : 0.0;
+    g.e = ok ? at<int>(arena, d.off_mie + 32 * (int64_t)d.mie_L)[l - 1] : NO_EXP;
+    g.pad_ = 0;
+    return g;
+}
+
+// 2^e for e < 1024, 0 below the normal numbers (what it multiplies is then
+// below 2^-700, its square 0).
+__device__ __forceinline__ double exp2i(int e) { return __hiloint2double(max(e + 1023, 0) << 20, 0); }
+
+// One degree at one node, up to the node's √r: the four products of (t_l, p_l)
+// and the Mie factors (a_l, b_l), and the step to the next degree.
+__device__ __forceinline__ void degree_rows(const Deg& g, double m, double x, double& p, double& pp, int E, double& ta,
+                                            double& pb, double& pa, double& tb)
+{
+    const double t = fma(fma(g.l, x, g.t0), p, -(g.rt * pp)), q = m * p;
+    const double u = exp2i(E + g.e), ua = u * g.ma, ub = u * g.mb;
+    ta = t * ua;
+    pb = q * ub;
+    pa = q * ua;
+    tb = t * ub;
+    degree_step(g.c1, g.c2, x, p, pp);
+}
+
+// The squared norms of F's rows over degrees lmin + 16 c .. + 15 at 128 nodes (two
+// per lane: half the reads of the degrees' constants), four chunks c per workgroup, and per tile of 8 nodes
+// the exponent of the largest (c_k < 2^e); the degrees' constants for k_gram.
+// VALU-bound: 17 FP64 instructions per degree and node.
+__global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict__ desc, char* __restrict__ arena)
+{
+    const BlockDesc& d = desc[blockIdx.y];
+    const int nq = (d.n_chunks + 3) / 4, nw = (d.n_waves + 1) / 2;
+    if ((int)blockIdx.x >= nw * nq) return;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wave = blockIdx.x % d.n_waves, c = (blockIdx.x / d.n_waves) * 4 + wv;
-    const int nP = d.n_waves * 64, nT = nP >> 3, k = wave * 64 + lane;
-    const int m = d.m, mm = m > 0 ? m : 1;
-    struct Deg {
-        double c1, c2, l, rt, ma, mb;
-        int e, pad_;
-        double tf;
-    };
+    const int wave = blockIdx.x % nw, c = (blockIdx.x / nw) * 4 + wv;
+    const int nP = d.n_waves * 64;
+    const double m = d.m;
     __shared__ Deg degs[4][16];
     const bool in = c < d.n_chunks;
     if (in && lane < 16) {
-        const int l = d.lmin + 16 * c + lane;
-        const double den = 1 / sqrt((l + 1.0 - mm) * (l + 1.0 + mm));
-        Deg g;
-        g.l = l;
-        g.rt = sqrt(((double)l - mm) * ((double)l + mm));
-        g.c1 = (2.0 * l + 1) * den;
-        g.c2 = g.rt * den;
-        const double* a = at<double>(arena, d.off_mie) + (l - 1);
-        const bool ok = l < d.lmin + d.ldim;
-        g.ma = ok ? a[2 * (int64_t)d.mie_L] : 0.0;
-        g.mb = ok ? a[3 * (int64_t)d.mie_L] : 0.0;
-        g.e = ok ? at<int>(arena, d.off_mie + 32 * (int64_t)d.mie_L)[l - 1] : NO_EXP;
-        g.tf = sqrt((double)l * (l + 1.0));   // m = 0: t_l = P_l^1 = √(l(l+1)) S_l
+        const Deg g = degree(d, arena, d.lmin + 16 * c + lane);
         degs[wv][lane] = g;
+        if (wave == 0) at<Deg>(arena, d.off_deg)[16 * c + lane] = g;
     }
     __syncthreads();
     if (!in) return;
-    const int64_t ci = (int64_t)c * nP + k;
-    const int tile = k >> 3;
-    int* act = at<int>(arena, d.off_act) + (int64_t)c * nT + tile;
-    bool st = true;
-    if (STORE && !all) {
-        const int t0 = out[b].tile0;
-        st = tile >= t0 && tile < t0 + out[b].tiles && *act >= out[b].emin;
-        if (!__any(st)) return;
+    const double* nd = at<double>(arena, d.off_node);
+    double x[2], p[2], pp[2], ntm[2], nte[2];
+    int E[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int k = min(wave * 128 + 64 * h + lane, nP - 1);   // (an odd last wave: not stored)
+        const int64_t ci = (int64_t)c * nP + k;
+        const double2 s = at<double2>(arena, d.off_ck)[ci];
+        x[h] = nd[k];
+        p[h] = s.x;
+        pp[h] = s.y;
+        E[h] = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[ci];
+        ntm[h] = nte[h] = 0;
     }
+#pragma unroll 4
+    for (int j = 0; j < 16; j++) {
+        const Deg& g = degs[wv][j];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            double ta, pb, pa, tb;
+            degree_rows(g, m, x[h], p[h], pp[h], E[h], ta, pb, pa, tb);
+            ntm[h] = fma(ta, ta, fma(pb, pb, ntm[h]));
+            nte[h] = fma(pa, pa, fma(tb, tb, nte[h]));
+            if ((j & 3) == 3) rescale(p[h], pp[h], E[h]);
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int k = wave * 128 + 64 * h + lane;
+        if (k >= nP) break;   // uniform over the wavefront
+        const double stm = nd[nP + k], ste = nd[2 * nP + k];
+        const double norm = stm * stm * ntm[h] + ste * ste * nte[h];
+        at<double>(arena, d.off_norm)[(int64_t)c * nP + k] = norm;
+        int e = norm > 0 ? ilogb(norm) + 1 : NO_EXP;   // a NaN norm: the trace is NaN
+        e = max(e, dpp_i<DPP_QUAD_X1>(e));
+        e = max(e, dpp_i<DPP_QUAD_X2>(e));
+        e = max(e, dpp_i<DPP_HALF_MIRROR>(e));
+        if ((lane & 7) == 0) at<int>(arena, d.off_act)[(int64_t)c * (nP >> 3) + (k >> 3)] = e;
+    }
+}
+
+// F itself, F[2(l-lmin) + (0: a_l, 1: b_l)][row], over 16 degrees and 64 nodes per
+// wavefront (k_wave_matrix; k_gram makes its own).
+__global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__ desc, char* __restrict__ arena)
+{
+    const BlockDesc& d = desc[blockIdx.y];
+    const int nq = (d.n_chunks + 3) / 4;
+    if ((int)blockIdx.x >= d.n_waves * nq) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int wave = blockIdx.x % d.n_waves, c = (blockIdx.x / d.n_waves) * 4 + wv;
+    const int nP = d.n_waves * 64, k = wave * 64 + lane;
+    const double m = d.m;
+    __shared__ Deg degs[4][16];
+    const bool in = c < d.n_chunks;
+    if (in && lane < 16) degs[wv][lane] = degree(d, arena, d.lmin + 16 * c + lane);
+    __syncthreads();
+    if (!in) return;
+    const int64_t ci = (int64_t)c * nP + k, ldf = 2 * (int64_t)nP;
     const double* nd = at<double>(arena, d.off_node);
     const double x = nd[k], stm = nd[nP + k], ste = nd[2 * nP + k];
     const double2 s = at<double2>(arena, d.off_ck)[ci];
     double p = s.x, pp = s.y;
     int E = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[ci];
-    const int64_t ldf = 2 * (int64_t)nP;
-    double* F = STORE ? at<double>(arena, d.off_rows) + 32 * (int64_t)c * ldf + row_of(k, 0) : nullptr;
-    double norm = 0;
+    double* F = at<double>(arena, d.off_rows) + 32 * (int64_t)c * ldf + 2 * k;
 #pragma unroll 4
     for (int j = 0; j < 16; j++) {
-        const Deg& g = degs[wv][j];
-        const double t = m > 0 ? fma(g.l * x, p, -(g.rt * pp)) : g.tf * p;
-        const double u = ldexp(1.0, E + g.e);
-        const double utm = u * stm, ute = u * ste, mp = d.m * p;
-        const double f0 = t * utm * g.ma, f1 = mp * utm * g.mb;   // TM row: a_l, b_l
-        const double f2 = mp * ute * g.ma, f3 = t * ute * g.mb;   // TE row
-        if (STORE) {
-            if (st) {
-                F[0] = f0;
-                F[8] = f2;
-                F[ldf] = f1;
-                F[ldf + 8] = f3;
-            }
-            F += 2 * ldf;
-        } else {
-            norm = fma(f0, f0, fma(f1, f1, fma(f2, f2, fma(f3, f3, norm))));
-        }
-        degree_step(g.c1, g.c2, x, p, pp);
+        double ta, pb, pa, tb;
+        degree_rows(degs[wv][j], m, x, p, pp, E, ta, pb, pa, tb);
+        *reinterpret_cast<double2*>(F) = make_double2(stm * ta, ste * pa);
+        *reinterpret_cast<double2*>(F + ldf) = make_double2(stm * pb, ste * tb);
+        F += 2 * ldf;
         if ((j & 3) == 3) rescale(p, pp, E);
-    }
-    if (!STORE) {
-        at<double>(arena, d.off_norm)[ci] = norm;
-        int e = norm > 0 ? ilogb(norm) + 1 : NO_EXP;   // a NaN norm: the trace is NaN
-        e = max(e, dpp_i<DPP_QUAD_X1>(e));
-        e = max(e, dpp_i<DPP_QUAD_X2>(e));
-        e = max(e, dpp_i<DPP_HALF_MIRROR>(e));
-        if ((lane & 7) == 0) *act = e;
     }
 }
 
@@ -360,139 +400,195 @@ __global__ void __launch_bounds__(256) k_wave_window(BlockDesc* __restrict__ des
     o.tile0 = lo_s >> 3;
     o.tiles = o.skip || hi_s < 0 ? 0 : (hi_s >> 3) - (lo_s >> 3) + 1;
     o.etr = fin && trace > 0 ? ilogb(trace) : 0;
-    // a chunk of a row is left out where √c < 2^-68 √tr: with any other row
-    // it adds less than 2^-68 tr to an element of G
-    o.emin = o.etr - 137;
     if (dense) desc[b].N = 16 * o.tiles;
 }
 
-// The band of -G = -F Fᵀ on FP64 MFMA (v_mfma_f64_16x16x4f64): a workgroup takes
-// the four column tiles 4 s .. 4 s + 3 and for each its BAND_TILES tiles on
-// and below the diagonal (one column per wavefront, seven accumulators, the
-// column's own tile being both operands of the diagonal one); the rows of all
-// ten tiles go through LDS, 16 of F's columns per double-buffered stage.
-// Only chunks of 16 degrees in which some pair of the workgroup's rows has a
-// product of norms above 2^-68 tr are read (R/L = 200: a third of them).
-// The chunks left are cut into GRAM_SPLIT equal runs, each summed from zero
-// and added in order; a batch too small to fill the GPU gives each run its
-// own workgroup (partial sums added by k_gram_sum in the same order, so the
-// bits do not depend on the batch).
-__global__ void __launch_bounds__(256) k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                              const BlockOut* __restrict__ out, int split, int delta_only)
+// The band of -G = -F Fᵀ on FP64 MFMA (v_mfma_f64_16x16x4f64): a workgroup of four
+// wavefronts takes NC column tiles and for each its BAND_TILES tiles on and
+// below the diagonal (the column's own tile is both operands of the diagonal
+// one).  The rows of these tiles are made on the spot, a chunk of 16 degrees
+// at a time, from the states that k_wave_start kept (20 bytes instead of 512
+// per node and chunk): eight tiles are the 64 lanes of a wavefront, which
+// makes degrees 4 w .. 4 w + 3; then the pairs are multiplied.  (Making the next
+// chunk in four more wavefronts beside the products gains nothing: FP64
+// instructions and FP64 MFMA do not overlap.  Bound by the two together:
+// 130 us without the products, 212 without the rows.)
+// A row's ridge covers a few chunks: a pair of tiles is multiplied over a
+// chunk only if the product of their largest chunk norms is at least 2^-60
+// tr (by Cauchy-Schwarz what is left out is smaller, below the last bit of
+// the trace; R/L = 200, NC = 4: 25 of 75 chunks per strip, 12 of 28 pairs).
+// The pairs that count in a chunk lie next to each other, so NC = 4 deals them
+// out along the diagonals: wavefront w has tile j + r of column j = (w + r) % 4, for r = 0
+// .. 6; the busiest one then has 3.4 on average of 2.9 (whole columns: 4.8).
+// The three pairs with the strip's ninth and tenth tile are a step of their
+// own over tiles 2 .. 9, where they count at all.
+// NC = 1 for batches that would leave CUs idle: two chunks per step in twice
+// the wavefronts, a pair each (one block of R/L = 200: 30 us; 38 a chunk at a
+// time).
+// An element sums the same products in the same order for either NC, so its
+// bits do not depend on the batch.
+// 222 blocks of R/L = 200: 296 us; with F's rows stored by a kernel of their
+// own and read back 478 + 124 us, bound by the loads' latency.
+template <int NC>
+__global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
+    k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena, const BlockOut* __restrict__ out, int delta_only)
 {
-    constexpr int NR = BAND_TILES + 3, RW = 16 * NR, PITCH = RW + 16, KS = 16;
-    constexpr int LD2 = RW / 2, PER = KS * LD2 / 256;   // 16-byte loads per lane and stage
-    static_assert(KS * LD2 % 256 == 0, "whole loads");
-    __shared__ double S[2][KS][PITCH];
-    __shared__ int list[MAX_CHUNKS];
+    static_assert(NC == 1 || NC == 4, "columns per workgroup");
+    constexpr int NR = NC + BAND_TILES - 1, NS = 8, PITCH = 16 * NS + 16, KS = 32;
+    constexpr int NG = NC == 4 ? 1 : 2, NW = 4 * NG;   // chunks per step, wavefronts
+    constexpr int PS = NC == 4 ? BAND_TILES : 1;       // pairs per wavefront
+    static_assert(NW * PS <= 32 && (NC == 4 || NW >= BAND_TILES), "a bit and a place for every pair");
+    static_assert(NR <= NS + 2, "tiles 0 .. 7 and 2 .. 9");
+    __shared__ double W[NG][KS][PITCH];   // [2 (l - l0) + (0: a_l, 1: b_l)][row of eight tiles]
+    alignas(16) __shared__ Deg degs[NG][16];
     __shared__ int nlist;
+    extern __shared__ int2 list[];    // chunk, first tile 0 or 2 (bit 10); pairs (bit PS w + i)
     const int b = blockIdx.y;
     const BlockDesc& d = desc[b];
     const BlockOut& o = out[b];
-    const int T = o.tiles, J0 = 4 * ((int)blockIdx.x / split), run = blockIdx.x % split;
+    const int T = o.tiles, J0 = NC * (int)blockIdx.x;
     if (o.skip || J0 >= T || (delta_only && !o.delta)) return;
-    const int nP = d.n_waves * 64, nT = nP >> 3, nt = min(NR, T - J0), ncol = min(4, T - J0);
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
-    // the chunks that count, with the mask of the tiles that are not zero
+    const int nP = d.n_waves * 64, nT = nP >> 3, nt = min(NR, T - J0);
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lk = lane >> 4;
+    // pair i of wavefront w: column col_of(w, i), tile col_of + row_of
+    auto col_of = [](int w, int i) { return NC == 4 ? (w + i) & 3 : 0; };
+    auto row_of = [](int w, int i) { return NC == 4 ? i : w; };
     if (wv == 0) {
         const int* act = at<int>(arena, d.off_act) + o.tile0 + J0;
+        const int lim = 2 * o.etr - 120;
         int n = 0;
         for (int c0 = 0; c0 < d.n_chunks; c0 += 64) {
             const int c = c0 + lane;
-            int er = NO_EXP, ec = NO_EXP, mask = 0;
-            if (c < d.n_chunks)
-                for (int t = 0; t < nt; t++) {
-                    const int e = act[(int64_t)c * nT + t];
-                    er = max(er, e);
-                    if (t < ncol) ec = max(ec, e);
-                    if (e >= o.emin) mask |= 1 << t;
+            int e[NR];
+            unsigned pa = 0, pb = 0;
+#pragma unroll
+            for (int t = 0; t < NR; t++) e[t] = c < d.n_chunks && t < nt ? act[(int64_t)c * nT + t] : NO_EXP;
+#pragma unroll
+            for (int w = 0; w < NW; w++)
+#pragma unroll
+                for (int i = 0; i < PS; i++) {
+                    const int j = col_of(w, i), r = row_of(w, i);
+                    if (r >= BAND_TILES) continue;
+                    const unsigned on = e[j] + e[j + r] >= lim;
+                    (j + r < NS ? pa : pb) |= on << (PS * w + i);
                 }
-            const bool ok = er + ec >= 2 * o.etr - 136;
-            const unsigned long long bal = __ballot(ok);
-            if (ok) list[n + __popcll(bal & ((1ull << lane) - 1))] = c | (mask << 16);
-            n += __popcll(bal);
+            const unsigned long long ba = __ballot(pa != 0), bb = __ballot(pb != 0), below = (1ull << lane) - 1;
+            const int i = n + __popcll(ba & below) + __popcll(bb & below);
+            if (pa) list[i] = make_int2(c, (int)pa);
+            if (pb) list[i + (pa != 0)] = make_int2(c | 1 << 10, (int)pb);
+            n += __popcll(ba) + __popcll(bb);
         }
         if (lane == 0) nlist = n;
     }
     __syncthreads();
-    const int64_t ldf = 2 * (int64_t)nP;
-    const double* F = at<double>(arena, d.off_rows) + 16 * (int64_t)(o.tile0 + J0);
-    double4_t tot[BAND_TILES];
+    const int ns = nlist;
+    const int k0 = 8 * (o.tile0 + J0);
+    const double* nd = at<double>(arena, d.off_node);
+    const double2* ck = at<double2>(arena, d.off_ck);
+    const int* cE = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP);
+    const int* dg = at<int>(arena, d.off_deg) + (tid & 255);   // 4 bytes of a chunk's constants per lane
+    // this lane's node: in the (lane/8)-th of the step's eight tiles, from
+    // tile 0 or tile 2 on (nodes past the block's are loaded as its last one
+    // and not used)
+    const int slot = lane >> 3, ka = min(k0 + lane, nP - 1), kb = min(k0 + lane + 16, nP - 1);
+    const double xa = nd[ka], xb = nd[kb], m = d.m;
+    const int grp = wv >> 2, sub = wv & 3;   // its chunk of the step and four degrees
+    // states and constants of a step, loaded two steps ahead
+    struct State {
+        double2 s;
+        int E, dg, en, pm[NG];
+    };
+    auto load = [&](int s, State& v) {
+        v.en = __builtin_amdgcn_readfirstlane(list[min(NG * s + grp, ns - 1)].x);
 #pragma unroll
-    for (int r = 0; r < BAND_TILES; r++) tot[r] = (double4_t){0, 0, 0, 0};
-    typedef double double2_t __attribute__((ext_vector_type(2)));
-    double2_t pf[PER];
-    const int g0 = split > 1 ? run : 0, g1 = split > 1 ? run + 1 : GRAM_SPLIT;
-    for (int g = g0; g < g1; g++) {
-        const int s0 = 2 * (nlist * g / GRAM_SPLIT), s1 = 2 * (nlist * (g + 1) / GRAM_SPLIT);
-        double4_t acc[BAND_TILES];
+        for (int g = 0; g < NG; g++) {
+            const unsigned pm = list[min(NG * s + g, ns - 1)].y;
+            v.pm[g] = NG * s + g < ns ? __builtin_amdgcn_readfirstlane((pm >> (PS * wv)) & ((1u << PS) - 1)) : 0;
+        }
+        const int c = v.en & 1023;
+        const int64_t ci = (int64_t)c * nP + (v.en & 1024 ? kb : ka);
+        v.s = ck[ci];
+        v.E = cE[ci];
+        v.dg = dg[256 * c];
+    };
+    double4_t acc[PS];
 #pragma unroll
-        for (int r = 0; r < BAND_TILES; r++) acc[r] = (double4_t){0, 0, 0, 0};
-        auto fetch = [&](int s) {
-            const int en = list[s >> 1];
-            const double* Fs = F + (int64_t)(32 * (en & 0xffff) + 16 * (s & 1)) * ldf;
+    for (int i = 0; i < PS; i++) acc[i] = (double4_t){0, 0, 0, 0};
+    auto step = [&](int s, State& v) {
+        const int en = v.en;
+        unsigned pm[NG];
 #pragma unroll
-            for (int t = 0; t < PER; t++) {
-                const int i = tid + 256 * t, kk = i / LD2, q = i % LD2;
-                pf[t] = (en >> (16 + (q >> 3))) & 1 ? *reinterpret_cast<const double2_t*>(Fs + kk * ldf + 2 * q)
-                                                    : (double2_t){0, 0};
+        for (int g = 0; g < NG; g++) pm[g] = v.pm[g];
+        // (every wavefront is past the constants of the step before)
+        reinterpret_cast<int*>(degs)[tid] = v.dg;
+        double p = v.s.x, pp = v.s.y;
+        int e = v.E;
+        load(s + 2, v);
+        __syncthreads();   // and past its products
+        {
+            // (lanes of tiles that no pair needs run along: numbers, never read)
+            const double x = en & 1024 ? xb : xa;
+#pragma unroll
+            for (int j = 0; j < 12; j += 4) {
+                if (j >= 4 * sub) break;
+                double2 cc[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) cc[q] = *reinterpret_cast<const double2*>(&degs[grp][j + q].c1);
+#pragma unroll
+                for (int q = 0; q < 4; q++) degree_step(cc[q].x, cc[q].y, x, p, pp);
+                rescale(p, pp, e);
             }
-        };
-        if (s0 < s1) fetch(s0);
-        for (int s = s0; s < s1; s++) {
-            double(*W)[PITCH] = S[s & 1];
+            Deg g[4];
 #pragma unroll
-            for (int t = 0; t < PER; t++) {
-                const int i = tid + 256 * t;
-                *reinterpret_cast<double2_t*>(&W[i / LD2][2 * (i % LD2)]) = pf[t];
-            }
-            __syncthreads();   // the other buffer's readers have passed the barrier before this one
-            if (s + 1 < s1) fetch(s + 1);
-            if (wv < ncol) {
+            for (int j = 0; j < 4; j++) g[j] = degs[grp][4 * sub + j];
+            double2* w = reinterpret_cast<double2*>(&W[grp][8 * sub][2 * lane]);
 #pragma unroll
-                for (int kk = 0; kk < KS; kk += 4) {
-                    const double* w = &W[kk + lk][16 * wv + li];
-                    const double cv = w[0];
-#pragma unroll
-                    for (int r = 0; r < BAND_TILES; r++)
-                        acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv, w[16 * r], acc[r], 0, 0, 0);
-                }
+            for (int j = 0; j < 4; j++) {
+                double ta, pb, pa, tb;
+                degree_rows(g[j], m, x, p, pp, e, ta, pb, pa, tb);
+                w[j * PITCH] = make_double2(ta, pa);
+                w[j * PITCH + PITCH / 2] = make_double2(pb, tb);
             }
         }
-        // the stage buffers are free for the next run's first stage only when
-        // all wavefronts are done with this run's last one
         __syncthreads();
 #pragma unroll
-        for (int r = 0; r < BAND_TILES; r++) tot[r] += acc[r];
-    }
-    if (wv >= ncol) return;
-    // lane l, register q: column l/16 + 4q of the column tile, row l%16; tiles
-    // are kept column by column
-    double* B = at<double>(arena, split > 1 ? d.off_part + (int64_t)run * nT * (BAND_TILES * 256 * 8) : d.off_band)
-              + (int64_t)(J0 + wv) * (BAND_TILES * 256);
+        for (int i = 0; i < NG * PS; i++)
+            if (pm[i / PS] >> (i % PS) & 1) {
+                const double* wc = &W[i / PS][lk][li - (NC == 4 && en & 1024 ? 32 : 0)] + 16 * col_of(wv, i % PS);
+                const double* wr = wc + 16 * row_of(wv, i % PS);
+                double cv[KS / 4], rv[KS / 4];
 #pragma unroll
-    for (int r = 0; r < BAND_TILES; r++)
-        if (J0 + wv + r < T) {
+                for (int q = 0; q < KS / 4; q++) {
+                    cv[q] = wc[4 * q * PITCH];
+                    rv[q] = NC == 4 && i == 0 ? cv[q] : wr[4 * q * PITCH];
+                }
 #pragma unroll
-            for (int q = 0; q < 4; q++) B[r * 256 + 64 * q + lane] = split > 1 ? tot[r][q] : -tot[r][q];
+                for (int q = 0; q < KS / 4; q++)
+                    acc[i % PS] = __builtin_amdgcn_mfma_f64_16x16x4f64(cv[q], rv[q], acc[i % PS], 0, 0, 0);
+            }
+    };
+    if (ns > 0) {
+        State v0, v1;
+        load(0, v0);
+        load(1, v1);
+        for (int s = 0; NG * s < ns; s += 2) {
+            step(s, v0);
+            if (NG * (s + 1) < ns) step(s + 1, v1);
         }
-}
-
-__global__ void __launch_bounds__(256) k_gram_sum(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                  const BlockOut* __restrict__ out, int delta_only)
-{
-    const int b = blockIdx.y;
-    const BlockDesc& d = desc[b];
-    const BlockOut& o = out[b];
-    const int J = blockIdx.x / BAND_TILES, r = blockIdx.x % BAND_TILES;
-    if (o.skip || J + r >= o.tiles || (delta_only && !o.delta)) return;
-    const int64_t per = (int64_t)(d.n_waves * 8) * (BAND_TILES * 256);
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    const double* P = at<double>(arena, d.off_part) + i;
-    double s = 0;
+    }
+    // lane l, register q: column l/16 + 4q of the column tile, row l%16; tiles
+    // are kept column by column; -√r √r' of the two rows at the end
+    const double* sr = nd + k0 + nP + (li & 1) * nP + (li >> 1);   // row l%16 of tile 0
+    const double* sc = nd + k0 + nP + (lk & 1) * nP + (lk >> 1);   // column l/16 (+ 4q: node + 2q) of tile 0
 #pragma unroll
-    for (int g = 0; g < GRAM_SPLIT; g++) s += P[g * per];
-    at<double>(arena, d.off_band)[i] = -s;
+    for (int i = 0; i < PS; i++) {
+        const int j = col_of(wv, i), r = row_of(wv, i);
+        if (r >= BAND_TILES || J0 + j + r >= T) continue;
+        double* B = at<double>(arena, d.off_band) + ((int64_t)(J0 + j) * BAND_TILES + r) * 256 + lane;
+        const double s = -sr[8 * (j + r)];
+#pragma unroll
+        for (int q = 0; q < 4; q++) B[64 * q] = acc[i][q] * (s * sc[8 * j + 2 * q]);
+    }
 }
 
 // log det(1 - G) of one block by LDLᵀ without pivoting (1 - G is symmetric
@@ -751,17 +847,16 @@ void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const Bloc
                        arena, status);
 }
 
-// max_wq: largest n_waves ceil(n_chunks/4) of the blocks
-void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_wq,
-                             hipStream_t s)
+// max_wq: largest n_waves ceil(n_chunks/4) of the blocks (128 nodes per
+// workgroup of k_wave_norms: fewer are needed)
+void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, int nblocks, int max_wq, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wave_rows<false>, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena, out, 0);
+    hipLaunchKernelGGL(k_wave_norms, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena);
 }
 
-void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_wq, int all,
-                            hipStream_t s)
+void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, int nblocks, int max_wq, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wave_rows<true>, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena, out, all);
+    hipLaunchKernelGGL(k_wave_rows, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena);
 }
 
 void capsd_launch_wave_window(BlockDesc* desc, char* arena, BlockOut* out, const int* status, int nblocks, int allow,
@@ -770,14 +865,16 @@ void capsd_launch_wave_window(BlockDesc* desc, char* arena, BlockOut* out, const
     hipLaunchKernelGGL(k_wave_window, dim3(nblocks), dim3(256), 0, s, desc, arena, out, status, allow, dense);
 }
 
-// The band of -G; split != 0: one workgroup per run of chunks and a sum
-void capsd_launch_gram(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves, int split,
-                       int delta_only, hipStream_t s)
+// The band of -G, ncol (1 or 4) column tiles per workgroup; max_chunks: the
+// blocks' largest n_chunks
+void capsd_launch_gram(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves,
+                       int max_chunks, int ncol, int delta_only, hipStream_t s)
 {
-    const int T = max_waves * 8, ns = split ? GRAM_SPLIT : 1;
-    hipLaunchKernelGGL(k_gram, dim3((T + 3) / 4 * ns, nblocks), dim3(256), 0, s, desc, arena, out, ns, delta_only);
-    if (split)
-        hipLaunchKernelGGL(k_gram_sum, dim3(T * BAND_TILES, nblocks), dim3(256), 0, s, desc, arena, out, delta_only);
+    const int T = max_waves * 8;
+    const size_t lds = 2 * (size_t)max_chunks * sizeof(int2);   // two steps per chunk at most
+    if (ncol == 1) hipLaunchKernelGGL(k_gram<1>, dim3(T, nblocks), dim3(512), lds, s, desc, arena, out, delta_only);
+    else
+        hipLaunchKernelGGL(k_gram<4>, dim3((T + 3) / 4, nblocks), dim3(256), lds, s, desc, arena, out, delta_only);
 }
 
 void capsd_launch_band_ldl(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int mercator, hipStream_t s)
