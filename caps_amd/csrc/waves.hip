@@ -591,148 +591,335 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
     }
 }
 
+// Broadcasts within 16 lanes as DPP operands of the FMAs: v_fmac_f64 takes
+// row_newbcast, but the compiler makes a move and an FMA of them, and puts off
+// the rows x, which costs 128 spilled registers.  Two wait states have to lie
+// between a VALU write and a DPP read of it: the instructions between, or
+// s_nop.
+#define FMAC_ROW(x, a, l) "v_fmac_f64_dpp %" #x ", %" #a ", %[" #l "] row_newbcast:%[t] row_mask:0xf bank_mask:0xf\n"
+#define MOV_ROW(d, a) "v_mov_b64_dpp %" #d ", %" #a " row_newbcast:%[u] row_mask:0xf bank_mask:0xf\n"
+
+// x += a(lane T) lx, a += a(lane T) la for column T + 1 (and x of the two
+// behind it); returns the next pivot, a(lane T + 1) of column T + 1
+template <int T>
+__device__ __forceinline__ double column_next(double (&x)[16], double (&a)[16], double lx, double la)
+{
+    double d;
+    if constexpr (T < 13)
+        asm volatile("s_nop 1\n" FMAC_ROW(0, 4, lx) FMAC_ROW(4, 4, la) FMAC_ROW(1, 5, lx) FMAC_ROW(2, 6, lx) MOV_ROW(3, 4)
+                     : "+v"(x[T + 1]), "+v"(x[T + 2]), "+v"(x[T + 3]), "=&v"(d), "+v"(a[T + 1])
+                     : "v"(a[T + 2]), "v"(a[T + 3]), [lx] "v"(lx), [la] "v"(la), [t] "n"(T), [u] "n"(T + 1));
+    else
+        asm volatile("s_nop 1\n" FMAC_ROW(0, 2, lx) FMAC_ROW(2, 2, la) "s_nop 1\n" MOV_ROW(1, 2)
+                     : "+v"(x[T + 1]), "=&v"(d), "+v"(a[T + 1])
+                     : [lx] "v"(lx), [la] "v"(la), [t] "n"(T), [u] "n"(T + 1));
+    return d;
+}
+
+// ... for a of columns J .. 15 and x of those that column_next left
+template <int T, int J>
+__device__ __forceinline__ void columns_rest(double (&x)[16], double (&a)[16], double lx, double la)
+{
+    if constexpr (J < 16) {
+        if constexpr (T >= 13 || J > T + 3)
+            asm volatile(FMAC_ROW(0, 1, lx) : "+v"(x[J]) : "v"(a[J]), [lx] "v"(lx), [t] "n"(T));
+        asm volatile(FMAC_ROW(0, 0, la) : "+v"(a[J]) : [la] "v"(la), [t] "n"(T));
+        columns_rest<T, J + 1>(x, a, lx, la);
+    }
+}
+#undef FMAC_ROW
+#undef MOV_ROW
+
+// value of lane N of the lane's 16
+template <int N>
+__device__ __forceinline__ double row_d(double x)
+{
+    return __longlong_as_double(
+        __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(x), 0x150 + N, 0xf, 0xf, true));
+}
+
+template <int N, class F, int... I>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for_<N>(f, std::make_integer_sequence<int, N>{});
+}
+
 // log det(1 - G) of one block by LDLᵀ without pivoting (1 - G is symmetric
 // positive definite, so the elimination is stable in any order), in the
 // delta form: the matrix holds -G, pivots are u = 1 + d with d the stored
 // diagonal, and log u = log1p(d) keeps the accuracy of small blocks.  One
-// workgroup of eight wavefronts; the seven tile columns of the active band
-// live in LDS (100 KB), the next one is loaded while a column is eliminated.
-// Per tile column: wavefronts 0 and 1 factor its 16 columns, one lane per
-// row (the 16 diagonal rows in both, so that no other exchange is needed
-// than lane broadcasts), wavefront 2 takes the logs of the column before;
-// then all update the up to 21 tiles behind it on MFMA.  Bound by the chain
-// of 16 pivots per column.
+// workgroup of sixteen wavefronts.
+// What bounds it is the chain of pivots, 16 per tile column, so
+//  - the band is eliminated from both ends at once towards the six tile columns
+//    in its middle (half 1 has the order of the tiles reversed; what it
+//    subtracts from the middle is added to half 0's before these follow);
+//  - a column's pivots run beside the update of the column before: wavefronts
+//    0 .. 3 factor, two per half, the others update the tiles behind on MFMA,
+//    the next column's first;
+//  - the tiles behind stay in registers from the load to their own column:
+//    a wavefront has one diagonal of tiles, and only the column in work and
+//    the next one are in LDS.
+// The pivots' FMAs and the MFMAs share the SIMDs' FP64 units, 1900 and 2800
+// cycles of the 7200 that a step takes.  26, 79 and 15 tile columns: 55, 136 and
+// 39 us; column after column from one end, through LDS, 94, 282 and 55 us.
 // mercator: the LU-mode rule of src/matrix.c:489-505 first (||M||_F² = tr M² =
 // Σ G_ij²; skip = 2: the host returns the two-term series).
-__global__ void __launch_bounds__(512) k_band_ldl(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                  BlockOut* __restrict__ out, int mercator)
+__global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                   BlockOut* __restrict__ out, int mercator)
 {
-    constexpr int NW = 8, NTH = 64 * NW, BT = BAND_TILES, COL = BT * 256;
-    __shared__ double S[BT * COL];
-    __shared__ double us[2][16], ds[2][16];
-    __shared__ double red[NTH];
+    constexpr int NTH = 1024, BT = BAND_TILES, COL = BT * 256, MID = BT - 1;
+    static_assert(BT == 7, "six diagonals of tiles, dealt to twelve wavefronts");
+    __shared__ double S[2][2][COL];
     const int b = blockIdx.x;
     const BlockDesc& d = desc[b];
     BlockOut& o = out[b];
     const int T = o.tiles;
     if (o.skip || !o.delta || T <= 0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
-    const double* __restrict__ B = at<double>(arena, d.off_band);
+    const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    double* B = at<double>(arena, d.off_band);
     if (mercator) {
-        double f = 0;
-        for (int64_t i = tid; i < (int64_t)T * COL; i += NTH) {
-            const int r = (int)(i % COL) >> 8, J = (int)(i / COL);
-            if (J + r < T) f += (r ? 2.0 : 1.0) * (B[i] * B[i]);
+        // ||G||_F >= tr G / √N: most blocks are past the rule without a look at G
+        const double tr = o.trace, low = fabs(tr) / sqrt(16.0 * T);
+        bool may = low < 1;
+        if (may) may = low * low / 2 + low + log1p(-low) >= -2e-8 * (fabs(tr) + tr * tr / 2);
+        if (may) {
+            double* red = &S[0][0][0];
+            double f = 0;
+            for (int64_t i = tid; i < (int64_t)T * COL; i += NTH) {
+                const int r = (int)(i % COL) >> 8, J = (int)(i / COL);
+                if (J + r < T) f += (r ? 2.0 : 1.0) * (B[i] * B[i]);
+            }
+            red[tid] = f;
+            __syncthreads();
+            for (int s = NTH / 2; s > 0; s >>= 1) {
+                if (tid < s) red[tid] += red[tid + s];
+                __syncthreads();
+            }
+            const double f2 = red[0], norm = sqrt(f2);
+            bool take = false;
+            if (norm < 1) {
+                const double merc = -o.trace - f2 / 2, err = fabs(norm * norm / 2 + norm + log1p(-norm));
+                take = fabs(err / merc) < 1e-8;
+            }
+            __syncthreads();
+            if (tid == 0) {
+                o.frob2 = o.tr2 = f2;
+                if (take) o.skip = 2;
+            }
+            if (take) return;
         }
-        red[tid] = f;
+    }
+    const int mid = T < MID ? T : MID, n0 = (T - mid + 1) / 2, n1 = (T - mid) / 2;   // columns of the halves
+    // N elements of tile (I, K) of half h from the band: e, e + 64, ..; 0 for
+    // what is not there and half 1's middle (both without a use of what is
+    // loaded: the wait comes a step later)
+    auto load = [&](int h, int I, int K, int e, auto& v) {
+        const bool on = I < (h ? n1 : n0) + mid && K >= 0 && !(h && K >= n1);
+        const int src = on ? ((h ? T - 1 - I : K) * BT + I - K) * 256 : 0;
+#pragma unroll
+        for (double& w : v) {
+            w = B[src + (h ? (e & 15) << 4 | e >> 4 : e)];
+            e += 64;
+        }
+        return on ? 1.0 : 0.0;
+    };
+    // pivots of tile column J of half h and the nb tiles below, -L in place of
+    // these: a lane has a row of the tiles below (wavefront part 0 the first 64)
+    // and a row of the diagonal tile, which every 16 lanes hold, so that a
+    // pivot's row comes as a broadcast within 16 lanes (a done row's lane goes
+    // on with what nobody reads)
+    auto factor = [&](int h, int J, int nb, int part) {
+        double* dp = &S[h][J & 1][li];
+        double* tp = dp + (1 + min(4 * part + lk, MID - 1)) * 256;
+        double a[16], x[16];
+#pragma unroll
+        for (int t = 0; t < 16; t++) a[t] = dp[16 * t];
+#pragma unroll
+        for (int t = 0; t < 16; t++) x[t] = tp[16 * t];
+        double dt = row_d<0>(a[0]);
+        static_for<16>([&](auto tc) {
+            constexpr int t = tc;
+            // -1/u from the hardware's estimate r: -r (1 + e + e²), e = 1 - u r
+            const double u = 1.0 + dt, r = __builtin_amdgcn_rcp(u);
+            const double e = fma(-u, r, 1.0), n = fma(-r, fma(e, e, e), -r);
+            x[t] *= n;
+            if constexpr (t < 15) {
+                const double la = a[t] * n;
+                dt = column_next<t>(x, a, x[t], la);
+                columns_rest<t, t + 2>(x, a, x[t], la);
+            }
+        });
+        if (4 * part + lk < nb) {
+#pragma unroll
+            for (int t = 0; t < 16; t++) tp[16 * t] = x[t];
+        }
+        if (part == 0 && lane < 16) {
+#pragma unroll
+            for (int t = 0; t < 16; t++) dp[16 * t] = a[t];   // its diagonal: the d
+        }
+    };
+    {
+        const int h = wv >> 3;   // column 0: 512 threads
+        for (int i = tid & 511; i < COL; i += 512) {
+            double v[1];
+            const double f = load(h, i >> 8, 0, i & 255, v);
+            S[h][0][i] = f != 0 ? v[0] : 0.0;
+        }
+    }
+    // Two programs with the same barriers, so that the registers of one are not
+    // held in the other.
+    if (wv < 4) {
+        const int h = wv >> 1, part = wv & 1, nh = h ? n1 : n0, end = h ? n1 : n0 + mid;
+        double pf[2], on = load(h, 7, 1, part * 128 + lane, pf);   // half of the next column's last tile
         __syncthreads();
-        for (int s = NTH / 2; s > 0; s >>= 1) {
-            if (tid < s) red[tid] += red[tid + s];
+        for (int J = 0; J < n0 + mid; J++) {
+            if (J == n0 && J > 0) {
+                if (n1 > 0) {
+                    __syncthreads();
+                    __syncthreads();
+                }
+                __syncthreads();
+            }
+            const int nb = min(MID, n0 + mid - 1 - J);
+            if (J == 0 || J == n0) {
+                if (J < end) factor(h, J, nb, part);
+                __syncthreads();
+            }
+            if (J + 1 < nh) {
+                double* t = &S[h][(J + 1) & 1][MID * 256 + part * 128 + lane];
+#pragma unroll
+                for (int s = 0; s < 2; s++) t[64 * s] = on != 0 ? pf[s] : 0.0;
+                on = load(h, J + 8, J + 2, part * 128 + lane, pf);
+            }
+            if (J < end && part == 0 && lane < 16)
+                B[(h ? T - 1 - J : J) * COL + lane] = S[h][J & 1][17 * lane];   // d, for the logs
+            __syncthreads();
+            if (J + 1 != nh && J + 1 < end) factor(h, J + 1, min(MID, nb - (J + 1 > n0)), part);
             __syncthreads();
         }
-        const double f2 = red[0], norm = sqrt(f2);
-        bool take = false;
-        if (norm < 1) {
-            const double merc = -o.trace - f2 / 2, err = fabs(norm * norm / 2 + norm + log1p(-norm));
-            take = fabs(err / merc) < 1e-8;
+    } else {
+        // half and diagonal I - K = fd of the tiles (J + 1 + i + fd, J + 1 + i) in
+        // acc[i]; the wavefronts of a SIMD (modulo 4) have 11 or 10 of a step's 42
+        const int h = (wv >> 1) & 1, fd = (wv & 1 ? 0x431 : 0x520) >> (4 * ((wv >> 2) - 1)) & 7, nh = h ? n1 : n0;
+        double4_t acc[MID];
+        double pf[4], on;
+#pragma unroll
+        for (int i = 0; i < MID; i++) {
+            const double f = load(h, 1 + i + fd, 1 + i, lane, pf);
+#pragma unroll
+            for (int q = 0; q < 4; q++) acc[i][q] = f != 0 ? pf[q] : 0.0;
         }
+        on = load(h, 7, 7 - fd, lane, pf);   // the tile that comes in after this step
         __syncthreads();
-        if (tid == 0) {
-            o.frob2 = o.tr2 = f2;
-            if (take) o.skip = 2;
+        for (int J = 0; J < n0 + mid; J++) {
+            auto put = [&](double* col) {   // acc[0] to LDS and to the end
+                const double4_t t = acc[0];
+#pragma unroll
+                for (int q = 0; q < 4; q++) col[256 * fd + 64 * q + lane] = t[q];
+#pragma unroll
+                for (int i = 0; i + 1 < MID; i++) acc[i] = acc[i + 1];
+                acc[MID - 1] = t;
+            };
+            if (J == n0 && J > 0) {   // the middle: the halves' sum
+                double* M = &S[0][0][0] + fd * (2 * MID + 1 - fd) / 2 * 256;
+                if (n1 > 0) {
+#pragma unroll
+                    for (int i = 0; i < MID; i++)
+                        if (h && i + fd < MID) {
+#pragma unroll
+                            for (int q = 0; q < 4; q++)
+                                M[(MID - 1 - fd - i) * 256 + 16 * li + 4 * q + lk] = acc[i][q];
+                        }
+                    __syncthreads();
+#pragma unroll
+                    for (int i = 0; i < MID; i++)
+                        if (!h && i + fd < MID) {
+#pragma unroll
+                            for (int q = 0; q < 4; q++) acc[i][q] += M[i * 256 + 64 * q + lane];
+                        }
+                    __syncthreads();
+                }
+                if (!h) put(S[0][J & 1]);
+                __syncthreads();
+            }
+            if (J == 0 || J == n0) __syncthreads();
+            const int nb = J < n1 || h == 0 ? min(MID, n0 + mid - 1 - J) : 0;
+            const double* const L = S[h][J & 1];
+            const bool last = J + 1 == nh;
+            double u[4];
+            auto update = [&](int i, int k) {   // acc[i], K = J + 1 + k: -= L_I u L_Kᵀ (-L is stored, and d on the diagonal)
+                const double *LK = L + 256 * (1 + k) + lane, *LI = LK + 256 * fd;
+                double x[4], y[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    x[q] = LK[64 * q];
+                    y[q] = LI[64 * q];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q] * u[q], y[q], acc[i], 0, 0, 0);
+            };
+            if (fd < nb) {   // the next column
+#pragma unroll
+                for (int q = 0; q < 4; q++) u[q] = -1.0 - L[17 * (4 * q + lk)];
+                update(0, 0);
+                put(S[h][(J + 1) & 1]);
+            }
+            __syncthreads();
+            if (fd < nb) {   // the others
+#pragma unroll
+                for (int i = 0; i + 1 < MID; i++)
+                    if (i + 1 + fd < nb) update(i, i + 1);
+                if (last) {   // back for the sum
+                    const double4_t t = acc[MID - 1];
+#pragma unroll
+                    for (int i = MID - 1; i > 0; i--) acc[i] = acc[i - 1];
+                    acc[0] = t;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < MID; i++)
+                        if (i + fd + 1 == MID) {
+#pragma unroll
+                            for (int q = 0; q < 4; q++) acc[i][q] = on != 0 ? pf[q] : 0.0;
+                        }
+                    on = load(h, J + 8, J + 8 - fd, lane, pf);
+                }
+            }
+            __syncthreads();
         }
-        if (take) return;
     }
-    for (int K = 0; K < BT && K < T; K++)
-        for (int i = tid; i < COL; i += NTH) S[K * COL + i] = B[(int64_t)K * COL + i];
-    __syncthreads();
-    double ls = 0, lc = 0;   // wavefront 2, lanes 0 .. 15: Σ log u in double-double
-    auto add_log = [&](int J) {
-        const double dv = ds[J & 1][li];
-        const double v = dv > -0.5 ? log1p(dv) : log(fabs(1.0 + dv));
+    // Σ log u in double-double
+    double ls = 0, lc = 0;
+    auto add = [&](double v, double c) {
         double t, e;
         two_sum(ls, v, t, e);
         ls = t;
-        lc += e;
+        lc = (lc + c) + e;
     };
-    constexpr int PFN = (COL + NTH - 1) / NTH;
-    double pf[PFN];
-    for (int J = 0; J < T; J++) {
-        const int nb = min(BT - 1, T - 1 - J), sj = J % BT;
-        const bool more = J + BT < T;
-        if (more) {
-#pragma unroll
-            for (int s = 0; s < PFN; s++)
-                if (tid + s * NTH < COL) pf[s] = B[(int64_t)(J + BT) * COL + tid + s * NTH];
-        }
-        if (wv < 2) {
-            const int pr = wv * 48 + lane - 16;
-            const bool dg = lane < 16, on = dg || pr < nb * 16;
-            double* tp = S + sj * COL + (dg ? lane : (1 + (pr >> 4)) * 256 + (pr & 15));
-            double a[16];
-#pragma unroll
-            for (int t = 0; t < 16; t++) a[t] = on ? tp[16 * t] : 0.0;
-#pragma unroll
-            for (int t = 0; t < 16; t++) {
-                const double ru = rcp_nr(1.0 + lane_d(a[t], t));
-                const double l = lane > t ? a[t] * ru : 0.0;
-#pragma unroll
-                for (int j = t + 1; j < 16; j++) a[j] = fma(-l, lane_d(a[j], t), a[j]);
-                a[t] = lane > t ? l : a[t];
-            }
-            if (!dg && on) {
-#pragma unroll
-                for (int t = 0; t < 16; t++) tp[16 * t] = a[t];
-            }
-            if (wv == 0 && dg) {
-                double dv = a[0];
-#pragma unroll
-                for (int t = 1; t < 16; t++) dv = lane == t ? a[t] : dv;
-                us[J & 1][lane] = 1.0 + dv;
-                ds[J & 1][lane] = dv;
-            }
-        } else if (wv == 2 && J > 0 && lane < 16) {
-            add_log(J - 1);
-        }
-        __syncthreads();
-        // tile (I, K) of the columns behind: -= L_I u L_Kᵀ
-        const double* Lc = S + sj * COL;
-        for (int i = wv; i < nb * (nb + 1) / 2; i += NW) {
-            int I = 1, K = i;
-            while (K >= I) K -= I++;
-            K++;
-            double* C = S + ((J + K) % BT) * COL + (I - K) * 256;
-            double4_t acc;
-#pragma unroll
-            for (int q = 0; q < 4; q++) acc[q] = C[64 * q + lane];
-#pragma unroll
-            for (int kk = 0; kk < 16; kk += 4) {
-                const int e = 16 * (kk + lk) + li;
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Lc[K * 256 + e] * us[J & 1][kk + lk], -Lc[I * 256 + e], acc,
-                                                           0, 0, 0);
-            }
-#pragma unroll
-            for (int q = 0; q < 4; q++) C[64 * q + lane] = acc[q];
-        }
-        __syncthreads();
-        if (more) {
-#pragma unroll
-            for (int s = 0; s < PFN; s++)
-                if (tid + s * NTH < COL) S[sj * COL + tid + s * NTH] = pf[s];
-        }
+    for (int i = tid; i < 16 * T; i += NTH) {
+        const double dv = B[(int64_t)(i >> 4) * COL + (i & 15)];
+        add(dv > -0.5 ? log1p(dv) : log(fabs(1.0 + dv)), 0.0);
     }
-    if (wv != 2) return;
-    if (lane < 16) add_log(T - 1);
-    else ls = lc = 0;
 #pragma unroll
-    for (int off = 8; off >= 1; off >>= 1) {
+    for (int off = 32; off >= 1; off >>= 1) {
         const double so = __shfl_xor(ls, off), co = __shfl_xor(lc, off);
-        double t, e;
-        two_sum(ls, so, t, e);
-        ls = t;
-        lc = (lc + co) + e;
+        add(so, co);
     }
-    if (lane == 0) o.logdet = ls + lc;
+    double* red = &S[0][0][0];
+    if (lane == 0) {
+        red[2 * wv] = ls;
+        red[2 * wv + 1] = lc;
+    }
+    __syncthreads();
+    if (tid != 0) return;
+    for (int w = 1; w < NTH / 64; w++) add(red[2 * w], red[2 * w + 1]);
+    o.logdet = ls + lc;
 }
 
 // -G dense, column-major (zero outside the band), for the LU's kernels:
@@ -879,7 +1066,7 @@ void capsd_launch_gram(const BlockDesc* desc, char* arena, const BlockOut* out, 
 
 void capsd_launch_band_ldl(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int mercator, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_band_ldl, dim3(nblocks), dim3(512), 0, s, desc, arena, out, mercator);
+    hipLaunchKernelGGL(k_band_ldl, dim3(nblocks), dim3(1024), 0, s, desc, arena, out, mercator);
 }
 
 void capsd_launch_band_dense(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves,

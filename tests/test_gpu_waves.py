@@ -103,3 +103,21 @@ def test_cholesky_mode_takes_the_matrix(ca):
     ms = [0, 1, 2, 5, 9]
     v, w = c.logdetD_batch([1.5] * 5, ms), h.logdetD_batch([1.5] * 5, ms)
     assert np.max(np.abs(v / w - 1)) < 20 * 300 * EPS + 1e-12
+
+
+@pytest.mark.parametrize("rbyl,ldim", [(0.05, 5), (0.2, 5), (0.5, 8), (1, 12), (2, 20), (5, 40), (12, 80)])
+def test_few_tiles(ca, rbyl, ldim):
+    """Windows of 1 to some 15 tile columns: the two halves of the band have
+    none, one, or one column more than the other before they meet."""
+    from caps_amd import autotune as at
+    c = make(ca, rbyl, ldim, 1)
+    ms = [m for m in range(13) if m <= ldim - 1]
+    xs = [0.4] * len(ms)
+    v, tr, fl = c.logdetD_batch(xs, ms, info=True)
+    try:
+        at.set_config(1, 1, 0, 128)
+        w, tw, fw = c.logdetD_batch(xs, ms, info=True)
+    finally:
+        at.set_config(0)
+    assert np.array_equal(tr, tw) and np.array_equal(fl, fw)
+    assert np.max(np.abs(v / w - 1)) < 1e-12
