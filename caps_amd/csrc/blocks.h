@@ -34,11 +34,13 @@ struct BlockDesc {
     int lda;                // leading dimension of the matrix, if there is one
     // byte offsets into the arena; nP = 64 n_waves
     int64_t off_mie;    // the block's MieDesc table
-    int64_t off_node;   // 3 nP doubles: x, √r_TM, √|r_TE|
+    int64_t off_node;   // 4 nP doubles: x, √r_TM, √|r_TE|, S_m; nP ints: its exponent
+    int64_t off_run;    // per run of 64 degrees but the last: 2 nP double2 (k_wave_start's
+                        // matrices by columns), then nP ints of each: their exponents
     int64_t off_ck;     // n_chunks nP double2: S_l, S_{l-1} at each chunk's start, then
                         // n_chunks nP ints: their exponents
-    int64_t off_norm;   // n_chunks nP doubles: squared norms of the rows' chunks
-    int64_t off_act;    // n_chunks nP/8 ints: exponent of a tile's largest of them
+    int64_t off_norm;   // n_segs nP doubles: squared norms of the rows' runs of 64 degrees
+    int64_t off_act;    // n_chunks nP/8 ints: exponent of a tile's largest chunk norm
     int64_t off_dn;     // nP doubles: squared norms of the rows
     int64_t off_deg;    // 16 n_chunks Deg: the degrees' constants
     int64_t off_rows;   // F: 32 n_chunks rows (degree; a_l, b_l) of 2 nP doubles
@@ -54,7 +56,10 @@ struct BlockDesc {
     int64_t off_cpart;  // n_rtiles x N doubles: per row tile, the column sums
                         // of |M_ij| over i != j (written with the matrix)
     int n_rtiles;       // row tiles of off_cpart (0: none)
-    int pad_;
+    int n_below, n_segs;    // runs of 64 degrees below the window and in it
+    // units of the blocks before this one: k_wave_start's workgroups, and
+    // k_wave_norms' workgroups (split) or wavefronts
+    int unit_start, unit_split, unit_pair;
 };
 
 // The band of G: tiles on and below the diagonal per column of 16 x 16 tiles

@@ -36,7 +36,7 @@ struct capsx_mlp;
 extern "C" {
 void capsx_mlp_predict(capsx_mlp* h, const float* X, int n, float* Y);
 void capsd_launch_wave_start(const void*, int, int, const BlockDesc*, char*, int, int, int*, hipStream_t);
-void capsd_launch_wave_norms(const BlockDesc*, char*, int, int, hipStream_t);
+void capsd_launch_wave_norms(const BlockDesc*, char*, int, int, int, int, int, hipStream_t);
 void capsd_launch_wave_window(BlockDesc*, char*, BlockOut*, const int*, int, int, int, hipStream_t);
 void capsd_launch_wave_rows(const BlockDesc*, char*, int, int, hipStream_t);
 void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, int, hipStream_t);
@@ -556,6 +556,8 @@ enum Form { FORM_BAND, FORM_GRAM, FORM_M };
 
 struct BatchPlan {
     int n = 0, ntab = 0, maxN = 0, minN = 0, max_ldim = 0, max_waves = 0, max_wq = 0, max_mie = 0;
+    // units of the launches over all blocks (BlockDesc::unit_*)
+    int u_start = 0, u_split = 0, u_pair = 0, max_runs = 0;
     size_t bytes = 0;
     Job job = JOB_LOGDET;
     Form form = FORM_BAND;
@@ -660,9 +662,13 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             tab.L = std::max(tab.L, d.lmin + ldim - 1);
             wave_grid_for(d);
             const int64_t nP = 64 * (int64_t)d.n_waves, nc = d.n_chunks;
-            d.off_node = take(3 * nP * 8);
+            const int mm = std::max(d.m, 1);
+            d.n_below = (d.lmin - mm + 63) / 64;
+            d.n_segs = (d.n_chunks + 3) / 4;
+            d.off_node = take(nP * 36);
+            d.off_run = take((d.n_below + d.n_segs - 1) * nP * 36);
             d.off_ck = take(nc * nP * 20);
-            d.off_norm = take(nc * nP * 8);
+            d.off_norm = take(d.n_segs * nP * 8);
             d.off_act = take(nc * (nP / 8) * 4);
             d.off_dn = take(nP * 8);
             d.off_deg = take(16 * nc * sizeof(capsd::Deg));
@@ -683,6 +689,15 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             tab_of.pop_back();
             break;
         }
+        if (job != JOB_TABLES) {
+            d.unit_start = p.u_start;
+            d.unit_split = p.u_split;
+            d.unit_pair = p.u_pair;
+            p.u_start += d.n_waves * std::max(1, d.n_below + d.n_segs - 1);
+            p.u_split += d.n_waves * d.n_segs;
+            p.u_pair += (d.n_waves + 1) / 2 * d.n_segs;
+            p.max_runs = std::max(p.max_runs, d.n_below + d.n_segs);
+        }
         p.n = b + 1;
         p.minN = b == 0 ? d.N : std::min(p.minN, d.N);
         p.maxN = std::max(p.maxN, d.N);
@@ -692,6 +707,13 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
         p.sum_waves += d.n_waves;
         p.max_nK = std::max(p.max_nK, d.nK);
         p.max_nl = std::max(p.max_nl, d.nl);
+    }
+    // rounded up to an eighth of a power of two, so that alike batches share a
+    // captured graph (what is past the last unit returns at once)
+    for (int* u : {&p.u_start, &p.u_split, &p.u_pair}) {
+        int q = 1;
+        while (16 * q <= *u) q *= 2;
+        *u = (*u + q - 1) / q * q;
     }
     // four columns per workgroup make 1.8 times as many rows as the band has,
     // one column seven times in four times as many workgroups, which is faster
@@ -826,13 +848,12 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
         return 0;
     }
     const bool det = p.job != JOB_MATRIX, piv = p.job == JOB_PIVOTED;
-    capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.max_waves, c->d_status, s);
+    capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.u_start, c->d_status, s);
     mark(1);
-    if (det) {
-        capsd_launch_wave_norms(c->d_desc, c->arena, n, p.max_wq, s);
+    capsd_launch_wave_norms(c->d_desc, c->arena, n, p.u_split, p.u_pair, p.max_runs, p.max_waves, s);
+    if (det)
         capsd_launch_wave_window(c->d_desc, c->arena, c->d_out, c->d_status, n, piv ? 0 : g_delta_mode,
                                  p.form == FORM_GRAM, s);
-    }
     mark(2);
     if (p.form == FORM_M) capsd_launch_wave_rows(c->d_desc, c->arena, n, p.max_wq, s);
     mark(3);
@@ -864,7 +885,7 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
 std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
 {
     struct {
-        int n, ntab, maxN, max_ldim, max_waves, max_wq, max_mie, max_nK, max_nl, kseg, job, form, dmode, gram_cols;
+        int n, ntab, maxN, max_ldim, max_waves, max_wq, u_start, u_split, u_pair, max_runs, max_mie, max_nK, max_nl, kseg, job, form, dmode, gram_cols;
         int is_pr, lu_kinds, delta_mode;
         int levels, streams, xcd, tile;
         int lu_bnd[MAX_LU_STREAMS + 1], lu_gN[MAX_LU_STREAMS];   // the LU's stream groups (lu_groups)
@@ -878,6 +899,10 @@ std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
     k.max_ldim = p.max_ldim;
     k.max_waves = p.max_waves;
     k.max_wq = p.max_wq;
+    k.u_start = p.u_start;
+    k.u_split = p.u_split;
+    k.u_pair = p.u_pair;
+    k.max_runs = p.max_runs;
     k.max_mie = p.max_mie;
     k.max_nK = p.max_nK;
     k.max_nl = p.max_nl;

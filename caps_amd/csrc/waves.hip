@@ -110,91 +110,128 @@ __device__ void mie_entry(const MieDesc& t, char* __restrict__ arena, int l)
     at<int>(arena, t.off + 32 * (int64_t)t.L)[l - 1] = (int)fa;
 }
 
-// blockIdx.y < ntab: Mie coefficients of table blockIdx.y, one lane per l.
-// Else block blockIdx.y - ntab: 64 nodes per wavefront, one lane each; a
-// chain of one FMA per degree, 17 cycles a step (R/L = 200: 9 µs of a single
-// block), so the rest of F's work is left to the kernels that start from the
-// states kept here and take all chunks of degrees at once.
-__global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ tabs, int ntab,
-                                                   const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                   int* __restrict__ status)
+// The block whose units (workgroups or wavefronts of a launch over all
+// blocks) u is one of: first holds the sums of the counts before each block.
+__device__ __forceinline__ int block_of(const BlockDesc* __restrict__ desc, int n, int u, int BlockDesc::*first)
 {
-    if ((int)blockIdx.y < ntab) {
-        mie_entry(tabs[blockIdx.y], arena, blockIdx.x * 64 + threadIdx.x + 1);
+    int lo = 0, hi = n - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (desc[mid].*first <= u) lo = mid;
+        else hi = mid - 1;
+    }
+    return lo;
+}
+
+// A run's matrix (columns a, b, times 2^e) applied to the state (p, dp) 2^E at
+// its start; p in [1, 2)
+__device__ __forceinline__ void next_run(double2 a, double2 b, int e, double& p, double& dp, int& E)
+{
+    const double t = fma(a.x, p, b.x * dp), dt = fma(a.y, p, b.y * dp);
+    const int f = __builtin_amdgcn_frexp_exp(t) - 1;
+    p = ldexp(t, -f);
+    dp = ldexp(dt, -f);
+    E += e + f;
+}
+
+// The first ntab mie_units workgroups: Mie coefficients, one lane per l.  Then
+// per block, 64 nodes per wavefront, one lane each: the degrees' recurrence as
+// a chain over all of them takes 45 cycles a step (R/L = 2000: 224 us of a
+// block's 620; 14 us and k_wave_prefix's 16 so).  Instead each run of 64
+// degrees, from d.n_below runs below the window on (the first one shorter),
+// gives the 2 x 2 matrix that takes the state at its start to the next run's,
+// and k_wave_prefix or k_wave_norms multiply them.
+// The state is (S_l, D_l = S_l - S_{l-1}), in which all of the recurrence is
+// positive, and with it the matrices and their products lose nothing:
+// D_{l+1} = κ S_l + c2 D_l, S_{l+1} = S_l + D_{l+1}, κ = c1 x - c2 - 1 =
+// c1 (x-1) + c3.
+__global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ tabs, int ntab, int mie_units,
+                                                   const BlockDesc* __restrict__ desc, int n,
+                                                   char* __restrict__ arena, int* __restrict__ status)
+{
+    const int lane = threadIdx.x;
+    int u = blockIdx.x;
+    if (u < ntab * mie_units) {
+        mie_entry(tabs[u / mie_units], arena, (u % mie_units) * 64 + lane + 1);
         return;
     }
-    const BlockDesc& d = desc[blockIdx.y - ntab];
-    const int wave = blockIdx.x, lane = threadIdx.x;
-    if (wave >= d.n_waves) return;
-    const int k = wave * 64 + lane, nP = d.n_waves * 64;
+    u -= ntab * mie_units;
+    const BlockDesc& d = desc[block_of(desc, n, u, &BlockDesc::unit_start)];
+    u -= d.unit_start;
+    const int run = u / d.n_waves, k = (u % d.n_waves) * 64 + lane, nP = d.n_waves * 64;
+    const int runs = d.n_below + d.n_segs - 1;   // the last one leads nowhere
+    if (run >= max(runs, 1)) return;
     const int mm = d.m > 0 ? d.m : 1;
-    double x = 1, p = 0, pp = 0, stm = 0, ste = 0;
-    int E = NO_EXP;   // lanes without a node: 0 times a power of two that is 0
-    if (k < d.n_nodes) {
-        const double v = d.v0 + k * d.h;
-        const double L = v > 40 ? v : log1p(exp(v));
-        const double sg = 1 / (1 + exp(-v));
-        const double xm1 = d.A * d.A * L * L;
-        x = 1 + xm1;
-        const double x2m1 = xm1 * (x + 1);
-        const double dx = 2 * d.A * d.A * L * sg;
-        // S_mm = √(C(2mm,mm)/4^mm) (x²-1)^{mm/2}, times e^{-ξx} √(h dx) and, for
-        // m > 0, the 1/√(x²-1) of p_l and t_l
-        const double lb = 0.5 * (log_central_binomial(mm) + (d.m > 0 ? mm - 1 : mm) * log(x2m1) + log(d.h * dx))
-                        - d.xi_ * x;
-        const double lb2 = lb * (1 / LOG2), fl = floor(lb2);
-        E = (int)fl;
-        p = exp((lb2 - fl) * LOG2);
-        double rte, rtm;
-        fresnel(d.epsm1_plate, d.xi_, d.xi_ * sqrt(x2m1), rte, rtm);
-        stm = sqrt(fabs(rtm));
-        ste = sqrt(fabs(rte));
-        if (!(stm > 0 && ste > 0 && isfinite(stm) && isfinite(ste) && isfinite(lb))) atomicOr(status, 1);
+    double x = 1;
+    const bool on = k < d.n_nodes;
+    const double v = d.v0 + k * d.h, L = v > 40 ? v : log1p(exp(v)), xm1 = d.A * d.A * L * L;
+    if (on) x = 1 + xm1;
+    if (run == 0) {
+        double p = 0, stm = 0, ste = 0;
+        int E = NO_EXP;   // lanes without a node: 0 times a power of two that is 0
+        if (on) {
+            const double sg = 1 / (1 + exp(-v));
+            const double x2m1 = xm1 * (x + 1);
+            const double dx = 2 * d.A * d.A * L * sg;
+            // S_mm = √(C(2mm,mm)/4^mm) (x²-1)^{mm/2}, times e^{-ξx} √(h dx) and, for
+            // m > 0, the 1/√(x²-1) of p_l and t_l
+            const double lb = 0.5 * (log_central_binomial(mm) + (d.m > 0 ? mm - 1 : mm) * log(x2m1) + log(d.h * dx))
+                            - d.xi_ * x;
+            const double lb2 = lb * (1 / LOG2), fl = floor(lb2);
+            E = (int)fl;
+            p = exp((lb2 - fl) * LOG2);
+            double rte, rtm;
+            fresnel(d.epsm1_plate, d.xi_, d.xi_ * sqrt(x2m1), rte, rtm);
+            stm = sqrt(fabs(rtm));
+            ste = sqrt(fabs(rte));
+            if (!(stm > 0 && ste > 0 && isfinite(stm) && isfinite(ste) && isfinite(lb))) atomicOr(status, 1);
+        }
+        double* nd = at<double>(arena, d.off_node);
+        nd[k] = x;
+        nd[nP + k] = stm;
+        nd[2 * nP + k] = ste;
+        nd[3 * nP + k] = p;
+        at<int>(arena, d.off_node + 32 * (int64_t)nP)[k] = E;
     }
-    double* nd = at<double>(arena, d.off_node);
-    nd[k] = x;
-    nd[nP + k] = stm;
-    nd[2 * nP + k] = ste;
-
-    __shared__ double c1s[64], c2s[64];
-    auto coefficients = [&](int l0) {
-        const double l = l0 + lane;
-        const double den = 1 / sqrt((l + 1 - mm) * (l + 1 + mm));
-        c1s[lane] = (2 * l + 1) * den;
-        c2s[lane] = sqrt((l - mm) * (l + mm)) * den;
-        __syncthreads();
+    if (runs == 0) return;
+    const int l1 = d.lmin + 64 * (run - d.n_below + 1), l0 = max(l1 - 64, mm), n4 = (l1 - l0) & ~3;
+    __shared__ double2 cs[64];
+    __shared__ double c3s[64];
+    {
+        const double l = l0 + lane, m2 = (double)mm * mm;
+        const double r0 = sqrt((l - mm) * (l + mm)), r1 = sqrt((l + 1 - mm) * (l + 1 + mm)), den = 1 / r1;
+        cs[lane] = make_double2((2 * l + 1) * den, r0 * den);
+        c3s[lane] = (m2 / (l + r0) + m2 / (l + 1 + r1)) * den;   // c1 - c2 - 1
+    }
+    __syncthreads();
+    const double y = on ? xm1 : 0;
+    double p = 1, dp = 0, q = 0, dq = 1;   // the two solutions
+    int E = 0, j = 0;
+    auto step = [&](int i) {
+        const double2 c = cs[i];
+        const double kap = fma(c.x, y, c3s[i]);
+        dp = fma(kap, p, c.y * dp);
+        dq = fma(kap, q, c.y * dq);
+        p += dp;
+        q += dq;
     };
-    for (int l0 = mm; l0 < d.lmin; l0 += 64) {   // below the window
-        coefficients(l0);
-        const int n = min(64, d.lmin - l0);
-        int j = 0;
-        for (; j + 4 <= n; j += 4) {
+    for (; j < n4; j += 4) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) degree_step(c1s[j + q], c2s[j + q], x, p, pp);
-            rescale(p, pp, E);
+        for (int t = 0; t < 4; t++) step(j + t);
+        if (p > 0x1p300) {   // q < 64 p
+            p *= 0x1p-300;
+            dp *= 0x1p-300;
+            q *= 0x1p-300;
+            dq *= 0x1p-300;
+            E += 300;
         }
-        for (; j < n; j++) degree_step(c1s[j], c2s[j], x, p, pp);
-        rescale(p, pp, E);
-        __syncthreads();
     }
-    double2* cp = at<double2>(arena, d.off_ck);
-    int* ce = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP);
-    for (int c0 = 0; c0 < d.n_chunks; c0 += 4) {
-        coefficients(d.lmin + 16 * c0);
-        const int nc = min(4, d.n_chunks - c0);
-        for (int c = 0; c < nc; c++) {
-            const int64_t i = (int64_t)(c0 + c) * nP + k;
-            cp[i] = make_double2(p, pp);
-            ce[i] = E;
-#pragma unroll
-            for (int j = 0; j < 16; j += 4) {
-#pragma unroll
-                for (int q = 0; q < 4; q++) degree_step(c1s[16 * c + j + q], c2s[16 * c + j + q], x, p, pp);
-                rescale(p, pp, E);
-            }
-        }
-        __syncthreads();
-    }
+    for (; j < l1 - l0; j++) step(j);
+    const int e = __builtin_amdgcn_frexp_exp(p) - 1;
+    double2* T = at<double2>(arena, d.off_run) + (int64_t)run * 2 * nP;
+    T[k] = make_double2(ldexp(p, -e), ldexp(dp, -e));
+    T[nP + k] = make_double2(ldexp(q, -e), ldexp(dq, -e));
+    at<int>(arena, d.off_run + 32 * (int64_t)runs * nP)[run * nP + k] = E + e;
 }
 
 // What one degree needs, the same for all nodes of a block: c1, c2 of
@@ -238,66 +275,172 @@ __device__ __forceinline__ void degree_rows(const Deg& g, double m, double x, do
     degree_step(g.c1, g.c2, x, p, pp);
 }
 
-// The squared norms of F's rows over degrees lmin + 16 c .. + 15 at 128 nodes (two
-// per lane: half the reads of the degrees' constants), four chunks c per workgroup, and per tile of 8 nodes
-// the exponent of the largest (c_k < 2^e); the degrees' constants for k_gram.
-// VALU-bound: 17 FP64 instructions per degree and node.
-__global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict__ desc, char* __restrict__ arena)
+// The states at the runs' starts, in place of the matrices that lead to them
+// (what k_wave_norms does by itself where the runs are few).
+__global__ void __launch_bounds__(64) k_wave_prefix(const BlockDesc* __restrict__ desc, char* __restrict__ arena)
 {
     const BlockDesc& d = desc[blockIdx.y];
-    const int nq = (d.n_chunks + 3) / 4, nw = (d.n_waves + 1) / 2;
-    if ((int)blockIdx.x >= nw * nq) return;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wave = blockIdx.x % nw, c = (blockIdx.x / nw) * 4 + wv;
-    const int nP = d.n_waves * 64;
+    if ((int)blockIdx.x >= d.n_waves) return;
+    const int nP = d.n_waves * 64, k = blockIdx.x * 64 + threadIdx.x, runs = d.n_below + d.n_segs - 1;
+    const double* nd = at<double>(arena, d.off_node);
+    double2* T = at<double2>(arena, d.off_run) + k;
+    int* TE = at<int>(arena, d.off_run + 32 * (int64_t)runs * nP) + k;
+    double p = nd[3 * nP + k], dp = p;   // S_{m-1} = 0
+    int E = at<int>(arena, d.off_node + 32 * (int64_t)nP)[k];
+    constexpr int AHEAD = 8;
+    double2 a[2][AHEAD], b[2][AHEAD];
+    int e[2][AHEAD];
+    auto fetch = [&](int g, int h) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int r = min(g + i, runs - 1);
+            a[h][i] = T[(int64_t)r * 2 * nP];
+            b[h][i] = T[((int64_t)r * 2 + 1) * nP];
+            e[h][i] = TE[r * nP];
+        }
+    };
+    auto steps = [&](int g, int h) {
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++)
+            if (g + i < runs) {
+                next_run(a[h][i], b[h][i], e[h][i], p, dp, E);
+                T[(int64_t)(g + i) * 2 * nP] = make_double2(p, dp);
+                TE[(g + i) * nP] = E;
+            }
+    };
+    if (runs == 0) return;
+    fetch(0, 0);
+    for (int g = 0; g < runs; g += 2 * AHEAD) {
+        fetch(g + AHEAD, 1);
+        steps(g, 0);
+        fetch(g + 2 * AHEAD, 0);
+        steps(g + AHEAD, 1);
+    }
+}
+
+// Runs of 64 degrees at 64 nodes: the state at the run's start from
+// k_wave_start's matrices, the states at its chunks of 16 (for k_gram), the
+// squared norms of F's rows over the run, and per chunk and tile of 8 nodes
+// the exponent of the largest chunk norm (c_k < 2^e); the degrees' constants
+// for k_gram.  Bound by FP64 instructions, 17 per degree and node.
+// SPLIT: a workgroup per run and 64 nodes, a chunk per wavefront, which gets
+// to its chunk with the bare recurrence; else a run of 128 nodes per wavefront
+// (two per lane: half the reads of the degrees' constants), which a batch
+// takes that has enough of them.  Both make the same sums.
+template <bool SPLIT>
+__global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict__ desc, int n, char* __restrict__ arena,
+                                                    int prefixed)
+{
+    constexpr int NH = SPLIT ? 1 : 2;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int u = SPLIT ? blockIdx.x : 4 * blockIdx.x + wv;
+    const int BlockDesc::*first = SPLIT ? &BlockDesc::unit_split : &BlockDesc::unit_pair;
+    const BlockDesc& d = desc[block_of(desc, n, u, const_cast<int BlockDesc::*>(first))];
+    u -= SPLIT ? d.unit_split : d.unit_pair;
+    const int nw = SPLIT ? d.n_waves : (d.n_waves + 1) / 2, wave = u % nw, s = u / nw, nP = d.n_waves * 64;
     const double m = d.m;
-    __shared__ Deg degs[4][16];
-    const bool in = c < d.n_chunks;
-    if (in && lane < 16) {
-        const Deg g = degree(d, arena, d.lmin + 16 * c + lane);
-        degs[wv][lane] = g;
-        if (wave == 0) at<Deg>(arena, d.off_deg)[16 * c + lane] = g;
+    __shared__ Deg degs_[SPLIT ? 64 : 256];
+    __shared__ double part[SPLIT ? 4 : 1][64];
+    Deg* degs = degs_ + (SPLIT ? 0 : 64 * wv);
+    const int nc = s < d.n_segs ? min(4, d.n_chunks - 4 * s) : 0;
+    if ((!SPLIT || wv == 0) && lane < 16 * nc) {
+        const Deg g = degree(d, arena, d.lmin + 64 * s + lane);
+        degs[lane] = g;
+        if (wave == 0) at<Deg>(arena, d.off_deg)[64 * s + lane] = g;
     }
     __syncthreads();
-    if (!in) return;
     const double* nd = at<double>(arena, d.off_node);
-    double x[2], p[2], pp[2], ntm[2], nte[2];
-    int E[2];
+    double x[NH], p[NH], pp[NH], sum[NH];
+    int E[NH], k[NH];
+    if (SPLIT ? wv < nc : nc > 0) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int k = min(wave * 128 + 64 * h + lane, nP - 1);   // (an odd last wave: not stored)
-        const int64_t ci = (int64_t)c * nP + k;
-        const double2 s = at<double2>(arena, d.off_ck)[ci];
-        x[h] = nd[k];
-        p[h] = s.x;
-        pp[h] = s.y;
-        E[h] = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[ci];
-        ntm[h] = nte[h] = 0;
-    }
+        for (int h = 0; h < NH; h++) {
+            k[h] = min(wave * 64 * NH + 64 * h + lane, nP - 1);   // (an odd last wave: not stored)
+            x[h] = nd[k[h]];
+            p[h] = nd[3 * nP + k[h]];
+            pp[h] = p[h];   // S - S_{l-1}, until the run's start
+            E[h] = at<int>(arena, d.off_node + 32 * (int64_t)nP)[k[h]];
+            sum[h] = 0;
+        }
+        const int runs = d.n_below + d.n_segs - 1;
+        const double2* T = at<double2>(arena, d.off_run);
+        const int* TE = at<int>(arena, d.off_run + 32 * (int64_t)runs * nP);
+        const int to = d.n_below + s;
 #pragma unroll 4
-    for (int j = 0; j < 16; j++) {
-        const Deg& g = degs[wv][j];
+        for (int g = prefixed ? max(to - 1, 0) : 0; g < to; g++)
 #pragma unroll
-        for (int h = 0; h < 2; h++) {
-            double ta, pb, pa, tb;
-            degree_rows(g, m, x[h], p[h], pp[h], E[h], ta, pb, pa, tb);
-            ntm[h] = fma(ta, ta, fma(pb, pb, ntm[h]));
-            nte[h] = fma(pa, pa, fma(tb, tb, nte[h]));
-            if ((j & 3) == 3) rescale(p[h], pp[h], E[h]);
+            for (int h = 0; h < NH; h++) {
+                const double2 a = T[(int64_t)g * 2 * nP + k[h]], b = T[(int64_t)(g * 2 + 1) * nP + k[h]];
+                const int e = TE[g * nP + k[h]];
+                if (prefixed) {
+                    p[h] = a.x;
+                    pp[h] = a.y;
+                    E[h] = e;
+                } else {
+                    next_run(a, b, e, p[h], pp[h], E[h]);
+                }
+            }
+#pragma unroll
+        for (int h = 0; h < NH; h++) pp[h] = p[h] - pp[h];
+    }
+    for (int c = 0; c < nc; c++) {
+        if (SPLIT && c < wv) {
+#pragma unroll 4
+            for (int j = 0; j < 16; j++) {
+                const Deg& g = degs[16 * c + j];
+                degree_step(g.c1, g.c2, x[0], p[0], pp[0]);
+                if ((j & 3) == 3) rescale(p[0], pp[0], E[0]);
+            }
+            continue;
+        }
+        if (SPLIT && c > wv) break;
+        const int ch = 4 * s + c;
+        double ntm[NH], nte[NH];
+#pragma unroll
+        for (int h = 0; h < NH; h++) {
+            ntm[h] = nte[h] = 0;
+            if (wave * 64 * NH + 64 * h < nP) {
+                at<double2>(arena, d.off_ck)[(int64_t)ch * nP + k[h]] = make_double2(p[h], pp[h]);
+                at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[(int64_t)ch * nP + k[h]] = E[h];
+            }
+        }
+#pragma unroll 4
+        for (int j = 0; j < 16; j++) {
+            const Deg& g = degs[16 * c + j];
+#pragma unroll
+            for (int h = 0; h < NH; h++) {
+                double ta, pb, pa, tb;
+                degree_rows(g, m, x[h], p[h], pp[h], E[h], ta, pb, pa, tb);
+                ntm[h] = fma(ta, ta, fma(pb, pb, ntm[h]));
+                nte[h] = fma(pa, pa, fma(tb, tb, nte[h]));
+                if ((j & 3) == 3) rescale(p[h], pp[h], E[h]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < NH; h++) {
+            const double stm = nd[nP + k[h]], ste = nd[2 * nP + k[h]];
+            const double norm = stm * stm * ntm[h] + ste * ste * nte[h];
+            sum[h] += norm;
+            int e = norm > 0 ? ilogb(norm) + 1 : NO_EXP;   // a NaN norm: the trace is NaN
+            e = max(e, dpp_i<DPP_QUAD_X1>(e));
+            e = max(e, dpp_i<DPP_QUAD_X2>(e));
+            e = max(e, dpp_i<DPP_HALF_MIRROR>(e));
+            if ((lane & 7) == 0 && wave * 64 * NH + 64 * h < nP)
+                at<int>(arena, d.off_act)[(int64_t)ch * (nP >> 3) + (k[h] >> 3)] = e;
         }
     }
+    double* norm = at<double>(arena, d.off_norm) + (int64_t)s * nP;
+    if (SPLIT) {
+        part[wv][lane] = wv < nc ? sum[0] : 0;
+        __syncthreads();
+        if (wv > 0 || nc == 0) return;
+        double v = part[0][lane];
+        for (int c = 1; c < nc; c++) v += part[c][lane];
+        norm[wave * 64 + lane] = v;
+    } else if (nc > 0) {
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        const int k = wave * 128 + 64 * h + lane;
-        if (k >= nP) break;   // uniform over the wavefront
-        const double stm = nd[nP + k], ste = nd[2 * nP + k];
-        const double norm = stm * stm * ntm[h] + ste * ste * nte[h];
-        at<double>(arena, d.off_norm)[(int64_t)c * nP + k] = norm;
-        int e = norm > 0 ? ilogb(norm) + 1 : NO_EXP;   // a NaN norm: the trace is NaN
-        e = max(e, dpp_i<DPP_QUAD_X1>(e));
-        e = max(e, dpp_i<DPP_QUAD_X2>(e));
-        e = max(e, dpp_i<DPP_HALF_MIRROR>(e));
-        if ((lane & 7) == 0) at<int>(arena, d.off_act)[(int64_t)c * (nP >> 3) + (k >> 3)] = e;
+        for (int h = 0; h < NH; h++)
+            if (wave * 64 * NH + 64 * h < nP) norm[k[h]] = sum[h];
     }
 }
 
@@ -335,37 +478,69 @@ __global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__
     }
 }
 
-// Trace of M = the sum of all rows' squared norms (per node in chunk order,
-// then over the nodes with compensated sums in a fixed order), the trace
-// shortcut |tr M| < 1e-8 (src/matrix.c:78-82), and the window: tiles of 8
+// Trace of M = the sum of all rows' squared norms (per node over the runs of 64
+// degrees, in quarters, then over the nodes with compensated sums in a fixed
+// order), the trace shortcut |tr M| < 1e-8 (src/matrix.c:78-82), and the window: tiles of 8
 // nodes from the first to the last node whose rows carry more than 2^-60 of
 // the trace (together the others change the determinant by less than a few
 // 1e-17 of it; R/L = 20 .. 2000: 10-60 % of the nodes of large m).  dense:
 // the matrix dimension for the LU's kernels goes to desc[b].N.
-__global__ void __launch_bounds__(256) k_wave_window(BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                     BlockOut* __restrict__ out, const int* __restrict__ status,
-                                                     int allow, int dense)
+// NT: 1024 threads, one quarter of the runs each, or for batches that fill the GPU
+// 256 (block of R/L = 2000: 118 us with 256 threads over its chunks of 16
+// degrees, 28 so; 256 blocks of R/L = 100: 32 us with 1024, 16 with 256; below
+// that many 1024 are as fast or faster).
+template <int NT>
+__global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                    BlockOut* __restrict__ out, const int* __restrict__ status,
+                                                    int allow, int dense)
 {
     const int b = blockIdx.x, tid = threadIdx.x;
     const BlockDesc& d = desc[b];
     const int nP = d.n_waves * 64;
     const double* cn = at<double>(arena, d.off_norm);
     double* dn = at<double>(arena, d.off_dn);
+    constexpr int NQ = 1024 / NT;   // quarters per thread
+    __shared__ double part[4][NT == 1024 ? 256 : 1];
     double s = 0, comp = 0;
-    for (int k = tid; k < nP; k += 256) {
-        double v = 0;
+    for (int k0 = 0; k0 < nP; k0 += 256) {
+        const int k = k0 + (tid & 255);
+        double v[NQ];
+#pragma unroll
+        for (int i = 0; i < NQ; i++) {
+            const int quarter = NQ == 1 ? tid >> 8 : i;
+            const int r0 = quarter * d.n_segs / 4, r1 = (quarter + 1) * d.n_segs / 4;
+            v[i] = 0;
+            if (k < nP) {
 #pragma unroll 8
-        for (int c = 0; c < d.n_chunks; c++) v += cn[(int64_t)c * nP + k];
-        dn[k] = v;
-        double t, e;
-        two_sum(s, v, t, e);
-        s = t;
-        comp += e;
+                for (int r = r0; r < r1; r++) v[i] += cn[(int64_t)r * nP + k];
+            }
+        }
+        double q[4];
+        if constexpr (NQ == 1) {
+            part[tid >> 8][tid & 255] = v[0];
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[i] = part[i][tid & 255];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[i] = v[i];
+        }
+        if (tid < 256 && k < nP) {
+            const double w = (q[0] + q[1]) + (q[2] + q[3]);
+            dn[k] = w;
+            double t, e;
+            two_sum(s, w, t, e);
+            s = t;
+            comp += e;
+        }
+        __syncthreads();
     }
     __shared__ double hs[256], cs[256];
     __shared__ int lo_s, hi_s;
-    hs[tid] = s;
-    cs[tid] = comp;
+    if (tid < 256) {
+        hs[tid] = s;
+        cs[tid] = comp;
+    }
     if (tid == 0) {
         lo_s = nP;
         hi_s = -1;
@@ -381,7 +556,7 @@ __global__ void __launch_bounds__(256) k_wave_window(BlockDesc* __restrict__ des
         __syncthreads();
     }
     const double trace = hs[0] + cs[0], thr = trace * 0x1p-60;
-    for (int k = tid; k < nP; k += 256)
+    for (int k = tid; k < nP; k += NT)
         if (dn[k] > thr) {
             atomicMin(&lo_s, k);
             atomicMax(&hi_s, k);
@@ -1026,19 +1201,29 @@ using namespace capsd;
 
 extern "C" {
 
+// units: of all blocks together (BlockDesc::unit_*), or more
 void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const BlockDesc* desc, char* arena, int nblocks,
-                             int max_waves, int* status, hipStream_t s)
+                             int units, int* status, hipStream_t s)
 {
-    const int gx = max_waves > (max_mie + 63) / 64 ? max_waves : (max_mie + 63) / 64;
-    hipLaunchKernelGGL(k_wave_start, dim3(gx, ntab + nblocks), dim3(64), 0, s, (const MieDesc*)tabs, ntab, desc,
-                       arena, status);
+    const int mu = (max_mie + 63) / 64;
+    hipLaunchKernelGGL(k_wave_start, dim3(ntab * mu + units), dim3(64), 0, s, (const MieDesc*)tabs, ntab, mu, desc,
+                       nblocks, arena, status);
 }
 
-// max_wq: largest n_waves ceil(n_chunks/4) of the blocks (128 nodes per
-// workgroup of k_wave_norms: fewer are needed)
-void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, int nblocks, int max_wq, hipStream_t s)
+// split, pairs: the units of k_wave_norms' two forms.  Whole runs in one
+// wavefront need one of them per SIMD (16 blocks of R/L = 200, norms and
+// window: 30 us whole and 29 us split; 8: 29 and 23; 64: 49 and 61).
+// max_runs: with more than 8 runs k_wave_prefix pays for its launch (2 runs: 10
+// us with it and 6 without; 222 blocks of 19: 93 and 107; 188: 38 and 142).
+void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, int nblocks, int split, int pairs, int max_runs,
+                             int max_waves, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wave_norms, dim3(max_wq, nblocks), dim3(256), 0, s, desc, arena);
+    const int prefixed = max_runs > 8;
+    if (prefixed) hipLaunchKernelGGL(k_wave_prefix, dim3(max_waves, nblocks), dim3(64), 0, s, desc, arena);
+    if (pairs < 1024)
+        hipLaunchKernelGGL(k_wave_norms<true>, dim3(split), dim3(256), 0, s, desc, nblocks, arena, prefixed);
+    else
+        hipLaunchKernelGGL(k_wave_norms<false>, dim3((pairs + 3) / 4), dim3(256), 0, s, desc, nblocks, arena, prefixed);
 }
 
 void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, int nblocks, int max_wq, hipStream_t s)
@@ -1049,7 +1234,10 @@ void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, int nblocks, int
 void capsd_launch_wave_window(BlockDesc* desc, char* arena, BlockOut* out, const int* status, int nblocks, int allow,
                               int dense, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wave_window, dim3(nblocks), dim3(256), 0, s, desc, arena, out, status, allow, dense);
+    if (nblocks < 256)
+        hipLaunchKernelGGL(k_wave_window<1024>, dim3(nblocks), dim3(1024), 0, s, desc, arena, out, status, allow, dense);
+    else
+        hipLaunchKernelGGL(k_wave_window<256>, dim3(nblocks), dim3(256), 0, s, desc, arena, out, status, allow, dense);
 }
 
 // The band of -G, ncol (1 or 4) column tiles per workgroup; max_chunks: the
