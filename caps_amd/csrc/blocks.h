@@ -37,8 +37,7 @@ struct BlockDesc {
     int64_t off_node;   // 4 nP doubles: x, √r_TM, √|r_TE|, S_m; nP ints: its exponent
     int64_t off_run;    // per run of 64 degrees but the last: 2 nP double2 (k_wave_start's
                         // matrices by columns), then nP ints of each: their exponents
-    int64_t off_ck;     // n_chunks nP double2: S_l, S_{l-1} at each chunk's start, then
-                        // n_chunks nP ints: their exponents
+    int64_t off_ck;     // 2 n_chunks nP double2: S_l, S_{l-1} every 8 degrees (degree())
     int64_t off_norm;   // n_segs nP doubles: squared norms of the rows' runs of 64 degrees
     int64_t off_act;    // n_chunks nP/8 ints: exponent of a tile's largest chunk norm
     int64_t off_dn;     // nP doubles: squared norms of the rows
@@ -73,8 +72,8 @@ constexpr int BAND_TILES = 7;
 
 // Constants of one degree of a block's window (see degree() in waves.hip).
 struct Deg {
-    double c1, c2, l, t0, rt, ma, mb;
-    int e, pad_;
+    double c1, c2, l, rt, ma, mb, pad_;
+    int e, sh;
 };
 
 // One Mie table: degrees 1 .. L at one ξ of one object; at off: L doubles each

@@ -667,7 +667,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             d.n_segs = (d.n_chunks + 3) / 4;
             d.off_node = take(nP * 36);
             d.off_run = take((d.n_below + d.n_segs - 1) * nP * 36);
-            d.off_ck = take(nc * nP * 20);
+            d.off_ck = take(nc * nP * 32);
             d.off_norm = take(d.n_segs * nP * 8);
             d.off_act = take(nc * (nP / 8) * 4);
             d.off_dn = take(nP * 8);
@@ -718,7 +718,8 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
     // four columns per workgroup make 1.8 times as many rows as the band has,
     // one column seven times in four times as many workgroups, which is faster
     // as long as strips of four would be fewer than CUs (R/L = 200, four columns
-    // and one: 1 block 83 and 32 us, 32 blocks 89 and 87, 64 blocks 124 and 170)
+    // and one: 1 block 67 and 29 us, 32 blocks 73 and 79, 40 blocks 99 and 96,
+    // 64 blocks 111 and 152)
     if (strips < 256) p.gram_cols = 1;
     if (job != JOB_TABLES) {
         p.ntab = (int)tabs.size();

@@ -67,17 +67,6 @@ __device__ __forceinline__ void degree_step(double c1, double c2, double x, doub
     p = pn;
 }
 
-// Powers of two moved from S into its exponent E (every fourth step: a step
-// multiplies by less than 2x + 1).
-__device__ __forceinline__ void rescale(double& p, double& pp, int& E)
-{
-    if (p > 0x1p300) {
-        p *= 0x1p-300;
-        pp *= 0x1p-300;
-        E += 300;
-    }
-}
-
 // log(C(2m, m)/4^m): a product for small m, else the asymptotic series of
 // log Γ(m+½)/Γ(m+1) (DLMF 5.11.13), whose first neglected term is below 1e-16
 // from m = 16.
@@ -235,43 +224,51 @@ __global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ t
 }
 
 // What one degree needs, the same for all nodes of a block: c1, c2 of
-// degree_step; t_l = (l x + t0) S_l - rt S_{l-1} (m = 0: t_l = P_l^1 = √(l(l+1)) S_l);
-// mantissas and exponent of the Mie factors (zero past the window).
+// degree_step; t_l = l x S_l - rt S_{l-1} (m = 0: l S_l with l = √(l(l+1)), t_l =
+// P_l^1); the Mie factors (zero past the window) over 2^e, e the exponent of the
+// first of each four degrees, and sh = e less that of the four before.  The
+// state (S_l, S_{l-1}) is kept times 2^e: numbers of the size of F over a
+// factor near 1, so that no degree needs an exponent of its own.
 __device__ __forceinline__ Deg degree(const BlockDesc& d, char* arena, int l)
 {
-    const int mm = d.m > 0 ? d.m : 1;
+    const int mm = d.m > 0 ? d.m : 1, last = d.lmin + d.ldim - 1;
     const double den = 1 / sqrt((l + 1.0 - mm) * (l + 1.0 + mm));
     const double rt = sqrt(((double)l - mm) * ((double)l + mm));
+    const int l4 = l - ((l - d.lmin) & 3);
+    const double* a = at<double>(arena, d.off_mie) + (l - 1);
+    const int* ea = at<int>(arena, d.off_mie + 32 * (int64_t)d.mie_L);
     Deg g;
     g.c1 = (2.0 * l + 1) * den;
     g.c2 = rt * den;
-    g.l = d.m > 0 ? l : 0;
-    g.t0 = d.m > 0 ? 0.0 : sqrt((double)l * (l + 1.0));
+    g.l = d.m > 0 ? l : sqrt((double)l * (l + 1.0));
     g.rt = d.m > 0 ? rt : 0.0;
-    const double* a = at<double>(arena, d.off_mie) + (l - 1);
-    const bool ok = l < d.lmin + d.ldim;
-    g.ma = ok ? a[2 * (int64_t)d.mie_L] : 0.0;
-    g.mb = ok ? a[3 * (int64_t)d.mie_L] : 0.0;
-    g.e = ok ? at<int>(arena, d.off_mie + 32 * (int64_t)d.mie_L)[l - 1] : NO_EXP;
-    g.pad_ = 0;
+    g.e = ea[min(l4, last) - 1];
+    g.sh = l4 > d.lmin ? g.e - ea[min(l4 - 4, last) - 1] : 0;
+    g.ma = g.mb = g.pad_ = 0;
+    if (l <= last) {
+        const int e = ea[l - 1] - g.e;
+        g.ma = ldexp(a[2 * (int64_t)d.mie_L], e);
+        g.mb = ldexp(a[3 * (int64_t)d.mie_L], e);
+    }
     return g;
 }
 
-// 2^e for e < 1024, 0 below the normal numbers (what it multiplies is then
-// below 2^-700, its square 0).
-__device__ __forceinline__ double exp2i(int e) { return __hiloint2double(max(e + 1023, 0) << 20, 0); }
+__device__ __forceinline__ void shift(double& p, double& pp, int e)
+{
+    p = ldexp(p, e);
+    pp = ldexp(pp, e);
+}
 
 // One degree at one node, up to the node's √r: the four products of (t_l, p_l)
-// and the Mie factors (a_l, b_l), and the step to the next degree.
-__device__ __forceinline__ void degree_rows(const Deg& g, double m, double x, double& p, double& pp, int E, double& ta,
-                                            double& pb, double& pa, double& tb)
+// and the Mie factors (a_l, b_l), and the step to the next degree.  xt: x, 1 for m = 0.
+__device__ __forceinline__ void degree_rows(const Deg& g, double m, double x, double xt, double& p, double& pp,
+                                            double& ta, double& pb, double& pa, double& tb)
 {
-    const double t = fma(fma(g.l, x, g.t0), p, -(g.rt * pp)), q = m * p;
-    const double u = exp2i(E + g.e), ua = u * g.ma, ub = u * g.mb;
-    ta = t * ua;
-    pb = q * ub;
-    pa = q * ua;
-    tb = t * ub;
+    const double t = fma(g.l * xt, p, -(g.rt * pp)), q = m * p;
+    ta = t * g.ma;
+    pb = q * g.mb;
+    pa = q * g.ma;
+    tb = t * g.mb;
     degree_step(g.c1, g.c2, x, p, pp);
 }
 
@@ -319,10 +316,10 @@ __global__ void __launch_bounds__(64) k_wave_prefix(const BlockDesc* __restrict_
 }
 
 // Runs of 64 degrees at 64 nodes: the state at the run's start from
-// k_wave_start's matrices, the states at its chunks of 16 (for k_gram), the
+// k_wave_start's matrices, the states every 8 degrees (for k_gram), the
 // squared norms of F's rows over the run, and per chunk and tile of 8 nodes
 // the exponent of the largest chunk norm (c_k < 2^e); the degrees' constants
-// for k_gram.  Bound by FP64 instructions, 17 per degree and node.
+// for k_gram.  Bound by FP64 instructions, 15 per degree and node.
 // SPLIT: a workgroup per run and 64 nodes, a chunk per wavefront, which gets
 // to its chunk with the bare recurrence; else a run of 128 nodes per wavefront
 // (two per lane: half the reads of the degrees' constants), which a batch
@@ -381,15 +378,18 @@ __global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict_
                 }
             }
 #pragma unroll
-        for (int h = 0; h < NH; h++) pp[h] = p[h] - pp[h];
+        for (int h = 0; h < NH; h++) {
+            pp[h] = p[h] - pp[h];
+            shift(p[h], pp[h], E[h] + degs[0].e);
+        }
     }
     for (int c = 0; c < nc; c++) {
         if (SPLIT && c < wv) {
 #pragma unroll 4
             for (int j = 0; j < 16; j++) {
                 const Deg& g = degs[16 * c + j];
+                if ((j & 3) == 0 && c + j > 0) shift(p[0], pp[0], g.sh);
                 degree_step(g.c1, g.c2, x[0], p[0], pp[0]);
-                if ((j & 3) == 3) rescale(p[0], pp[0], E[0]);
             }
             continue;
         }
@@ -399,21 +399,20 @@ __global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict_
 #pragma unroll
         for (int h = 0; h < NH; h++) {
             ntm[h] = nte[h] = 0;
-            if (wave * 64 * NH + 64 * h < nP) {
-                at<double2>(arena, d.off_ck)[(int64_t)ch * nP + k[h]] = make_double2(p[h], pp[h]);
-                at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[(int64_t)ch * nP + k[h]] = E[h];
-            }
+            if (c > 0) shift(p[h], pp[h], degs[16 * c].sh);
         }
-#pragma unroll 4
+#pragma unroll 8
         for (int j = 0; j < 16; j++) {
             const Deg& g = degs[16 * c + j];
 #pragma unroll
             for (int h = 0; h < NH; h++) {
                 double ta, pb, pa, tb;
-                degree_rows(g, m, x[h], p[h], pp[h], E[h], ta, pb, pa, tb);
+                if ((j & 3) == 0 && j > 0) shift(p[h], pp[h], g.sh);
+                if ((j & 7) == 0 && wave * 64 * NH + 64 * h < nP)
+                    at<double2>(arena, d.off_ck)[(int64_t)(2 * ch + (j >> 3)) * nP + k[h]] = make_double2(p[h], pp[h]);
+                degree_rows(g, m, x[h], m > 0 ? x[h] : 1.0, p[h], pp[h], ta, pb, pa, tb);
                 ntm[h] = fma(ta, ta, fma(pb, pb, ntm[h]));
                 nte[h] = fma(pa, pa, fma(tb, tb, nte[h]));
-                if ((j & 3) == 3) rescale(p[h], pp[h], E[h]);
             }
         }
 #pragma unroll
@@ -460,21 +459,20 @@ __global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__
     if (in && lane < 16) degs[wv][lane] = degree(d, arena, d.lmin + 16 * c + lane);
     __syncthreads();
     if (!in) return;
-    const int64_t ci = (int64_t)c * nP + k, ldf = 2 * (int64_t)nP;
+    const int64_t ci = 2 * (int64_t)c * nP + k, ldf = 2 * (int64_t)nP;
     const double* nd = at<double>(arena, d.off_node);
     const double x = nd[k], stm = nd[nP + k], ste = nd[2 * nP + k];
     const double2 s = at<double2>(arena, d.off_ck)[ci];
     double p = s.x, pp = s.y;
-    int E = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP)[ci];
     double* F = at<double>(arena, d.off_rows) + 32 * (int64_t)c * ldf + 2 * k;
 #pragma unroll 4
     for (int j = 0; j < 16; j++) {
         double ta, pb, pa, tb;
-        degree_rows(degs[wv][j], m, x, p, pp, E, ta, pb, pa, tb);
+        if ((j & 3) == 0 && j > 0) shift(p, pp, degs[wv][j].sh);
+        degree_rows(degs[wv][j], m, x, m > 0 ? x : 1.0, p, pp, ta, pb, pa, tb);
         *reinterpret_cast<double2*>(F) = make_double2(stm * ta, ste * pa);
         *reinterpret_cast<double2*>(F + ldf) = make_double2(stm * pb, ste * tb);
         F += 2 * ldf;
-        if ((j & 3) == 3) rescale(p, pp, E);
     }
 }
 
@@ -582,12 +580,12 @@ __global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc
 // wavefronts takes NC column tiles and for each its BAND_TILES tiles on and
 // below the diagonal (the column's own tile is both operands of the diagonal
 // one).  The rows of these tiles are made on the spot, a chunk of 16 degrees
-// at a time, from the states that k_wave_start kept (20 bytes instead of 512
+// at a time, from the states that k_wave_norms kept (32 bytes instead of 512
 // per node and chunk): eight tiles are the 64 lanes of a wavefront, which
 // makes degrees 4 w .. 4 w + 3; then the pairs are multiplied.  (Making the next
 // chunk in four more wavefronts beside the products gains nothing: FP64
 // instructions and FP64 MFMA do not overlap.  Bound by the two together:
-// 130 us without the products, 212 without the rows.)
+// 99 us without the products, 223 without the rows.)
 // A row's ridge covers a few chunks: a pair of tiles is multiplied over a
 // chunk only if the product of their largest chunk norms is at least 2^-60
 // tr (by Cauchy-Schwarz what is left out is smaller, below the last bit of
@@ -598,11 +596,12 @@ __global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc
 // The three pairs with the strip's ninth and tenth tile are a step of their
 // own over tiles 2 .. 9, where they count at all.
 // NC = 1 for batches that would leave CUs idle: two chunks per step in twice
-// the wavefronts, a pair each (one block of R/L = 200: 30 us; 38 a chunk at a
-// time).
+// the wavefronts, a pair each (one block of R/L = 200: 27 us; 38 a chunk at a
+// time, before degrees lost their exponents).
 // An element sums the same products in the same order for either NC, so its
 // bits do not depend on the batch.
-// 222 blocks of R/L = 200: 296 us; with F's rows stored by a kernel of their
+// 222 blocks of R/L = 200: 271 us (309 with an exponent and a power of two per
+// degree and the states every 16 degrees); with F's rows stored by a kernel of their
 // own and read back 478 + 124 us, bound by the loads' latency.
 template <int NC>
 __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
@@ -614,10 +613,11 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
     constexpr int PS = NC == 4 ? BAND_TILES : 1;       // pairs per wavefront
     static_assert(NW * PS <= 32 && (NC == 4 || NW >= BAND_TILES), "a bit and a place for every pair");
     static_assert(NR <= NS + 2, "tiles 0 .. 7 and 2 .. 9");
+    constexpr int LATE = 1 << 30;
     __shared__ double W[NG][KS][PITCH];   // [2 (l - l0) + (0: a_l, 1: b_l)][row of eight tiles]
     alignas(16) __shared__ Deg degs[NG][16];
     __shared__ int nlist;
-    extern __shared__ int2 list[];    // chunk, first tile 0 or 2 (bit 10); pairs (bit PS w + i)
+    extern __shared__ int2 list[];    // chunk, LATE if from tile 2 on; pairs (bit PS w + i)
     const int b = blockIdx.y;
     const BlockDesc& d = desc[b];
     const BlockOut& o = out[b];
@@ -650,7 +650,7 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
             const unsigned long long ba = __ballot(pa != 0), bb = __ballot(pb != 0), below = (1ull << lane) - 1;
             const int i = n + __popcll(ba & below) + __popcll(bb & below);
             if (pa) list[i] = make_int2(c, (int)pa);
-            if (pb) list[i + (pa != 0)] = make_int2(c | 1 << 10, (int)pb);
+            if (pb) list[i + (pa != 0)] = make_int2(c | LATE, (int)pb);
             n += __popcll(ba) + __popcll(bb);
         }
         if (lane == 0) nlist = n;
@@ -660,7 +660,6 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
     const int k0 = 8 * (o.tile0 + J0);
     const double* nd = at<double>(arena, d.off_node);
     const double2* ck = at<double2>(arena, d.off_ck);
-    const int* cE = at<int>(arena, d.off_ck + 16 * (int64_t)d.n_chunks * nP);
     const int* dg = at<int>(arena, d.off_deg) + (tid & 255);   // 4 bytes of a chunk's constants per lane
     // this lane's node: in the (lane/8)-th of the step's eight tiles, from
     // tile 0 or tile 2 on (nodes past the block's are loaded as its last one
@@ -671,7 +670,7 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
     // states and constants of a step, loaded two steps ahead
     struct State {
         double2 s;
-        int E, dg, en, pm[NG];
+        int dg, en, pm[NG];
     };
     auto load = [&](int s, State& v) {
         v.en = __builtin_amdgcn_readfirstlane(list[min(NG * s + grp, ns - 1)].x);
@@ -680,10 +679,8 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
             const unsigned pm = list[min(NG * s + g, ns - 1)].y;
             v.pm[g] = NG * s + g < ns ? __builtin_amdgcn_readfirstlane((pm >> (PS * wv)) & ((1u << PS) - 1)) : 0;
         }
-        const int c = v.en & 1023;
-        const int64_t ci = (int64_t)c * nP + (v.en & 1024 ? kb : ka);
-        v.s = ck[ci];
-        v.E = cE[ci];
+        const int c = v.en & ~LATE;
+        v.s = ck[(int64_t)(2 * c + (sub >> 1)) * nP + (v.en & LATE ? kb : ka)];
         v.dg = dg[256 * c];
     };
     double4_t acc[PS];
@@ -697,21 +694,20 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
         // (every wavefront is past the constants of the step before)
         reinterpret_cast<int*>(degs)[tid] = v.dg;
         double p = v.s.x, pp = v.s.y;
-        int e = v.E;
         load(s + 2, v);
         __syncthreads();   // and past its products
         {
             // (lanes of tiles that no pair needs run along: numbers, never read)
-            const double x = en & 1024 ? xb : xa;
-#pragma unroll
-            for (int j = 0; j < 12; j += 4) {
-                if (j >= 4 * sub) break;
+            const double x = en & LATE ? xb : xa, xt = m > 0 ? x : 1.0;
+            if (sub & 1) {   // the state is kept every 8 degrees
+                const int j = 4 * (sub - 1);
                 double2 cc[4];
 #pragma unroll
                 for (int q = 0; q < 4; q++) cc[q] = *reinterpret_cast<const double2*>(&degs[grp][j + q].c1);
+                const int e = degs[grp][j + 4].sh;
 #pragma unroll
                 for (int q = 0; q < 4; q++) degree_step(cc[q].x, cc[q].y, x, p, pp);
-                rescale(p, pp, e);
+                shift(p, pp, e);
             }
             Deg g[4];
 #pragma unroll
@@ -720,7 +716,7 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 double ta, pb, pa, tb;
-                degree_rows(g[j], m, x, p, pp, e, ta, pb, pa, tb);
+                degree_rows(g[j], m, x, xt, p, pp, ta, pb, pa, tb);
                 w[j * PITCH] = make_double2(ta, pa);
                 w[j * PITCH + PITCH / 2] = make_double2(pb, tb);
             }
@@ -729,7 +725,7 @@ __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
 #pragma unroll
         for (int i = 0; i < NG * PS; i++)
             if (pm[i / PS] >> (i % PS) & 1) {
-                const double* wc = &W[i / PS][lk][li - (NC == 4 && en & 1024 ? 32 : 0)] + 16 * col_of(wv, i % PS);
+                const double* wc = &W[i / PS][lk][li - (NC == 4 && en & LATE ? 32 : 0)] + 16 * col_of(wv, i % PS);
                 const double* wr = wc + 16 * row_of(wv, i % PS);
                 double cv[KS / 4], rv[KS / 4];
 #pragma unroll
