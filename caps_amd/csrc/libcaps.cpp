@@ -3129,7 +3129,8 @@ int capsx_lu_logdet_batch_noalloc(double* dA, int dim, int lda, int n, double* d
     const int64_t off_buf = off_out + align256((int64_t)n * sizeof(BlockOut));
     // + 256: the trailing update's 16-byte operand loads may read one
     // element past the last U buffer (odd lda), which must stay in the array
-    const int64_t need = off_buf + (int64_t)n * per + 256;
+    const int64_t need = align256((int64_t)n * 192) + align256((int64_t)n * sizeof(LuSide)) + align256((int64_t)n * 48)
+                       + (int64_t)n * per + 256;   // as the limit counts (NOALLOC_SCRATCH_BYTES)
     if (need > (int64_t)cap) {
         fprintf(stderr,
                 "capsx_lu_logdet_batch_noalloc: %d matrices of dimension %d need %lld bytes of scratch, the "

@@ -7,14 +7,16 @@
 // restricted to the step's own columns, followed by one K = 128 (K = 256)
 // update of the trailing matrix (schedules at capsd_launch_lu):
 //   k_lu_panel      one workgroup per matrix factors the N-k x 64 panel:
-//                   left-looking over leaves of 2..8 columns, each leaf held
+//                   left-looking over leaves of 2..16 columns, each leaf held
 //                   in registers (R rows per lane; 256, 512 or 1024 lanes by
 //                   panel height), pivot search reduced over the wavefronts,
 //                   rows swapped through a logical->physical row map in LDS
 //                   (no row moves in HBM during the panel); writes the
-//                   factored panel in pivoted order to a side buffer, the
-//                   pivots (LAPACK ipiv convention) and log|u_ii|;
+//                   row map, the pivots (LAPACK ipiv convention) and
+//                   log|u_ii|; k_lu_panel_copy takes the factored panel to a
+//                   side buffer in pivoted order;
 //   k_lu_swap_trsm  applies the row interchanges to the trailing columns
+//                   (gathered from the row map)
 //                   and solves U12 = L11^{-1} A12 (one lane per column),
 //                   writing U12 to the step's row-major U buffer;
 //   k_lu_gemm_dma   A22 -= L21 U12 on FP64 MFMA (v_mfma_f64_16x16x4f64),
@@ -86,6 +88,23 @@ __device__ __forceinline__ double* inv_buf(char* arena, const LuSide& sd, int pb
     return at<double>(arena, sd.off_inv) + (int64_t)pb * 2 * NB * NB;
 }
 
+// Pivoted blocks use the place of the delta form's inverses for what a panel's
+// row interchanges come to: the row map (row r holds what was row map[r] of
+// the panel), read by k_lu_panel_copy, and per panel of a step the same as
+// lists for k_lu_swap_trsm: where the panel's own 64 rows came from, and the
+// rows below them that took one of these (n; -1: only the pivots are known).
+struct PanelSwaps {
+    int top[3 * NB];   // NB each: top, dst, src
+    int n, pad_[63];
+};
+__device__ __forceinline__ int* row_map(char* arena, const LuSide& sd) { return at<int>(arena, sd.off_inv); }
+__device__ __forceinline__ PanelSwaps& panel_swaps(char* arena, const LuSide& sd, int pb)
+{
+    return at<PanelSwaps>(arena, sd.off_inv + 24 * 1024 * sizeof(int))[pb];
+}
+static_assert(24 * 1024 * sizeof(int) + NPANEL * sizeof(PanelSwaps) <= NPANEL * 2 * NB * NB * sizeof(double),
+              "fits the inverses' place");
+
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
 // log|1 + d| of a delta-form pivot u = 1 + d: log1p keeps the relative
@@ -124,16 +143,23 @@ __device__ __forceinline__ void wave_argmax(double& v, int& idx)
 }
 
 // Panel body: R rows per lane, leaves of LF columns, NT threads, the
-// left-looking update in chunks of CW columns of L (CW divides LF); the
-// logical->physical row map lives in dynamic LDS (R*NT ints).  Every leaf
-// re-reads the L columns left of it (64 columns, leaves of 4: 480 L columns
-// per panel; of 8: 224), while each column's pivot exchange and elimination
-// touch all R x LF leaf registers: leaves of 8 are the fastest measured.
+// left-looking update in chunks of CW columns of L (CW divides LF), the next
+// chunk loaded during this one; the logical->physical row map lives in
+// dynamic LDS (R*NT ints).  Bound by the chain of 64 columns, so a column has
+// one barrier: before it every wavefront publishes its candidate for the pivot
+// together with that row, and row c; after it everybody picks the winner.  Four
+// wavefronts, one per SIMD: what each of them does for itself is issued once per
+// SIMD.  Panels of up to 1024, 512 and 1200 rows: 142, 105 and 173 us
+// (two barriers a column, leaves of 8, the panel's copy at the end, the last
+// ones 8 rows a lane: 247, 163, 332).
 template <int R, int LF, int NT, int CW>
 __device__ __forceinline__ void lu_panel_body(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
                                               const LuSide* __restrict__ side, const BlockOut* __restrict__ out, int k,
                                               int pb)
 {
+    static_assert(NT >= NB, "row c < NB is row 0 of its lane");
+    constexpr int NW = NT / 64;
+    constexpr bool AHEAD = R <= 6;   // registers for the next chunk of L
     const int b = blockIdx.x;
     const BlockDesc& d = desc[b];
     if (out[b].skip || out[b].delta || k >= d.N) return;   // delta form: k_lu_diag / k_lu_l21
@@ -141,49 +167,60 @@ __device__ __forceinline__ void lu_panel_body(const BlockDesc* __restrict__ desc
     const int64_t lda = d.lda;
     const int np = N - k;                 // panel rows
     const int nbk = min(NB, np);          // panel columns
-    double* __restrict__ A = at<double>(arena, d.off_mat);
-    double* __restrict__ P = panel_buf(arena, side[b], lda, pb);
+    double* __restrict__ A = at<double>(arena, d.off_mat) + k + k * lda;
     double* __restrict__ logs = at<double>(arena, side[b].off_logs);
     int* __restrict__ ipiv = moved_buf(arena, side[b], pb);
-    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     extern __shared__ int perm[];   // R * NT
-    __shared__ double red_v2[2][NT / 64];
-    __shared__ int red_i2[2][NT / 64];
-    __shared__ double prow2[2][LF], xrow2[2][LF];
+    __shared__ double cand_v[2][NW], cand_row[2][NW][LF], xrow2[2][LF];
+    __shared__ int cand_i[2][NW];
     __shared__ double Uc[2][CW * LF];   // solved U rows of one chunk, [row][col]
     __shared__ double pivv[NB];         // |pivot| per panel column
+    __shared__ int moved;
 
-    for (int r = tid; r < np; r += NT) perm[r] = r;
+    for (int r = tid; r < R * NT; r += NT) perm[r] = r < np ? r : 0;   // (rows past the panel: computed, never used)
+    if (tid == 0) moved = 0;
     __syncthreads();
 
     double a[R][LF];
     for (int c0 = 0; c0 < nbk; c0 += LF) {
         const int w = min(LF, nbk - c0);
-        // load the leaf (logical rows, through the row map)
+        int held[AHEAD ? R : 1];   // logical rows, through the row map
+        if constexpr (AHEAD) {
 #pragma unroll
-        for (int i = 0; i < R; i++) {
-            const int r = tid + i * NT;
-#pragma unroll
-            for (int j = 0; j < LF; j++)
-                a[i][j] = (r < np && j < w) ? A[(k + perm[r]) + (k + c0 + j) * lda] : 0.0;
+            for (int i = 0; i < R; i++) held[i] = perm[tid + i * NT];
         }
+        auto row = [&](int i) { return A + (AHEAD ? held[AHEAD ? i : 0] : perm[tid + i * NT]); };
+#pragma unroll
+        for (int i = 0; i < R; i++)
+#pragma unroll
+            for (int j = 0; j < LF; j++) a[i][j] = row(i)[(c0 + min(j, w - 1)) * lda];
         // left-looking update with the panel's earlier columns, CW columns
         // of L per chunk.  Rows [cc0, cc0+CW) of the leaf (lanes cc0.. of
         // wave 0, register row 0) become final U rows by a forward
         // substitution inside the wavefront; every row below then subtracts
         // the chunk's rank-CW product.
+        double Ln[AHEAD ? R : 1][CW];
+        auto load_l = [&](int cc0, auto& L) {
+#pragma unroll
+            for (int i = 0; i < R; i++)
+#pragma unroll
+                for (int jj = 0; jj < CW; jj++) L[i][jj] = row(i)[(cc0 + jj) * lda];
+        };
+        if constexpr (AHEAD)
+            if (c0 > 0) load_l(0, Ln);
         for (int cc0 = 0; cc0 < c0; cc0 += CW) {
             const int buf = (cc0 / CW) & 1;
             double Lr[R][CW];
+            if constexpr (AHEAD) {
 #pragma unroll
-            for (int i = 0; i < R; i++) {
-                const int r = tid + i * NT;
-                const bool row_ok = r > cc0 && r < np;
-                const int64_t pr = k + (row_ok ? perm[r] : 0);
+                for (int i = 0; i < R; i++)
 #pragma unroll
-                for (int jj = 0; jj < CW; jj++)
-                    Lr[i][jj] = (row_ok && cc0 + jj < r) ? A[pr + (k + cc0 + jj) * lda] : 0.0;
+                    for (int jj = 0; jj < CW; jj++) Lr[i][jj] = Ln[i][jj];
+                load_l(min(cc0 + CW, c0 - CW), Ln);
+            } else {
+                load_l(cc0, Lr);
             }
             if (wid == 0) {
 #pragma unroll
@@ -215,66 +252,86 @@ __device__ __forceinline__ void lu_panel_body(const BlockDesc* __restrict__ desc
             }
         }
         // factor the leaf with partial pivoting (unrolled: j indexes registers)
-#pragma unroll
-        for (int j = 0; j < LF; j++) {
-            if (j >= w) break;
-            const int c = c0 + j;
-            // per-column scratch alternates between two buffers, so one
-            // barrier after the reduction and one after the pivot row is
-            // published suffice
-            double* red_v = red_v2[c & 1];
-            int* red_i = red_i2[c & 1];
-            double* prow = prow2[c & 1];
-            double* xrow = xrow2[c & 1];
+        static_for<LF>([&](auto jc) {
+            constexpr int j = jc;
+            if (j >= w) return;
+            const int c = c0 + j, par = c & 1;   // two buffers in turn: one barrier per column
             double bv = -1.0;
             int bi = 0x7fffffff;
 #pragma unroll
             for (int i = 0; i < R; i++) {
                 const int r = tid + i * NT;
                 const double v = fabs(a[i][j]);
-                if (r >= c && r < np && (v > bv || (v == bv && r < bi))) {
+                if ((i > 0 || r >= c) && r < np && v > bv) {   // rows ascend: the lowest of equal ones
                     bv = v;
                     bi = r;
                 }
             }
-            wave_argmax(bv, bi);
+            double m = bv;
+            m = fmax(m, dpp_d<DPP_QUAD_X1>(m));
+            m = fmax(m, dpp_d<DPP_QUAD_X2>(m));
+            m = fmax(m, dpp_d<DPP_HALF_MIRROR>(m));
+            m = fmax(m, dpp_d<DPP_MIRROR>(m));
+            m = fmax(fmax(lane_d(m, 0), lane_d(m, 16)), fmax(lane_d(m, 32), lane_d(m, 48)));
+            int p = 0x7fffffff;
+            if (m >= 0) {
+                unsigned long long has = __ballot(bv == m);
+                int from = __builtin_ctzll(has);
+                p = __builtin_amdgcn_readlane(bi, from);
+                while (has &= has - 1) {   // equal candidates: the lowest row
+                    const int l = __builtin_ctzll(has), o = __builtin_amdgcn_readlane(bi, l);
+                    if (o < p) {
+                        p = o;
+                        from = l;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < R; i++)
+                    if (p / NT == i && lane == from) {
+#pragma unroll
+                        for (int jj = 0; jj < LF; jj++) cand_row[par][wid][jj] = a[i][jj];
+                    }
+            }
             if (lane == 0) {
-                red_v[wid] = bv;
-                red_i[wid] = bi;
+                cand_v[par][wid] = m;
+                cand_i[par][wid] = p;
+            }
+            if (tid == c) {
+#pragma unroll
+                for (int jj = 0; jj < LF; jj++) xrow2[par][jj] = a[0][jj];
             }
             __syncthreads();
-            double gv = red_v[0];
-            int p = red_i[0];
-            for (int q = 1; q < NT / 64; q++)
-                if (red_v[q] > gv || (red_v[q] == gv && red_i[q] < p)) {
-                    gv = red_v[q];
-                    p = red_i[q];
-                }
+            double cv[NW];
+            int ci[NW], win = 0;
+#pragma unroll
+            for (int q = 0; q < NW; q++) {
+                cv[q] = cand_v[par][q];
+                ci[q] = cand_i[par][q];
+            }
+            double gv = cv[0];
+            p = ci[0];
+#pragma unroll
+            for (int q = 1; q < NW; q++) {   // (no branches)
+                const bool more = (cv[q] > gv) | ((cv[q] == gv) & (ci[q] < p));
+                gv = more ? cv[q] : gv;
+                p = more ? ci[q] : p;
+                win = more ? q : win;
+            }
+            p = __builtin_amdgcn_readfirstlane(p);
+            win = __builtin_amdgcn_readfirstlane(win);
+            const double* xrow = xrow2[par];
+            const double* from = cand_row[par][win];
             // no finite candidate (a column of NaN): keep row c, so the row
             // map and ipiv stay in range; the NaN reaches log|u| and the
             // determinant
             if (p >= np) {
                 p = c;
                 gv = NAN;
+                from = xrow;
             }
-            // owners of rows p and c publish them
-            const int own_p = p % NT, own_c = c % NT;
-            if (tid == own_p) {
+            double prow[LF];
 #pragma unroll
-                for (int i = 0; i < R; i++)
-                    if (tid + i * NT == p) {
-#pragma unroll
-                        for (int jj = 0; jj < LF; jj++) prow[jj] = a[i][jj];
-                    }
-            }
-            if (tid == own_c && p != c) {
-#pragma unroll
-                for (int i = 0; i < R; i++)
-                    if (tid + i * NT == c) {
-#pragma unroll
-                        for (int jj = 0; jj < LF; jj++) xrow[jj] = a[i][jj];
-                    }
-            }
+            for (int jj = 0; jj < LF; jj++) prow[jj] = from[jj];
             if (tid == 0) {
                 if (p != c) {
                     const int t = perm[c];
@@ -284,65 +341,85 @@ __device__ __forceinline__ void lu_panel_body(const BlockDesc* __restrict__ desc
                 pivv[c] = gv;
                 ipiv[c] = p;
             }
-            __syncthreads();
-            const double u = prow[j];
+            if (tid == c) {
 #pragma unroll
-            for (int i = 0; i < R; i++) {
-                const int r = tid + i * NT;
-                if (r == c) {
+                for (int jj = 0; jj < LF; jj++) a[0][jj] = prow[jj];
+            }
+            if (p != c) {
 #pragma unroll
-                    for (int jj = 0; jj < LF; jj++) a[i][jj] = prow[jj];
-                } else if (r == p) {
+                for (int i = 0; i < R; i++)
+                    if (p / NT == i && tid == p % NT) {
 #pragma unroll
-                    for (int jj = 0; jj < LF; jj++) a[i][jj] = xrow[jj];
-                }
+                        for (int jj = 0; jj < LF; jj++) a[i][jj] = xrow[jj];
+                    }
             }
             // l = a / u as a product with 1/u, as LAPACK's dgetf2 scales the
-            // column (a division only below the smallest normal number); u is
-            // the same in every lane, so the choice is uniform
-            const int by_rcp = __builtin_amdgcn_readfirstlane((int)(fabs(u) >= 2.2250738585072014e-308));
-            const double ru = 1.0 / u;
+            // column (below the smallest normal number both times 2^200)
+            const double u = prow[j], sc = fabs(u) >= 2.2250738585072014e-308 ? 1.0 : 0x1p200, ru = 1.0 / (u * sc);
+            double l[R];
 #pragma unroll
-            for (int i = 0; i < R; i++) {
-                const int r = tid + i * NT;
-                if (r > c && r < np) {
-                    const double l = by_rcp ? a[i][j] * ru : a[i][j] / u;
-                    a[i][j] = l;
+            for (int i = 0; i < R; i++) l[i] = (a[i][j] * sc) * ru;
+#pragma unroll
+            for (int i = 0; i < R; i++)
+                if (i > 0 || tid > c) {
+                    a[i][j] = l[i];
 #pragma unroll
                     for (int jj = 0; jj < LF; jj++)
-                        if (jj > j) a[i][jj] -= l * prow[jj];
+                        if (jj > j) a[i][jj] -= l[i] * prow[jj];
                 }
-            }
-        }
+        });
+        __syncthreads();   // the row map
         // write the leaf back through the row map
 #pragma unroll
         for (int i = 0; i < R; i++) {
             const int r = tid + i * NT;
             if (r < np) {
-                const int64_t pr = k + perm[r];
+                double* pr = A + perm[r];
 #pragma unroll
                 for (int j = 0; j < LF; j++)
-                    if (j < w) A[pr + (k + c0 + j) * lda] = a[i][j];
+                    if (j < w) pr[(c0 + j) * lda] = a[i][j];
             }
         }
         __syncthreads();
     }
-    // log|u_ii| and the panel in pivoted (logical) order
     if (tid < nbk) logs[k + tid] = log(pivv[tid]);
+    int* map = row_map(arena, side[b]);
+    PanelSwaps& ps = panel_swaps(arena, side[b], pb);
     for (int r = tid; r < np; r += NT) {
-        const int64_t pr = k + perm[r];
-#pragma unroll
-        for (int j0 = 0; j0 < NB; j0 += 16) {
-            double v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = j0 + j < nbk ? A[pr + (k + j0 + j) * lda] : 0.0;
-#pragma unroll
-            for (int j = 0; j < 16; j++)
-                if (j0 + j < nbk) P[r + (j0 + j) * lda] = v[j];
+        const int o = perm[r];
+        map[r] = o;
+        if (r < NB) ps.top[r] = o;
+        else if (o != r) {
+            const int e = atomicAdd(&moved, 1);   // at most NB rows, in any order
+            ps.top[NB + e] = r;
+            ps.top[2 * NB + e] = o;
         }
     }
+    __syncthreads();
+    if (tid == 0) ps.n = moved;
 }
 
+// The factored panel in pivoted (logical) order: 256 rows and 16 columns per
+// workgroup (at the end of the panel's one workgroup it took 43 us of 245).
+__global__ void __launch_bounds__(256) k_lu_panel_copy(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                       const LuSide* __restrict__ side,
+                                                       const BlockOut* __restrict__ out, int k, int pb)
+{
+    const int b = blockIdx.z;
+    const BlockDesc& d = desc[b];
+    const int r = blockIdx.x * 256 + threadIdx.x, np = d.N - k;
+    if (out[b].skip || out[b].delta || r >= np) return;
+    const int64_t lda = d.lda;
+    const int j0 = 16 * blockIdx.y, nj = min(16, min(NB, np) - j0);
+    const double* A = at<double>(arena, d.off_mat) + k + (k + j0) * lda + row_map(arena, side[b])[r];
+    double* P = panel_buf(arena, side[b], lda, pb) + r + j0 * lda;
+    double v[16];
+#pragma unroll
+    for (int j = 0; j < 16; j++) v[j] = A[min(j, max(nj - 1, 0)) * lda];
+#pragma unroll
+    for (int j = 0; j < 16; j++)
+        if (j < nj) P[j * lda] = v[j];
+}
 
 // ---- delta form: panels without pivot search --------------------------------
 // For a column diagonally dominant 1 - M (the matrix holds -M, out[b].delta)
@@ -854,6 +931,7 @@ __global__ void __launch_bounds__(GP_ROWS) k_gp_copy(const BlockDesc* __restrict
     const double* A = at<double>(arena, d.off_mat);
     double* P = panel_buf(arena, side[b], lda, pb);
     const int r = k + blockIdx.x * GP_ROWS + threadIdx.x;
+    if (r == k) panel_swaps(arena, side[b], pb).n = -1;
     if (r >= N) return;
     for (int j = 0; j < nbk; j++) P[(r - k) + (int64_t)j * lda] = A[r + (int64_t)(k + j) * lda];
 }
@@ -891,7 +969,10 @@ __device__ __forceinline__ void swap_rows_ipiv(double* __restrict__ Ac, const in
 // (relative to row k + q NB); then the column's 64 entries are solved in
 // registers with the unit lower L11 of panel buffer pb, staged once per
 // workgroup in LDS (every lane reads the same L11 entry at a time: one
-// broadcast LDS read instead of a vector load per entry).
+// broadcast LDS read instead of a vector load per entry).  A panel's
+// interchanges come to a gather of its 64 rows and at most 64 moves from them
+// to rows below, all independent loads, from the lists in PanelSwaps (one
+// exchange after the other: 85 us for 4 matrices of 1200, 45 so).
 template <int NTH>
 __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
                                                       const LuSide* __restrict__ side,
@@ -908,17 +989,55 @@ __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restric
     const int64_t lda = d.lda;
     const double* P = panel_buf(arena, side[b], lda, pb);
     for (int idx = threadIdx.x; idx < NB * NB; idx += NTH) sL[idx] = P[(idx % NB) + (int64_t)(idx / NB) * lda];
+    __shared__ int lists[NPANEL][3 * NB], counts[NPANEL];   // of the panels in swaps: PanelSwaps' top, dst, src; n
+    for (int q = 0; q < NPANEL; q++)
+        if ((swaps >> q) & 1) {
+            const PanelSwaps& ps = panel_swaps(arena, side[b], q);
+            for (int i = threadIdx.x; i < 3 * NB; i += NTH) lists[q][i] = ps.top[i];
+            if (threadIdx.x == 0) counts[q] = ps.n;
+        }
     __syncthreads();
     const int col = r0 + cs_off + blockIdx.x * NTH + threadIdx.x;
     if (col >= cend) return;
     double* Ac = at<double>(arena, d.off_mat) + (int64_t)col * lda;
     // the pivots of the panel at row k + q NB cover min(NB, N - k - q NB)
-    // columns
-    for (int q = 0; q < NPANEL; q++)
-        if ((swaps >> q) & 1) swap_rows_ipiv(Ac, moved_buf(arena, side[b], q), min(NB, N - k - q * NB), k + q * NB);
+    // columns; the lists cover full panels (all but the last, which has no
+    // columns behind it)
     double x[NB];
+    bool have = false;   // x: the 64 rows after panel q = pb's interchanges
+    for (int q = 0; q < NPANEL; q++)
+        if ((swaps >> q) & 1) {
+            const int *top = lists[q], *dst = top + NB, *src = dst + NB;
+            const int n = __builtin_amdgcn_readfirstlane(counts[q]), rq = k + q * NB;
+            if (rq + NB > N) continue;
+            if (n < 0) {
+                swap_rows_ipiv(Ac, moved_buf(arena, side[b], q), NB, rq);
+            } else {
+                double z[NB];
 #pragma unroll
-    for (int i = 0; i < NB; i++) x[i] = Ac[r0 + i];
+                for (int i = 0; i < NB; i++) z[i] = Ac[rq + top[i]];
+                for (int e0 = 0; e0 < n; e0 += 16) {   // rows below: from the 64
+                    double y[16];
+#pragma unroll
+                    for (int e = 0; e < 16; e++) y[e] = Ac[rq + src[min(e0 + e, n - 1)]];
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        if (e0 + e < n) Ac[rq + dst[e0 + e]] = y[e];
+                }
+                if (q == pb) {
+                    have = true;
+#pragma unroll
+                    for (int i = 0; i < NB; i++) x[i] = z[i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NB; i++) Ac[rq + i] = z[i];
+                }
+            }
+        }
+    if (!have) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) x[i] = Ac[r0 + i];
+    }
 #pragma unroll
     for (int i = 0; i < NB; i++) {
 #pragma unroll
@@ -1360,8 +1479,12 @@ __global__ void k_lu_fill(const BlockDesc* __restrict__ desc, char* __restrict__
 // (each GPU holds its own copy until the process ends); host code never
 // uses the array's name as an address, only the pointer that
 // hipGetSymbolAddress returns for the device (noalloc_scratch_ptr).
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;
-static __device__ __align__(256) char scratch[NOALLOC_SCRATCH_BYTES];
+// The bytes count a batch by what its descriptors had when the limit was set
+// (192 and 48 bytes), so that what fits does not depend on their size; the
+// margin holds the rest (a matrix takes 0.5 MiB and more: fewer than 128).
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20, NOALLOC_MARGIN = (size_t)64 << 10;
+static_assert(128 * (sizeof(BlockDesc) - 192 + sizeof(BlockOut) - 48) + 512 <= NOALLOC_MARGIN, "descriptors fit");
+static __device__ __align__(256) char scratch[NOALLOC_SCRATCH_BYTES + NOALLOC_MARGIN];
 
 // Descriptors of n column-major dim x dim matrices at the caller's pointer
 // (arena offset a_off, matrix b at a_off + b lda dim doubles): BlockDesc at
@@ -1426,9 +1549,9 @@ int capsd_lu_nb(void) { return NB; }
 // needs 24 rows per lane).
 static int grid_panel_rows = 6144;
 // one-workgroup panel variants (CAPS_AMD_PANEL_SET): 1 (default) = leaves
-// of 8 columns with 256-lane workgroups up to 2560 rows, 0 = leaves of 4
-// above 512 rows.  Both give bit-identical factors: every entry subtracts
-// the same products in the same column order.
+// of 16 columns up to 2048 rows, then 8, with 256-lane workgroups up to 1024
+// rows, 0 = leaves of 4 above 512 rows.  Both give bit-identical factors:
+// every entry subtracts the same products in the same column order.
 static int panel_set = 1;
 // trailing-update kernel of the 128 x 128 tile (CAPS_AMD_GEMM_KERNEL):
 // k_lu_gemm_dma (operand stages moved straight into LDS, double-buffered)
@@ -1460,12 +1583,12 @@ static void launch_panel(int rows, const BlockDesc* desc, char* arena, const LuS
         }
         hipLaunchKernelGGL(k_gp_copy, dim3(nch, nb), dim3(GP_ROWS), 0, s, desc, arena, side, out, k, pb);
     } else if (panel_set == 1) {
-        // leaves of 8 left-looking in chunks of 4 (2 at 2560 rows), two
-        // 256-lane workgroups per CU up to 2560 rows
-        if (rows <= 2 * 256) PANEL(2, 8, 256, 2);
-        else if (rows <= 4 * 256) PANELC(4, 8, 256, 2, 4);
-        else if (rows <= 8 * 256) PANELC(8, 8, 256, 2, 4);
-        else if (rows <= 10 * 256) PANELC(10, 8, 256, 2, 2);
+        // left-looking in chunks of 4: leaves of 16 read the L columns left of
+        // them 96 times a panel, of 8 224 times (1024 rows: 142 and 160 us);
+        // 2048 rows as 4 per lane of 512: 173 us at 1200, as 8 of 256 332
+        if (rows <= 2 * 256) PANELC(2, 16, 256, 2, 4);
+        else if (rows <= 4 * 256) PANELC(4, 16, 256, 2, 4);
+        else if (rows <= 4 * 512) PANELC(4, 16, 512, 2, 4);
         else if (rows <= 6 * 512) PANELC(6, 8, 512, 2, 4);
         else if (rows <= 12 * 512) PANELC(12, 8, 512, 2, 1);
         else PANEL(24, 2, 1024, 4);
@@ -1480,6 +1603,9 @@ static void launch_panel(int rows, const BlockDesc* desc, char* arena, const LuS
     }
 #undef PANEL
 #undef PANELC
+    if (rows <= grid_panel_rows)
+        hipLaunchKernelGGL(k_lu_panel_copy, dim3((rows + 255) / 256, NB / 16, nb), dim3(256), 0, s, desc, arena, side,
+                           out, k, pb);
 }
 
 int capsd_noalloc_scratch(char** ptr, size_t* bytes);
@@ -1649,7 +1775,9 @@ int capsd_launch_lu(const BlockDesc* desc, char* arena, const void* side, BlockO
         const int c0 = k + pb * NB + cs_off;
         const int n = min(maxN - c0, cols);
         if (n <= 0) return;
-        if (piv && n > 64)
+        // workgroups of one wavefront while those of four would leave CUs
+        // without any (4 matrices of 1200: 45 and 56 us)
+        if (piv && (int64_t)((n + 255) / 256) * nblocks >= 256)
             hipLaunchKernelGGL(k_lu_swap_trsm<256>, dim3((n + 255) / 256, nblocks), dim3(256), 0, s, desc, arena, sd,
                                out, k, pb, cs_off, cols, swaps);
         else if (piv)

@@ -4,7 +4,22 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <utility>
+
 namespace capsd {
+
+// f(0) .. f(N - 1) with constants (register arrays that a loop too long for
+// "#pragma unroll" would send to scratch memory)
+template <class F, int... I>
+__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for_(f, std::make_integer_sequence<int, N>{});
+}
 
 template <int CTRL>
 __device__ __forceinline__ int dpp_i(int x)

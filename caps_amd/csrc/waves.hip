@@ -809,17 +809,6 @@ __device__ __forceinline__ double row_d(double x)
         __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(x), 0x150 + N, 0xf, 0xf, true));
 }
 
-template <int N, class F, int... I>
-__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>)
-{
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f)
-{
-    static_for_<N>(f, std::make_integer_sequence<int, N>{});
-}
-
 // log det(1 - G) of one block by LDLᵀ without pivoting (1 - G is symmetric
 // positive definite, so the elimination is stable in any order), in the
 // delta form: the matrix holds -G, pivots are u = 1 + d with d the stored
