@@ -183,18 +183,19 @@ def hbm_probe(nbytes=1 << 30, reps=3):
                       "dispatches": reps}))
 
 
-def gemm_traffic():
-    """HBM bytes per k_lu_gemm_dma launch measured with FETCH_SIZE and
-    WRITE_SIZE (profiles/k_lu_gemm_dma_c2_traffic.txt, scaled by the copy
-    calibration), or None when that summary is absent."""
-    path = os.path.join(ROOT, "profiles", "k_lu_gemm_dma_c2_traffic.txt")
-    if not os.path.exists(path):
-        return None
-    with open(path) as f:
-        for line in f:
-            if line.startswith("hbm_bytes_per_launch"):
-                return float(line.split("=")[1])
-    return None
+def gram_counters():
+    """FP64 operations and HBM bytes of k_gram in one step of this workload,
+    measured with SQ_INSTS_VALU_*_F64, FETCH_SIZE and WRITE_SIZE
+    (profiles/k_gram_c2_counters.txt); empty when that summary is absent."""
+    path = os.path.join(ROOT, "profiles", "k_gram_c2_counters.txt")
+    out = {}
+    if os.path.exists(path):
+        with open(path) as f:
+            for line in f:
+                if "_per_launch" in line:
+                    k, v = line.split("=")
+                    out[k.strip()] = float(v)
+    return out
 
 
 def large_aspect(ca):
@@ -419,13 +420,6 @@ def main():
     print("bench: eager step %.3f s" % dte, file=sys.stderr, flush=True)
     st_steps = 1
 
-    # one more step with HIP events around every launch of the dominant
-    # kernel (the LU's trailing update); its launches then run one at a time
-    c.profile(True)
-    gpu_step(c, form)
-    prof = c.stats(reset=True)
-    c.profile(False)
-
     heuristic = None
     if form == "surrogate":
         Fh, nbh, nch, dth = gpu_step(c, "batched")
@@ -438,20 +432,18 @@ def main():
                  "speedup_vs_plain": (nb / (total / args.steps)) / (nbp / dtp)}
         print("bench: plain step %.3f s, %d blocks" % (dtp, nbp), file=sys.stderr, flush=True)
 
-    # dominant kernel: the LU's trailing update (k_lu_gemm_dma), FP64 MFMA;
-    # its launches only (the trailing updates of regions one panel wide or
-    # high run on k_lu_gemm tiles and are reported beside it)
-    gemm_s = prof["gemm_ms"] / 1e3
-    achieved = prof["gemm_flops"] / gemm_s / 1e12 if gemm_s > 0 else None
-    roof = {"kernel": "k_lu_gemm_dma", "bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS,
-            "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS if achieved else None, "traffic": gemm_traffic(),
-            "traffic_source": "stored: profiles/k_lu_gemm_dma_c2_traffic.txt (FETCH_SIZE + WRITE_SIZE runs)",
-            "launches": prof["gemm_launches"],
-            "avg_launch_us": 1e3 * prof["gemm_ms"] / max(1, prof["gemm_launches"]),
-            "flops_per_launch": prof["gemm_flops"] / max(1, prof["gemm_launches"]),
-            "algorithmic_bytes_per_launch": prof["gemm_bytes"] / max(1, prof["gemm_launches"]),
-            "arithmetic_intensity_flop_per_byte": prof["gemm_flops"] / max(1.0, prof["gemm_bytes"]),
-            "other_update_launches_ms": prof["other_update_ms"]}
+    # dominant kernel: the band of the Gram matrix (k_gram), FP64 MFMA and
+    # vector instructions on the same units; its stage holds that kernel alone
+    gram_s = st["stage_ms"]["assemble"] / 1e3
+    cnt = gram_counters()
+    flops = cnt.get("mfma_flops_per_launch", 0) + cnt.get("vector_flops_per_launch", 0)
+    achieved = flops / gram_s / 1e12 if gram_s > 0 and flops else None
+    roof = {"kernel": "k_gram", "bound": "fp64 (mfma + vector)", "achieved": achieved, "peak": FP64_PEAK_TFLOPS,
+            "unit": "TFLOP/s", "frac": achieved / FP64_PEAK_TFLOPS if achieved else None,
+            "traffic": cnt.get("hbm_bytes_per_launch"),
+            "traffic_source": "stored: profiles/k_gram_c2_counters.txt (operations, FETCH_SIZE + WRITE_SIZE runs)",
+            "launches": 1, "avg_launch_us": 1e6 * gram_s, "flops_per_launch": flops or None,
+            "mfma_flops_per_launch": cnt.get("mfma_flops_per_launch")}
     lu_s = st["stage_ms"]["lu"] / 1e3
     mixed = None if args.no_mixed else mixed_aspect(caps_amd, args.steps)
     large = None if args.no_large else large_aspect(caps_amd)
