@@ -120,6 +120,7 @@ struct BlockOut {
     int tile0, tiles;   // the nodes that matter: tiles of 8 nodes (G has
                         // 16 tiles rows)
     int etr;            // exponent of the trace
+    int64_t t_end;      // wall_clock64 at the end of k_band_ldl
 };
 
 }  // namespace capsd

@@ -35,12 +35,13 @@ using capsd::MieDesc;
 struct capsx_mlp;
 extern "C" {
 void capsx_mlp_predict(capsx_mlp* h, const float* X, int n, float* Y);
-void capsd_launch_wave_start(const void*, int, int, const BlockDesc*, char*, int, int, int*, hipStream_t);
-void capsd_launch_wave_norms(const BlockDesc*, char*, int, int, int, int, int, hipStream_t);
+void capsd_launch_upload(const void*, void*, size_t, hipStream_t);
+void capsd_launch_wave_start(const void*, int, int, const BlockDesc*, char*, int, int, int*, int64_t*, hipStream_t);
+void capsd_launch_wave_norms(const BlockDesc*, char*, int, int, int, int, int, int64_t*, hipStream_t);
 void capsd_launch_wave_window(BlockDesc*, char*, BlockOut*, const int*, int, int, int, hipStream_t);
 void capsd_launch_wave_rows(const BlockDesc*, char*, int, int, hipStream_t);
-void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, int, hipStream_t);
-void capsd_launch_band_ldl(const BlockDesc*, char*, BlockOut*, int, int, hipStream_t);
+void capsd_launch_gram(const BlockDesc*, char*, const BlockOut*, int, int, int, int, int, int64_t*, hipStream_t);
+void capsd_launch_band_ldl(const BlockDesc*, char*, BlockOut*, BlockOut*, int, int, int64_t*, hipStream_t);
 void capsd_launch_band_dense(const BlockDesc*, char*, const BlockOut*, int, int, int, hipStream_t);
 void capsd_launch_wave_matrix(const BlockDesc*, char*, const BlockOut*, int, int, int, int, hipStream_t);
 void capsd_launch_a0(const BlockDesc*, char*, const double*, int, hipStream_t);
@@ -126,7 +127,7 @@ struct Ctx {
     hipEvent_t lu_ready = nullptr;        // a batch's dense matrices written
     char* arena = nullptr;
     size_t arena_size = 0;
-    // what a batch uploads, in one copy: the status word (zero), the block
+    // what a batch uploads at once: the status word (zero), the block
     // descriptors and right behind those in use the Mie tables' descriptors
     char* d_up = nullptr;
     char* h_up = nullptr;         // pinned
@@ -139,6 +140,8 @@ struct Ctx {
     LuSide* h_side = nullptr;
     BlockOut* h_out = nullptr;
     int* h_status = nullptr;
+    int64_t* h_clock = nullptr;   // pinned: when the stages of a banded batch began (stage_begins)
+    double clock_khz = 0;
     char* h_stage = nullptr;      // pinned, two pieces of copy_out
     hipEvent_t staged[2] = {};
     // staging buffer of the point APIs (capsx_*_points), grown on demand
@@ -189,7 +192,12 @@ Ctx* ctx_of(caps_t* self)
             HIPCHECK(hipEventCreateWithFlags(&c->lu_done[g], hipEventDisableTiming));
         }
         HIPCHECK(hipEventCreateWithFlags(&c->lu_ready, hipEventDisableTiming));
-        HIPCHECK(hipHostMalloc((void**)&c->h_status, sizeof(int), hipHostMallocDefault));
+        HIPCHECK(hipHostMalloc((void**)&c->h_status, 256, hipHostMallocDefault));
+        c->h_clock = (int64_t*)((char*)c->h_status + 64);
+        int dev, khz;
+        HIPCHECK(hipGetDevice(&dev));
+        HIPCHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+        c->clock_khz = khz;
         self->priv = c;
     }
     return (Ctx*)self->priv;
@@ -239,7 +247,7 @@ void ensure_blocks(Ctx* c, int n)
         hipHostFree(c->h_side);
         hipHostFree(c->h_out);
     }
-    const size_t up = UP_HEAD + cap * (sizeof(BlockDesc) + sizeof(MieDesc));
+    const size_t up = UP_HEAD + cap * (sizeof(BlockDesc) + sizeof(MieDesc)) + 16;   // (copied in words of 16 bytes)
     HIPCHECK(hipMalloc(&c->d_up, up));
     HIPCHECK(hipHostMalloc((void**)&c->h_up, up, hipHostMallocDefault));
     memset(c->h_up, 0, UP_HEAD);
@@ -561,6 +569,7 @@ struct BatchPlan {
     size_t bytes = 0;
     Job job = JOB_LOGDET;
     Form form = FORM_BAND;
+    bool banded() const { return job == JOB_LOGDET && form == FORM_BAND; }
     int dmode = 0;      // dense_mode of the determinant
     int gram_cols = 4;  // k_gram's column tiles per workgroup
     // determinant forms the LU launches kernels for (capsd_launch_lu kinds):
@@ -828,14 +837,15 @@ int k_segments(const BatchPlan& p)
 }
 
 // The kernels of one planned batch on the library's stream (and the LU
-// streams); stage events between the stages when `events`.  Returns the
+// streams); stage events between the stages when `events` (a banded batch's
+// kernels take the times themselves).  Returns the
 // number of trailing-update launches of the first LU group.
 int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
 {
     const int n = p.n;
     hipStream_t s = c->stream;
     auto mark = [&](int i) {
-        if (events) HIPCHECK(hipEventRecord(c->ev[i], s));
+        if (events && !p.banded()) HIPCHECK(hipEventRecord(c->ev[i], s));
     };
     mark(0);
     if (p.job == JOB_TABLES) {
@@ -849,9 +859,11 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
         return 0;
     }
     const bool det = p.job != JOB_MATRIX, piv = p.job == JOB_PIVOTED;
-    capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.u_start, c->d_status, s);
+    auto clock = [&](int i) { return p.banded() ? c->h_clock + i : nullptr; };
+    capsd_launch_wave_start(c->d_desc + n, p.ntab, p.max_mie, c->d_desc, c->arena, n, p.u_start, c->d_status,
+                            clock(0), s);
     mark(1);
-    capsd_launch_wave_norms(c->d_desc, c->arena, n, p.u_split, p.u_pair, p.max_runs, p.max_waves, s);
+    capsd_launch_wave_norms(c->d_desc, c->arena, n, p.u_split, p.u_pair, p.max_runs, p.max_waves, clock(1), s);
     if (det)
         capsd_launch_wave_window(c->d_desc, c->arena, c->d_out, c->d_status, n, piv ? 0 : g_delta_mode,
                                  p.form == FORM_GRAM, s);
@@ -863,7 +875,7 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
                                  det && !piv && p.lu_kinds == 6, s);
     else
         capsd_launch_gram(c->d_desc, c->arena, c->d_out, n, p.max_waves, (p.max_ldim + 15) / 16, p.gram_cols,
-                          p.form == FORM_BAND, s);
+                          p.form == FORM_BAND, clock(3), s);
     // the symmetric delta-form LU reads nothing above the diagonal outside its
     // 64 x 64 diagonal blocks; k_frobenius (LU mode) reads all of the matrix
     if (p.form == FORM_GRAM)
@@ -873,7 +885,7 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
     mark(4);
     if (!det) return 0;
     if (p.form == FORM_BAND) {
-        capsd_launch_band_ldl(c->d_desc, c->arena, c->d_out, n, p.dmode != 0, s);
+        capsd_launch_band_ldl(c->d_desc, c->arena, c->d_out, c->h_out, n, p.dmode != 0, clock(4), s);
         return 0;
     }
     HIPCHECK(hipEventRecord(c->lu_ready, s));
@@ -891,7 +903,7 @@ std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
         int levels, streams, xcd, tile;
         int lu_bnd[MAX_LU_STREAMS + 1], lu_gN[MAX_LU_STREAMS];   // the LU's stream groups (lu_groups)
         int lu_kernels[3], grid_panel_rows;   // LU kernel variants (capsx_lu_kernels, capsx_lu_grid_panel_rows)
-        const void *arena, *desc, *side, *out;
+        const void *arena, *desc, *side, *out, *host;
     } k;
     memset(&k, 0, sizeof(k));
     k.n = p.n;
@@ -931,6 +943,7 @@ std::vector<char> graph_key(Ctx* c, const BatchPlan& p)
     k.desc = c->d_desc;
     k.side = c->d_side;
     k.out = c->d_out;
+    k.host = c->h_out;
     const char* b = reinterpret_cast<const char*>(&k);
     return std::vector<char>(b, b + sizeof(k));
 }
@@ -944,8 +957,7 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p)
     const bool det = p.job == JOB_LOGDET || p.job == JOB_PIVOTED;
     hipStream_t s = c->stream;
     ensure_arena(c, p.bytes);
-    HIPCHECK(hipMemcpyAsync(c->d_up, c->h_up, UP_HEAD + n * sizeof(BlockDesc) + p.ntab * sizeof(MieDesc),
-                            hipMemcpyHostToDevice, s));
+    capsd_launch_upload(c->h_up, c->d_up, UP_HEAD + n * sizeof(BlockDesc) + p.ntab * sizeof(MieDesc), s);
     if (det && p.form != FORM_BAND)
         HIPCHECK(hipMemcpyAsync(c->d_side, c->h_side, n * sizeof(LuSide), hipMemcpyHostToDevice, s));
     const int nupd = capsd_lu_max_updates(p.maxN);
@@ -956,7 +968,7 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p)
         for (size_t i = old; i < c->gemm_ev.size(); i++) HIPCHECK(hipEventCreate(&c->gemm_ev[i]));
     }
     int nlaunched = 0;
-    const bool use_graph = c->graph && !c->prof;
+    const bool use_graph = c->graph && !c->prof, band = p.banded();
     if (use_graph) {
         const std::vector<char> key = graph_key(c, p);
         hipGraphExec_t exec = nullptr;
@@ -975,29 +987,38 @@ void run_batch(caps_t* self, Ctx* c, const BatchPlan& p)
             }
             c->graphs.push_back({key, exec});
         }
-        HIPCHECK(hipEventRecord(c->ev[0], s));
+        if (!band) HIPCHECK(hipEventRecord(c->ev[0], s));
         HIPCHECK(hipGraphLaunch(exec, s));
     } else {
         nlaunched = enqueue_batch(c, p, true);
     }
-    HIPCHECK(hipEventRecord(c->ev[5], s));
+    if (!band) HIPCHECK(hipEventRecord(c->ev[5], s));
     HIPCHECK(hipGetLastError());
-    // a determinant's status comes with its results
-    if (det) HIPCHECK(hipMemcpyAsync(c->h_out, c->d_out, n * sizeof(BlockOut), hipMemcpyDeviceToHost, s));
+    // a determinant's status comes with its results, those of the band with its last kernel
+    if (band) {
+    } else if (det) HIPCHECK(hipMemcpyAsync(c->h_out, c->d_out, n * sizeof(BlockOut), hipMemcpyDeviceToHost, s));
     else HIPCHECK(hipMemcpyAsync(c->h_status, c->d_status, sizeof(int), hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     float ms;
     if (use_graph) {
         // a replayed graph is timed as a whole (no stage events inside)
         for (int i = 0; i < 5; i++) c->timing[i] = 0;
-    } else {
+    } else if (!band) {
         for (int i = 0; i < 5; i++) {
             HIPCHECK(hipEventElapsedTime(&ms, c->ev[i], c->ev[i + 1]));
             c->timing[i] = ms;
         }
     }
-    HIPCHECK(hipEventElapsedTime(&ms, c->ev[0], c->ev[5]));
-    c->timing[5] = ms;
+    if (band) {
+        int64_t t[6] = {c->h_clock[0], c->h_clock[1], c->h_clock[3], c->h_clock[3], c->h_clock[4], c->h_clock[4]};
+        for (int b = 0; b < n; b++) t[5] = std::max(t[5], c->h_out[b].t_end);
+        if (!use_graph)
+            for (int i = 0; i < 5; i++) c->timing[i] = (t[i + 1] - t[i]) / c->clock_khz;
+        c->timing[5] = (t[5] - t[0]) / c->clock_khz;
+    } else {
+        HIPCHECK(hipEventElapsedTime(&ms, c->ev[0], c->ev[5]));
+        c->timing[5] = ms;
+    }
     const int status = det ? c->h_out[0].status : *c->h_status;
     TERMINATE(status != 0, "non-finite k-integral (flags %d) in a batch of %d blocks (xi_=%g, m=%d ...)", status, n,
               c->h_desc[0].xi_, c->h_desc[0].m);

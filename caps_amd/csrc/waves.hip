@@ -19,6 +19,7 @@
 // of 96; R/L = 2000, ldim = 12000: 24000 become about 1300.
 //
 // Kernels (blockIdx.y, or .x of the last, selects the block):
+//   k_upload       the descriptors;
 //   k_wave_start   the Mie coefficients of each (object, ξ), and beside them
 //                  the nodes with the degree recurrence of P_l^m over all l,
 //                  whose state is kept at the start of every 16 degrees;
@@ -123,6 +124,22 @@ __device__ __forceinline__ void next_run(double2 a, double2 b, int e, double& p,
     E += e + f;
 }
 
+// A batch's descriptors from pinned host memory.  A batch of one block is some
+// 80 us of kernels; a copy command before them, one for the results behind them (now
+// stores of k_band_ldl to pinned memory) and a timed event between every two stages
+// (now stores of the time by their first workgroups) took another 27 us (116, now 89; of an energy at T = 0, five batches: 2.20 ms, now 1.93).
+__global__ void __launch_bounds__(256) k_upload(const uint4* __restrict__ host, uint4* __restrict__ dev, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dev[i] = host[i];
+}
+
+// The time at which a stage began (clock: pinned host memory, or none).
+__device__ __forceinline__ void stage_begins(int64_t* clock)
+{
+    if (clock && threadIdx.x == 0 && blockIdx.x == 0 && blockIdx.y == 0) *clock = wall_clock64();
+}
+
 // The first ntab mie_units workgroups: Mie coefficients, one lane per l.  Then
 // per block, 64 nodes per wavefront, one lane each: the degrees' recurrence as
 // a chain over all of them takes 45 cycles a step (R/L = 2000: 224 us of a
@@ -136,8 +153,10 @@ __device__ __forceinline__ void next_run(double2 a, double2 b, int e, double& p,
 // c1 (x-1) + c3.
 __global__ void __launch_bounds__(64) k_wave_start(const MieDesc* __restrict__ tabs, int ntab, int mie_units,
                                                    const BlockDesc* __restrict__ desc, int n,
-                                                   char* __restrict__ arena, int* __restrict__ status)
+                                                   char* __restrict__ arena, int* __restrict__ status,
+                                                   int64_t* __restrict__ clock)
 {
+    stage_begins(clock);
     const int lane = threadIdx.x;
     int u = blockIdx.x;
     if (u < ntab * mie_units) {
@@ -274,8 +293,10 @@ __device__ __forceinline__ void degree_rows(const Deg& g, double m, double x, do
 
 // The states at the runs' starts, in place of the matrices that lead to them
 // (what k_wave_norms does by itself where the runs are few).
-__global__ void __launch_bounds__(64) k_wave_prefix(const BlockDesc* __restrict__ desc, char* __restrict__ arena)
+__global__ void __launch_bounds__(64) k_wave_prefix(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
+                                                    int64_t* __restrict__ clock)
 {
+    stage_begins(clock);
     const BlockDesc& d = desc[blockIdx.y];
     if ((int)blockIdx.x >= d.n_waves) return;
     const int nP = d.n_waves * 64, k = blockIdx.x * 64 + threadIdx.x, runs = d.n_below + d.n_segs - 1;
@@ -326,8 +347,9 @@ __global__ void __launch_bounds__(64) k_wave_prefix(const BlockDesc* __restrict_
 // takes that has enough of them.  Both make the same sums.
 template <bool SPLIT>
 __global__ void __launch_bounds__(256) k_wave_norms(const BlockDesc* __restrict__ desc, int n, char* __restrict__ arena,
-                                                    int prefixed)
+                                                    int prefixed, int64_t* __restrict__ clock)
 {
+    if (!prefixed) stage_begins(clock);
     constexpr int NH = SPLIT ? 1 : 2;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int u = SPLIT ? blockIdx.x : 4 * blockIdx.x + wv;
@@ -605,8 +627,10 @@ __global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc
 // own and read back 478 + 124 us, bound by the loads' latency.
 template <int NC>
 __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
-    k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena, const BlockOut* __restrict__ out, int delta_only)
+    k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena, const BlockOut* __restrict__ out, int delta_only,
+           int64_t* __restrict__ clock)
 {
+    stage_begins(clock);
     static_assert(NC == 1 || NC == 4, "columns per workgroup");
     constexpr int NR = NC + BAND_TILES - 1, NS = 8, PITCH = 16 * NS + 16, KS = 32;
     constexpr int NG = NC == 4 ? 1 : 2, NW = 4 * NG;   // chunks per step, wavefronts
@@ -829,9 +853,13 @@ __device__ __forceinline__ double row_d(double x)
 // 39 us; column after column from one end, through LDS, 94, 282 and 55 us.
 // mercator: the LU-mode rule of src/matrix.c:489-505 first (||M||_F² = tr M² =
 // Σ G_ij²; skip = 2: the host returns the two-term series).
+// host: pinned host memory for the results of all blocks, also of those that are
+// not factored here.
 __global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
-                                                   BlockOut* __restrict__ out, int mercator)
+                                                   BlockOut* __restrict__ out, BlockOut* __restrict__ host, int mercator,
+                                                   int64_t* __restrict__ clock)
 {
+    stage_begins(clock);
     constexpr int NTH = 1024, BT = BAND_TILES, COL = BT * 256, MID = BT - 1;
     static_assert(BT == 7, "six diagonals of tiles, dealt to twelve wavefronts");
     __shared__ double S[2][2][COL];
@@ -839,7 +867,14 @@ __global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__
     const BlockDesc& d = desc[b];
     BlockOut& o = out[b];
     const int T = o.tiles;
-    if (o.skip || !o.delta || T <= 0) return;
+    auto result = [&] {   // (by thread 0, which wrote what is new in it)
+        o.t_end = wall_clock64();
+        host[b] = o;
+    };
+    if (o.skip || !o.delta || T <= 0) {
+        if (threadIdx.x == 0) result();
+        return;
+    }
     const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, lk = lane >> 4;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     double* B = at<double>(arena, d.off_band);
@@ -870,7 +905,10 @@ __global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__
             __syncthreads();
             if (tid == 0) {
                 o.frob2 = o.tr2 = f2;
-                if (take) o.skip = 2;
+                if (take) {
+                    o.skip = 2;
+                    result();
+                }
             }
             if (take) return;
         }
@@ -1080,6 +1118,7 @@ __global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__
     if (tid != 0) return;
     for (int w = 1; w < NTH / 64; w++) add(red[2 * w], red[2 * w + 1]);
     o.logdet = ls + lc;
+    result();
 }
 
 // -G dense, column-major (zero outside the band), for the LU's kernels:
@@ -1186,13 +1225,21 @@ using namespace capsd;
 
 extern "C" {
 
-// units: of all blocks together (BlockDesc::unit_*), or more
+// bytes: rounded up to 16, within both buffers
+void capsd_launch_upload(const void* host, void* dev, size_t bytes, hipStream_t s)
+{
+    const int n = (int)((bytes + 15) / 16);
+    hipLaunchKernelGGL(k_upload, dim3((n + 255) / 256), dim3(256), 0, s, (const uint4*)host, (uint4*)dev, n);
+}
+
+// units: of all blocks together (BlockDesc::unit_*), or more; clock: where the time at
+// which the stage begins goes, or null (here and below)
 void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const BlockDesc* desc, char* arena, int nblocks,
-                             int units, int* status, hipStream_t s)
+                             int units, int* status, int64_t* clock, hipStream_t s)
 {
     const int mu = (max_mie + 63) / 64;
     hipLaunchKernelGGL(k_wave_start, dim3(ntab * mu + units), dim3(64), 0, s, (const MieDesc*)tabs, ntab, mu, desc,
-                       nblocks, arena, status);
+                       nblocks, arena, status, clock);
 }
 
 // split, pairs: the units of k_wave_norms' two forms.  Whole runs in one
@@ -1201,14 +1248,15 @@ void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const Bloc
 // max_runs: with more than 8 runs k_wave_prefix pays for its launch (2 runs: 10
 // us with it and 6 without; 222 blocks of 19: 93 and 107; 188: 38 and 142).
 void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, int nblocks, int split, int pairs, int max_runs,
-                             int max_waves, hipStream_t s)
+                             int max_waves, int64_t* clock, hipStream_t s)
 {
     const int prefixed = max_runs > 8;
-    if (prefixed) hipLaunchKernelGGL(k_wave_prefix, dim3(max_waves, nblocks), dim3(64), 0, s, desc, arena);
+    if (prefixed) hipLaunchKernelGGL(k_wave_prefix, dim3(max_waves, nblocks), dim3(64), 0, s, desc, arena, clock);
     if (pairs < 1024)
-        hipLaunchKernelGGL(k_wave_norms<true>, dim3(split), dim3(256), 0, s, desc, nblocks, arena, prefixed);
+        hipLaunchKernelGGL(k_wave_norms<true>, dim3(split), dim3(256), 0, s, desc, nblocks, arena, prefixed, clock);
     else
-        hipLaunchKernelGGL(k_wave_norms<false>, dim3((pairs + 3) / 4), dim3(256), 0, s, desc, nblocks, arena, prefixed);
+        hipLaunchKernelGGL(k_wave_norms<false>, dim3((pairs + 3) / 4), dim3(256), 0, s, desc, nblocks, arena, prefixed,
+                           clock);
 }
 
 void capsd_launch_wave_rows(const BlockDesc* desc, char* arena, int nblocks, int max_wq, hipStream_t s)
@@ -1228,18 +1276,20 @@ void capsd_launch_wave_window(BlockDesc* desc, char* arena, BlockOut* out, const
 // The band of -G, ncol (1 or 4) column tiles per workgroup; max_chunks: the
 // blocks' largest n_chunks
 void capsd_launch_gram(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves,
-                       int max_chunks, int ncol, int delta_only, hipStream_t s)
+                       int max_chunks, int ncol, int delta_only, int64_t* clock, hipStream_t s)
 {
     const int T = max_waves * 8;
     const size_t lds = 2 * (size_t)max_chunks * sizeof(int2);   // two steps per chunk at most
-    if (ncol == 1) hipLaunchKernelGGL(k_gram<1>, dim3(T, nblocks), dim3(512), lds, s, desc, arena, out, delta_only);
+    if (ncol == 1)
+        hipLaunchKernelGGL(k_gram<1>, dim3(T, nblocks), dim3(512), lds, s, desc, arena, out, delta_only, clock);
     else
-        hipLaunchKernelGGL(k_gram<4>, dim3((T + 3) / 4, nblocks), dim3(256), lds, s, desc, arena, out, delta_only);
+        hipLaunchKernelGGL(k_gram<4>, dim3((T + 3) / 4, nblocks), dim3(256), lds, s, desc, arena, out, delta_only, clock);
 }
 
-void capsd_launch_band_ldl(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int mercator, hipStream_t s)
+void capsd_launch_band_ldl(const BlockDesc* desc, char* arena, BlockOut* out, BlockOut* host, int nblocks, int mercator,
+                           int64_t* clock, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_band_ldl, dim3(nblocks), dim3(1024), 0, s, desc, arena, out, mercator);
+    hipLaunchKernelGGL(k_band_ldl, dim3(nblocks), dim3(1024), 0, s, desc, arena, out, host, mercator, clock);
 }
 
 void capsd_launch_band_dense(const BlockDesc* desc, char* arena, const BlockOut* out, int nblocks, int max_waves,

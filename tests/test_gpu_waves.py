@@ -121,3 +121,22 @@ def test_few_tiles(ca, rbyl, ldim):
         at.set_config(0)
     assert np.array_equal(tr, tw) and np.array_equal(fl, fw)
     assert np.max(np.abs(v / w - 1)) < 1e-12
+
+
+def test_results_and_times_from_the_kernels(ca):
+    """Results and stage times are stored by the kernels: batches of one and
+    of many blocks in turn (the buffers grow), factored and not, eager and as
+    graphs, give the same bits, and the stages add up to the whole."""
+    c = make(ca, 40, 240, 1)
+    xs, ms = np.linspace(0.5, 300, 300), np.arange(300) % 60
+    one = [c.logdetD(xs[i], int(ms[i])) for i in (0, 7, 59, 150)]
+    v, _, fl = c.logdetD_batch(xs, ms, info=True)
+    assert {f & 3 for f in fl} == {0, 1}
+    assert one == [v[i] for i in (0, 7, 59, 150)]
+    t = c.last_timing()
+    parts = [t[k] for k in ("mie", "K", "I", "assemble", "lu")]
+    assert min(parts) >= 0 and abs(sum(parts) - t["total"]) < 1e-9 and 0.01 < t["total"] < 100
+    c.set_graph(1)
+    for _ in range(3):
+        assert np.array_equal(c.logdetD_batch(xs, ms), v)
+        assert c.logdetD(xs[7], 7) == v[7]
