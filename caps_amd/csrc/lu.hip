@@ -972,7 +972,9 @@ __device__ __forceinline__ void swap_rows_ipiv(double* __restrict__ Ac, const in
 // broadcast LDS read instead of a vector load per entry).  A panel's
 // interchanges come to a gather of its 64 rows and at most 64 moves from them
 // to rows below, all independent loads, from the lists in PanelSwaps (one
-// exchange after the other: 85 us for 4 matrices of 1200, 45 so).
+// exchange after the other: 85 us for 4 matrices of 1200).  Bound by the latency
+// of its loads, one after the other where they need each other: L11 and the moves 32 a
+// lane at a time, 24 us (L11 one at a time, the moves 16: 39).
 template <int NTH>
 __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restrict__ desc, char* __restrict__ arena,
                                                       const LuSide* __restrict__ side,
@@ -988,7 +990,14 @@ __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restric
     const int cend = min(N, r0 + cs_off + climit);
     const int64_t lda = d.lda;
     const double* P = panel_buf(arena, side[b], lda, pb);
-    for (int idx = threadIdx.x; idx < NB * NB; idx += NTH) sL[idx] = P[(idx % NB) + (int64_t)(idx / NB) * lda];
+    constexpr int IN = NB * NB / NTH < 32 ? NB * NB / NTH : 32;   // loads in flight
+    for (int i0 = threadIdx.x; i0 < NB * NB; i0 += IN * NTH) {
+        double v[IN];
+#pragma unroll
+        for (int i = 0; i < IN; i++) v[i] = P[(i0 + i * NTH) % NB + (int64_t)((i0 + i * NTH) / NB) * lda];
+#pragma unroll
+        for (int i = 0; i < IN; i++) sL[i0 + i * NTH] = v[i];
+    }
     __shared__ int lists[NPANEL][3 * NB], counts[NPANEL];   // of the panels in swaps: PanelSwaps' top, dst, src; n
     for (int q = 0; q < NPANEL; q++)
         if ((swaps >> q) & 1) {
@@ -1016,12 +1025,12 @@ __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restric
                 double z[NB];
 #pragma unroll
                 for (int i = 0; i < NB; i++) z[i] = Ac[rq + top[i]];
-                for (int e0 = 0; e0 < n; e0 += 16) {   // rows below: from the 64
-                    double y[16];
+                for (int e0 = 0; e0 < n; e0 += 32) {   // rows below: from the 64
+                    double y[32];
 #pragma unroll
-                    for (int e = 0; e < 16; e++) y[e] = Ac[rq + src[min(e0 + e, n - 1)]];
+                    for (int e = 0; e < 32; e++) y[e] = Ac[rq + src[min(e0 + e, n - 1)]];
 #pragma unroll
-                    for (int e = 0; e < 16; e++)
+                    for (int e = 0; e < 32; e++)
                         if (e0 + e < n) Ac[rq + dst[e0 + e]] = y[e];
                 }
                 if (q == pb) {
@@ -1038,19 +1047,36 @@ __global__ void __launch_bounds__(NTH) k_lu_swap_trsm(const BlockDesc* __restric
 #pragma unroll
         for (int i = 0; i < NB; i++) x[i] = Ac[r0 + i];
     }
-#pragma unroll
-    for (int i = 0; i < NB; i++) {
-#pragma unroll
-        for (int j = i + 1; j < NB; j++) x[j] -= sL[i * NB + j] * x[i];
-    }
-    // the solved U rows go to the step's row-major U buffer (coalesced:
+    // TB rows per turn of the loop, in registers 0 .. TB - 1 (the rows below move
+    // up): all 64 one after the other are 41 kB of code, which a workgroup runs
+    // through once, waiting for each line of it (4 matrices of 1200: 44 us, 39 so).
+    // The solved U rows go to the step's row-major U buffer (coalesced:
     // lanes are columns), the B operand of every trailing update; nothing
     // reads them from the matrix again (the determinant needs only the
     // diagonal), so they are not written back there, which saved 64 stores
     // per lane that each touched 64 columns
+    constexpr int TB = 8;
     double* Ut = at<double>(arena, side[b].off_ut) + (int64_t)pb * NB * lda + col;
+#pragma unroll 1
+    for (int i0 = 0; i0 < NB; i0 += TB) {
+        const double* L = sL + i0 * (NB + 1);
 #pragma unroll
-    for (int i = 0; i < NB; i++) Ut[i * lda] = x[i];
+        for (int i = 0; i < TB; i++) {
+#pragma unroll
+            for (int j = i + 1; j < TB; j++) x[j] -= L[i * NB + j] * x[i];
+            Ut[(i0 + i) * lda] = x[i];
+        }
+#pragma unroll
+        for (int j0 = TB; j0 < NB; j0 += TB)
+            if (i0 + j0 < NB) {
+#pragma unroll
+                for (int j = j0; j < j0 + TB; j++)
+#pragma unroll
+                    for (int i = 0; i < TB; i++) x[j] -= L[i * NB + j] * x[i];
+            }
+#pragma unroll
+        for (int j = 0; j + TB < NB; j++) x[j] = x[j + TB];
+    }
 }
 
 // Later panels' row interchanges applied to the L rows of earlier panels of
