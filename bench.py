@@ -9,7 +9,7 @@ m of a Matsubara frequency in one launch sequence.  The same step in the
 plain one-block-at-a-time form is timed once beside it.
 
 Prints one JSON line (the driver's contract), with a roofline entry for the
-dominant kernel (HIP events on the library's stream) and a CPU baseline: the
+dominant kernel (times stored by the kernels) and a CPU baseline: the
 CPU oracle on a bounded sample of the workload's blocks on this host's cores,
 with the reference library's own timing on the build container beside it.
 

@@ -294,7 +294,8 @@ int capsx_lu_time(int dim, int n, int reps, int levels, int streams, int xcd, in
 int capsx_lu_logdet_batch_noalloc(double *dA, int dim, int lda, int n, double *d_logdet, void *stream);
 
 /* Extension: per-stage timing of the last batch on this caps object, in
- * milliseconds (HIP events on the library's stream): [0] Mie coefficients and
+ * milliseconds (times that a determinant's kernels store as they begin and
+ * end, otherwise HIP events on the library's stream): [0] Mie coefficients and
  * quadrature nodes, [1] row norms, trace and window, [2] rows of the
  * wave-number factor, [3] matrix, [4] LU, [5] total; of a block's K and I
  * tables [0] prefactors, [1] K, [2] I. */
