@@ -408,14 +408,14 @@ __global__ void __launch_bounds__(256) k_lu_panel_copy(const BlockDesc* __restri
     const int b = blockIdx.z;
     const BlockDesc& d = desc[b];
     const int r = blockIdx.x * 256 + threadIdx.x, np = d.N - k;
-    if (out[b].skip || out[b].delta || r >= np) return;
-    const int64_t lda = d.lda;
     const int j0 = 16 * blockIdx.y, nj = min(16, min(NB, np) - j0);
+    if (out[b].skip || out[b].delta || r >= np || nj <= 0) return;   // (a last panel has fewer columns)
+    const int64_t lda = d.lda;
     const double* A = at<double>(arena, d.off_mat) + k + (k + j0) * lda + row_map(arena, side[b])[r];
     double* P = panel_buf(arena, side[b], lda, pb) + r + j0 * lda;
     double v[16];
 #pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = A[min(j, max(nj - 1, 0)) * lda];
+    for (int j = 0; j < 16; j++) v[j] = A[min(j, nj - 1) * lda];
 #pragma unroll
     for (int j = 0; j < 16; j++)
         if (j < nj) P[j * lda] = v[j];

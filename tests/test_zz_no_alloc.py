@@ -98,3 +98,33 @@ def test_noalloc_lu_matches_allocating_entry():
         for p in bufs:
             hip.L.hipFree(p)
         hip.L.hipStreamDestroy(stream.value)
+
+
+@pytest.mark.parametrize("N,n", [(30, 5), (65, 3), (100, 3), (272, 3), (300, 2), (2000, 3)])
+def test_noalloc_lu_reads_nothing_past_the_matrices(N, n):
+    """Last panels of 1 to 48 columns, the last matrix at the very end of its
+    allocation (a multiple of 2 MiB): the kernels that work on whole panels or
+    tiles take no column or row that the matrix does not have."""
+    import caps_amd
+    f = caps_amd.lib().capsx_lu_logdet_batch_noalloc
+    f.restype = ctypes.c_int
+    f.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    hip = _Hip()
+    mats = _matrices(np.random.default_rng(N), N, n)
+    cm = np.ascontiguousarray(np.transpose(mats, (0, 2, 1)))
+    size = -(-cm.nbytes // (1 << 21)) * (1 << 21)
+    base = hip.malloc(size)
+    dout = hip.to_device(np.full(n, np.nan))
+    stream = ctypes.c_void_p()
+    assert hip.L.hipStreamCreate(ctypes.byref(stream)) == 0
+    try:
+        dA = base + size - cm.nbytes
+        assert hip.L.hipMemcpy(dA, cm.ctypes.data, cm.nbytes, 1) == 0
+        assert f(dA, N, N, n, dout, stream.value) == 0
+        assert hip.L.hipStreamSynchronize(stream.value) == 0
+        got = hip.to_host(dout, n)
+        assert np.max(np.abs(got - np.linalg.slogdet(mats)[1])) < 1e-10 * N
+    finally:
+        hip.L.hipFree(base)
+        hip.L.hipFree(dout)
+        hip.L.hipStreamDestroy(stream.value)
