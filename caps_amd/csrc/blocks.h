@@ -64,10 +64,10 @@ struct BlockDesc {
 // The band of G: tiles on and below the diagonal per column of 16 x 16 tiles
 // (8 nodes each).  Rows of F fall off like e^{-δ²/16} in the distance δ = h
 // times the node distance, and G_ij enters the determinant squared: what lies
-// more than 48 nodes (δ = 24) apart changes it by less than 1e-16 of its
+// more than 48 nodes (δ = 21.6) apart changes it by less than 1e-16 of its
 // value, the tail of x -> 1 of the smallest m included (scanned over R/L
-// 0.1 .. 1000, ξ 1e-3 .. 300, both materials: no difference to the full
-// matrix above 1e-15).
+// 0.1 .. 300, ξ 1e-4 .. 100, ε-1 from 0.1 to perfect reflectors, m up to 20: no
+// difference to the full matrix above the 2e-15 of the eigenvalues compared).
 constexpr int BAND_TILES = 7;
 
 // Constants of one degree of a block's window (see degree() in waves.hip).

@@ -521,11 +521,14 @@ void grid_for(BlockDesc& d)
     d.n_waves = (d.n_nodes + 63) / 64;
 }
 
-// Quadrature grid of the wave-number factor (k_wave_start): the same map with
-// step 0.5, at which the determinants agree with those of a much finer grid
-// to 2e-14 (scanned over R/L 0.1 .. 1000, ξ 1e-3 .. 300, small and large m,
-// both materials; 0.45: 2.0e-14, 0.55: 5.6e-14, 0.6: 1.0e-12), up to where the
-// integrand of the largest degree has fallen by e^{-50} from its peak.
+// Quadrature grid of the wave-number factor (k_wave_start): the map and the
+// step of grid_for, up to where the integrand of the largest degree has fallen
+// by e^{-50} from its peak.  For perfect reflectors and Drude metals the
+// determinants agree with those of a much finer grid to 2.0e-14 (scanned over
+// R/L 0.1 .. 1000, ξ 1e-3 .. 300, small and large m); a step of 0.5 would do
+// there.  Dielectrics decide: for ε-1 = 1 .. 100 and small ξ the singularities
+// of the Fresnel coefficients come near the path (ε-1 = 10, R/L = 0.1, ξ = 0.03:
+// 1.1e-12; 0.5: 2.0e-11; ε-1 = 10.7, R/L = 5, ξ = 0.02: 2.1e-13; 0.5: 5.6e-12).
 void wave_grid_for(BlockDesc& d)
 {
     const double alpha = d.alpha, nu = 2.0 * (d.lmin + d.ldim) - 1;
@@ -542,7 +545,7 @@ void wave_grid_for(BlockDesc& d)
         const double mid = 0.5 * (lo + hi);
         (g(mid) > target ? lo : hi) = mid;
     }
-    d.h = 0.5;
+    d.h = 0.45;
     d.v0 = -19;
     d.A = 0.5 / sqrt(alpha);
     const double s = sqrt(std::max(hi - 1, 60 / alpha)) / d.A;

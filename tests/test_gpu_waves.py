@@ -140,3 +140,22 @@ def test_results_and_times_from_the_kernels(ca):
     for _ in range(3):
         assert np.array_equal(c.logdetD_batch(xs, ms), v)
         assert c.logdetD(xs[7], 7) == v[7]
+
+
+@pytest.mark.parametrize("epsm1,rbyl,ldim,xi,m", [(10, 0.1, 10, 0.03, 0), (10, 0.1, 10, 0.03, 1), (10.7, 1, 20, 0.03, 0),
+                                                  (10.7, 1, 20, 0.03, 1), (10.7, 5, 40, 0.02, 1)])
+def test_grid_dielectrics_small_xi(ca, epsm1, rbyl, ldim, xi, m):
+    """Dielectrics at small ξ, whose Fresnel coefficients have singularities
+    near the integration path, against the oracle's adaptive quadrature (within
+    2e-14 of a grid of step 0.05 on these blocks).  Tolerance: the trapezoidal
+    rule of step 0.45 is off by at most 1.1e-12 here (step 0.5: 5.6e-12 to
+    2.0e-11), the sums and the Mie coefficients add some 1e-13."""
+    import pyoracle as po
+    c = ca.Caps(rbyl * 1e-6, 1e-6, ldim=ldim)
+    w = xi * 299792458.0 / ((rbyl + 1) * 1e-6)
+    wp = (2 * epsm1) ** 0.5 * w   # a Drude metal with γ = ξ: ε - 1 = ωp²/(2 ξ²)
+    c.set_drude(wp * ca.HBAR_EV, w * ca.HBAR_EV)
+    o = po.caps(rbyl * 1e-6, 1e-6, ldim=ldim, drude=(wp, w))
+    v, ref = c.logdetD(xi, m), po.logdetD(o, xi, m)
+    print("relative difference %.1e" % (v / ref - 1))
+    assert abs(v / ref - 1) < 2e-12, (v, ref)
