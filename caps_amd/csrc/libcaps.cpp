@@ -495,14 +495,18 @@ LuCfg lu_config(int maxN, int n)
     return c;
 }
 
+// Step and start of the quadrature grids (CAPS_AMD_QUAD_H, CAPS_AMD_QUAD_V0: a
+// caller's finer or longer grid), read once per batch.
+struct QuadGrid {
+    double h = env_double("CAPS_AMD_QUAD_H", 0.45), v0 = env_double("CAPS_AMD_QUAD_V0", -19.0);
+};
+
 // Quadrature grid of the K integrals of one block (see k_K_partial):
 // x(v) = 1 + A² softplus(v)², A = 0.5/sqrt(α), step h, from v0 to the end of
 // the tail of the largest ν (integrand below e^{-70} of its peak).
-void grid_for(BlockDesc& d)
+void grid_for(BlockDesc& d, const QuadGrid& q)
 {
-    const double alpha = d.alpha;
-    const double h = env_double("CAPS_AMD_QUAD_H", 0.45);
-    const double v0 = env_double("CAPS_AMD_QUAD_V0", -19.0);
+    const double alpha = d.alpha, h = q.h, v0 = q.v0;
     const double A = 0.5 / sqrt(alpha);
     const double nu = d.nu_max + 0.5;
     const double xp = sqrt(1 + (nu / alpha) * (nu / alpha));
@@ -529,7 +533,7 @@ void grid_for(BlockDesc& d)
 // there.  Dielectrics decide: for ε-1 = 1 .. 100 and small ξ the singularities
 // of the Fresnel coefficients come near the path (ε-1 = 10, R/L = 0.1, ξ = 0.03:
 // 1.1e-12; 0.5: 2.0e-11; ε-1 = 10.7, R/L = 5, ξ = 0.02: 2.1e-13; 0.5: 5.6e-12).
-void wave_grid_for(BlockDesc& d)
+void wave_grid_for(BlockDesc& d, const QuadGrid& q)
 {
     const double alpha = d.alpha, nu = 2.0 * (d.lmin + d.ldim) - 1;
     const double xp = hypot(1, nu / alpha);
@@ -545,8 +549,8 @@ void wave_grid_for(BlockDesc& d)
         const double mid = 0.5 * (lo + hi);
         (g(mid) > target ? lo : hi) = mid;
     }
-    d.h = 0.45;
-    d.v0 = -19;
+    d.h = q.h;
+    d.v0 = q.v0;
     d.A = 0.5 / sqrt(alpha);
     const double s = sqrt(std::max(hi - 1, 60 / alpha)) / d.A;
     const double vhi = s > 30 ? s : log(expm1(s));
@@ -561,8 +565,9 @@ enum Job { JOB_LOGDET, JOB_PIVOTED, JOB_MATRIX, JOB_TABLES };
 // The matrix that a determinant is taken of: the band of the Gram matrix
 // (one kernel per block); the Gram matrix dense, for the LU's kernels
 // (pivoted LU, a schedule fixed by capsx_lu_config, per-launch profiling,
-// CAPS_AMD_LU_SYM=0); M itself, dense (caps_M_init, and CHOLESKY, whose
-// shortcut rule looks at the lower triangle of M).
+// CAPS_AMD_LU_SYM=0); M itself, dense (caps_M_init, CHOLESKY, whose
+// shortcut rule looks at the lower triangle of M, and a caller's grid of a
+// finer step than the band of 48 nodes is made for).
 enum Form { FORM_BAND, FORM_GRAM, FORM_M };
 
 struct BatchPlan {
@@ -597,7 +602,8 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
     p.dmode = dmode;
     p.lu_kinds = job == JOB_PIVOTED ? 1 : env_double("CAPS_AMD_LU_SYM", 1) != 0 ? 6 : 2;
     const bool det = job == JOB_LOGDET || job == JOB_PIVOTED;
-    p.form = job == JOB_MATRIX || dmode == 2                                            ? FORM_M
+    const QuadGrid quad;
+    p.form = job == JOB_MATRIX || dmode == 2 || quad.h < 0.45                           ? FORM_M
              : job == JOB_PIVOTED || c->prof || p.lu_kinds != 6 || schedule_fixed() ? FORM_GRAM
                                                                                          : FORM_BAND;
     const size_t budget = arena_budget();
@@ -662,7 +668,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             d.nl = ldim + 2;
             d.nu_max = 2 * (d.lo + d.nl - 1);
             d.nK = d.nu_max - d.mu + 1;
-            grid_for(d);
+            grid_for(d, quad);
             d.off_a0 = take(3 * (int64_t)d.nl * 8);
             d.off_kpart = take((int64_t)d.n_waves * d.nK * sizeof(KPart));
             // K table after a zeroed guard of capsd::K_GUARD entries (k_K_combine):
@@ -672,7 +678,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             d.off_i = take(2 * (int64_t)d.nl * d.nl * 12);
         } else {
             tab.L = std::max(tab.L, d.lmin + ldim - 1);
-            wave_grid_for(d);
+            wave_grid_for(d, quad);
             const int64_t nP = 64 * (int64_t)d.n_waves, nc = d.n_chunks;
             const int mm = std::max(d.m, 1);
             d.n_below = (d.lmin - mm + 63) / 64;
@@ -875,7 +881,7 @@ int enqueue_batch(Ctx* c, const BatchPlan& p, bool events)
     mark(3);
     if (p.form == FORM_M)
         capsd_launch_wave_matrix(c->d_desc, c->arena, c->d_out, n, p.max_ldim, det ? 0 : 1,
-                                 det && !piv && p.lu_kinds == 6, s);
+                                 det && !piv && p.lu_kinds == 6 && p.dmode != 1, s);
     else
         capsd_launch_gram(c->d_desc, c->arena, c->d_out, n, p.max_waves, (p.max_ldim + 15) / 16, p.gram_cols,
                           p.form == FORM_BAND, clock(3), s);
@@ -3674,7 +3680,7 @@ int capsx_block_nodes(caps_t* self, double xi_, int m)
     d.lo = (int)lmin - 1;
     d.nl = self->ldim + 2;
     d.nu_max = 2 * (d.lo + d.nl - 1);
-    grid_for(d);
+    grid_for(d, QuadGrid());
     return d.n_nodes;
 }
 

@@ -159,3 +159,62 @@ def test_grid_dielectrics_small_xi(ca, epsm1, rbyl, ldim, xi, m):
     v, ref = c.logdetD(xi, m), po.logdetD(o, xi, m)
     print("relative difference %.1e" % (v / ref - 1))
     assert abs(v / ref - 1) < 2e-12, (v, ref)
+
+
+@pytest.mark.parametrize("detalg", [None, "LU"])
+def test_grid_of_the_caller(ca, detalg):
+    """CAPS_AMD_QUAD_H and CAPS_AMD_QUAD_V0 reach the determinants.  With step
+    0.2 the trapezoidal rule is exact to rounding, what is left against the
+    oracle are the sums and the Mie coefficients (3e-13; the default step's own
+    error is 6.0e-13 and 1.0e-12 on these blocks).  A grid from v = -4 on leaves
+    out part of the integral near x = 1: other values; one from -25.3 on is the
+    same rule with its nodes shifted, off by the default's error again."""
+    import os
+    import pyoracle as po
+    c = ca.Caps(0.1e-6, 1e-6, ldim=10, detalg=detalg)
+    w = 0.03 * 299792458.0 / 1.1e-6
+    wp = 20 ** 0.5 * w
+    c.set_drude(wp * ca.HBAR_EV, w * ca.HBAR_EV)
+    o = po.caps(0.1e-6, 1e-6, ldim=10, drude=(wp, w), detalg=1 if detalg else 0)
+    ref = np.array([po.logdetD(o, 0.03, m) for m in (0, 1)])
+
+    def with_env(name, value):
+        os.environ[name] = value
+        try:
+            return c.logdetD_batch([0.03, 0.03], [0, 1])
+        finally:
+            os.environ.pop(name)
+    v = c.logdetD_batch([0.03, 0.03], [0, 1])
+    fine = with_env("CAPS_AMD_QUAD_H", "0.2")
+    print("step 0.2: %s" % (fine / ref - 1))
+    assert np.max(np.abs(fine / ref - 1)) < 3e-13
+    assert not np.any(with_env("CAPS_AMD_QUAD_V0", "-4") == v)
+    assert np.max(np.abs(with_env("CAPS_AMD_QUAD_V0", "-25.3") / v - 1)) < 3e-12
+    assert np.array_equal(v, c.logdetD_batch([0.03, 0.03], [0, 1]))
+
+
+def test_fine_grid_matches_default(ca):
+    """A step of 0.1 (whose rows of F are wider than the band) on blocks where
+    the default step is exact to 2e-14: same values to the rounding of an LU of
+    N rows (20 N eps + 1e-12); LU mode with its Mercator rule, and re-run with
+    the pivoted LU."""
+    import os
+    L = ca.lib()
+    for rbyl, ldim, metal, detalg in ((20, 120, 1, None), (50, 251, 0, "LU")):
+        c = make(ca, rbyl, ldim, metal, detalg)
+        ms, xs = list(range(0, 40, 3)), [0.8 * rbyl] * 14
+        v, tr, fl = c.logdetD_batch(xs, ms, info=True)
+        os.environ["CAPS_AMD_QUAD_H"] = "0.1"
+        try:
+            w, tw, fw = c.logdetD_batch(xs, ms, info=True)
+            old = L.capsx_lu_delta_mode(0)
+            try:
+                p, _, _ = c.logdetD_batch(xs, ms, info=True)
+            finally:
+                L.capsx_lu_delta_mode(old)
+        finally:
+            os.environ.pop("CAPS_AMD_QUAD_H")
+        assert np.array_equal(fl, fw) and 0 < np.sum((fl & 3) == 0)
+        assert np.max(np.abs(tw / tr - 1)) < 1e-12
+        tol = 40 * ldim * EPS + 1e-12
+        assert np.max(np.abs(w / v - 1)) < tol and np.max(np.abs(p - v)) < tol * np.abs(v).max()
