@@ -631,7 +631,8 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
     std::vector<Tab> tabs;
     std::vector<MieDesc> mds;
     std::vector<int> tab_of;
-    int64_t strips = 0;
+    int64_t strips = 0, tab_bytes = 0;
+    auto table_bytes = [](int L) { return align256((int64_t)L * 36); };
     for (int b = 0; b < n; b++) {
         const int64_t off0 = off;
         caps_t* self = objs[b];
@@ -657,6 +658,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
             mds.push_back(md);
         }
         Tab& tab = tabs[at.first->second];
+        const int L0 = tab.L;   // 0: this block's own table
         d.epsm1_plate = tab.ep;
         d.epsm1_sphere = tab.es;
         tab_of.push_back(at.first->second);
@@ -702,9 +704,15 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
                 if (det) off = lu_side_layout(c->h_side[b], off, d.N, d.lda);
             }
         }
-        if (b > 0 && (size_t)off > budget) {
+        tab_bytes += table_bytes(tab.L) - table_bytes(L0);
+        if (b > 0 && (size_t)(off + tab_bytes) > budget) {   // without this block and what its table took
             off = off0;
             tab_of.pop_back();
+            tab.L = L0;
+            if (at.second) {
+                tabs.pop_back();
+                mds.pop_back();
+            }
             break;
         }
         if (job != JOB_TABLES) {
@@ -743,7 +751,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
         p.ntab = (int)tabs.size();
         for (int t = 0; t < p.ntab; t++) {
             mds[t].L = tabs[t].L;
-            mds[t].off = tabs[t].off = take((int64_t)tabs[t].L * 36);
+            mds[t].off = tabs[t].off = take(table_bytes(tabs[t].L));
             p.max_mie = std::max(p.max_mie, tabs[t].L);
         }
         // the tables' descriptors right behind the blocks'
@@ -1595,16 +1603,17 @@ static int logdetD_multi_ordered(caps_t* host, caps_t* const* objs, const double
     double tot[6] = {0, 0, 0, 0, 0, 0};
     // CAPS_AMD_PROGRESS=1: one line on stderr per launch sequence
     static const bool progress = env_double("CAPS_AMD_PROGRESS", 0) > 0;
+    // a batch of several launch sequences takes the whole budget at once:
+    // HIP kept a freed arena's memory from the next allocation (device memory
+    // free after growing a 92.6 GB arena to 100 GB: 115 of 309 GB), so an
+    // arena grown between sequences held both
+    auto whole_budget = [&](const BatchPlan& p) { ensure_arena(c, std::max(p.bytes, arena_budget())); };
     for (int b0 = 0; b0 < n;) {
         const double t_seq = progress ? wall_seconds() : 0;
         ensure_blocks(c, n - b0);
         const BatchPlan p = plan_batch_multi(objs + b0, c, xi_ + b0, m + b0, n - b0, JOB_LOGDET, lu_mode);
         const int k = p.n;
-        // a batch of several launch sequences takes the whole budget at once:
-        // HIP kept a freed arena's memory from the next allocation (device memory
-        // free after growing a 92.6 GB arena to 100 GB: 115 of 309 GB), so an
-        // arena grown between sequences held both
-        if (k < n) ensure_arena(c, arena_budget());
+        if (k < n) whole_budget(p);
         run_batch(host, c, p);
         // blocks left unfactored (the delta form ruled out by
         // capsx_lu_delta_mode): run them again with the pivoted LU
@@ -1634,6 +1643,7 @@ static int logdetD_multi_ordered(caps_t* host, caps_t* const* objs, const double
             for (int a0 = 0; a0 < (int)again.size();) {
                 const BatchPlan q = plan_batch_multi(ro.data() + a0, c, rx.data() + a0, rm.data() + a0,
                                                      (int)again.size() - a0, JOB_PIVOTED, lu_mode);
+                if (q.n < (int)again.size()) whole_budget(q);
                 run_batch(host, c, q);
                 for (int j = 0; j < q.n; j++) take(c->h_out[j], again[a0 + j]);
                 for (int i = 0; i < 6; i++) tot[i] += c->timing[i];

@@ -218,3 +218,43 @@ def test_fine_grid_matches_default(ca):
         assert np.max(np.abs(tw / tr - 1)) < 1e-12
         tol = 40 * ldim * EPS + 1e-12
         assert np.max(np.abs(w / v - 1)) < tol and np.max(np.abs(p - v)) < tol * np.abs(v).max()
+
+
+def test_sequences_keep_the_arena_budget(ca, capfd):
+    """A batch of many distinct frequencies and two geometries in launch
+    sequences of a small budget: the arena is allocated once, with the budget
+    (the Mie tables, 36 bytes per degree, object and frequency, are within it;
+    with the pivoted re-run in sequences of its own a second time), and the values are the bits
+    of one sequence.  The re-run with the pivoted LU: the rounding of an LU of N
+    <= 640 rows in other schedules, 640 eps + 1e-12 of the largest value."""
+    import os
+    import re
+    L = ca.lib()
+
+    def run(budget, pivoted):
+        a, b = make(ca, 20, 120, 1), make(ca, 31, 187, 0)
+        n = 40 if pivoted else 300
+        xs, ms = np.linspace(0.3, 9.3, n), np.arange(n) % 5
+        os.environ["CAPS_AMD_PROGRESS"] = "1"
+        if budget:
+            os.environ["CAPS_AMD_ARENA_GB"] = str(budget)
+        old = L.capsx_lu_delta_mode(0 if pivoted else 1)
+        try:
+            v = ca.logdetD_multi([a, b] * (n // 2), xs, ms)
+        finally:
+            L.capsx_lu_delta_mode(old)
+            os.environ.pop("CAPS_AMD_PROGRESS")
+            os.environ.pop("CAPS_AMD_ARENA_GB", None)
+        sizes = [float(x) for x in re.findall(r"capsx: arena ([0-9.]+) GB", capfd.readouterr().err)]
+        return v, a.stats()["batches"], sizes   # (a runs the batch: objs[0])
+
+    for budget, pivoted in ((0.010, False), (0.017, False), (0.040, True)):
+        v, n1, s1 = run(None, pivoted)
+        w, n2, s2 = run(budget, pivoted)
+        print("budget %g: %d sequences, arenas %s GB; without: %d, %s GB" % (budget, n2, s2, n1, s1))
+        assert n1 == 1 + pivoted and n2 >= 4
+        assert len(s2) <= 1 + pivoted and max(s2) <= budget + 1e-9, s2
+        if pivoted:
+            assert np.max(np.abs(w - v)) < (640 * EPS + 1e-12) * np.abs(v).max()
+        else:
+            assert np.array_equal(v, w)
