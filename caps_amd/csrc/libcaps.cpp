@@ -234,6 +234,10 @@ void ctx_free(Ctx* c)
 
 constexpr size_t UP_HEAD = 256;   // the status word's share of d_up
 
+// Blocks of one launch sequence at most: kernels have the block in the grid's y
+// or z, which takes 65535.
+constexpr int MAX_BLOCKS = 65535;
+
 void ensure_blocks(Ctx* c, int n)
 {
     if (n <= c->cap_blocks) return;
@@ -575,6 +579,7 @@ struct BatchPlan {
     // units of the launches over all blocks (BlockDesc::unit_*)
     int u_start = 0, u_split = 0, u_pair = 0, max_runs = 0;
     size_t bytes = 0;
+    bool cut = false;   // by the budget: the next block did not fit
     Job job = JOB_LOGDET;
     Form form = FORM_BAND;
     bool banded() const { return job == JOB_LOGDET && form == FORM_BAND; }
@@ -594,7 +599,7 @@ bool schedule_fixed()
 }
 
 // Descriptors and arena offsets of blocks [0, n), or of the first of them that
-// fit the HBM budget together (p.n, at least one).
+// fit the HBM budget together (p.n, at least one, at most MAX_BLOCKS).
 BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const int* m, int n, Job job, int dmode)
 {
     BatchPlan p;
@@ -633,6 +638,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
     std::vector<int> tab_of;
     int64_t strips = 0, tab_bytes = 0;
     auto table_bytes = [](int L) { return align256((int64_t)L * 36); };
+    n = std::min(n, MAX_BLOCKS);
     for (int b = 0; b < n; b++) {
         const int64_t off0 = off;
         caps_t* self = objs[b];
@@ -713,6 +719,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
                 tabs.pop_back();
                 mds.pop_back();
             }
+            p.cut = true;
             break;
         }
         if (job != JOB_TABLES) {
@@ -1606,11 +1613,14 @@ static int logdetD_multi_ordered(caps_t* host, caps_t* const* objs, const double
     // a batch of several launch sequences takes the whole budget at once:
     // HIP kept a freed arena's memory from the next allocation (device memory
     // free after growing a 92.6 GB arena to 100 GB: 115 of 309 GB), so an
-    // arena grown between sequences held both
-    auto whole_budget = [&](const BatchPlan& p) { ensure_arena(c, std::max(p.bytes, arena_budget())); };
+    // arena grown between sequences held both.  (One of many small blocks, cut
+    // at MAX_BLOCKS, takes what it needs while both would fit easily.)
+    auto whole_budget = [&](const BatchPlan& p) {
+        if (p.cut || p.bytes > arena_budget() / 4) ensure_arena(c, std::max(p.bytes, arena_budget()));
+    };
     for (int b0 = 0; b0 < n;) {
         const double t_seq = progress ? wall_seconds() : 0;
-        ensure_blocks(c, n - b0);
+        ensure_blocks(c, std::min(n - b0, MAX_BLOCKS));
         const BatchPlan p = plan_batch_multi(objs + b0, c, xi_ + b0, m + b0, n - b0, JOB_LOGDET, lu_mode);
         const int k = p.n;
         if (k < n) whole_budget(p);

@@ -258,3 +258,17 @@ def test_sequences_keep_the_arena_budget(ca, capfd):
             assert np.max(np.abs(w - v)) < (640 * EPS + 1e-12) * np.abs(v).max()
         else:
             assert np.array_equal(v, w)
+
+
+def test_more_blocks_than_a_grid_takes(ca):
+    """66000 blocks: kernels have the block in the grid's y or z (at most 65535),
+    so they run in two launch sequences, with the bits of smaller batches."""
+    c = ca.Caps(0.2e-6, 1e-6, ldim=3)
+    n = 66000
+    xs, ms = 0.2 + 1e-5 * (np.arange(n) // 3), np.arange(n) % 3
+    v = c.logdetD_batch(xs, ms)
+    assert c.stats(reset=True)["batches"] == 2
+    # (the library runs a batch's blocks in order of m: the last of m = 2 are the second sequence's)
+    for s in (slice(0, 300), slice(32000, 32300), slice(n - 300, n)):
+        assert np.array_equal(v[s], c.logdetD_batch(xs[s], ms[s]))
+    assert np.all(v < 0)
