@@ -1629,7 +1629,9 @@ static void launch_panel(int rows, const BlockDesc* desc, char* arena, const LuS
     }
 #undef PANEL
 #undef PANELC
-    if (rows <= grid_panel_rows)
+    // (a last panel's copy nobody reads; without it matrices of up to 64 rows
+    // have no kernel with the matrix in the grid's z, which takes 65535)
+    if (rows > NB && rows <= grid_panel_rows)
         hipLaunchKernelGGL(k_lu_panel_copy, dim3((rows + 255) / 256, NB / 16, nb), dim3(256), 0, s, desc, arena, side,
                            out, k, pb);
 }

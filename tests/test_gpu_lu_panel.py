@@ -65,3 +65,11 @@ def test_equal_candidates_and_degenerate_columns(ca):
     assert abs(v[0] - 128 * np.log(256)) < 100 * 256 * EPS
     assert not np.isfinite(v[1])   # a pivot of exactly 0
     assert np.isnan(v[2])
+
+
+def test_more_matrices_than_a_grid_takes(ca):
+    """66000 matrices of one panel: the grid's y and z take 65535, its x more.
+    (Some of so many are nearly singular: each by its own condition.)"""
+    A = mats(66000, 3, 11)
+    v = ca.lu_logdet_batch(A)
+    assert np.all(np.abs(v - np.linalg.slogdet(A)[1]) < 100 * 3 * EPS * np.linalg.cond(A))
