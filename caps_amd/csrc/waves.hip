@@ -811,17 +811,54 @@ __device__ __forceinline__ double column_next(double (&x)[16], double (&a)[16], 
     return d;
 }
 
-// ... for a of columns J .. 15 and x of those that column_next left
-template <int T, int J>
+// ... for a of columns T + 2 .. 15 and x of those that column_next left, from
+// column J on; up to four columns per statement (and the two whose x is done), each
+// with the wait states before its first read: what the compiler may have moved
+// to an operand's register just before it does not see the DPP.
+#define COLUMN(x, a) FMAC_ROW(x, a, lx) FMAC_ROW(a, a, la)
+template <int T, int J = T < 13 ? T + 4 : T + 2>
 __device__ __forceinline__ void columns_rest(double (&x)[16], double (&a)[16], double lx, double la)
 {
-    if constexpr (J < 16) {
-        if constexpr (T >= 13 || J > T + 3)
-            asm volatile(FMAC_ROW(0, 1, lx) : "+v"(x[J]) : "v"(a[J]), [lx] "v"(lx), [t] "n"(T));
-        asm volatile(FMAC_ROW(0, 0, la) : "+v"(a[J]) : [la] "v"(la), [t] "n"(T));
-        columns_rest<T, J + 1>(x, a, lx, la);
+#define LANES [lx] "v"(lx), [la] "v"(la), [t] "n"(T)
+    constexpr int N = J < 16 ? (16 - J < 4 ? 16 - J : 4) : 0;
+    if constexpr (T < 13 && J == T + 4) {   // a of T + 2 and T + 3 with it
+#define FIRST "s_nop 1\n" FMAC_ROW(0, 0, la) FMAC_ROW(1, 1, la)
+#define OPS "+v"(a[T + 2]), "+v"(a[T + 3])
+        if constexpr (N == 4)
+            asm volatile(FIRST COLUMN(2, 6) COLUMN(3, 7) COLUMN(4, 8) COLUMN(5, 9)
+                         : OPS, "+v"(x[J]), "+v"(x[J + 1]), "+v"(x[J + 2]), "+v"(x[J + 3]), "+v"(a[J]),
+                           "+v"(a[J + 1]), "+v"(a[J + 2]), "+v"(a[J + 3]) : LANES);
+        else if constexpr (N == 3)
+            asm volatile(FIRST COLUMN(2, 5) COLUMN(3, 6) COLUMN(4, 7)
+                         : OPS, "+v"(x[J]), "+v"(x[J + 1]), "+v"(x[J + 2]), "+v"(a[J]), "+v"(a[J + 1]),
+                           "+v"(a[J + 2]) : LANES);
+        else if constexpr (N == 2)
+            asm volatile(FIRST COLUMN(2, 4) COLUMN(3, 5)
+                         : OPS, "+v"(x[J]), "+v"(x[J + 1]), "+v"(a[J]), "+v"(a[J + 1]) : LANES);
+        else if constexpr (N == 1)
+            asm volatile(FIRST COLUMN(2, 3) : OPS, "+v"(x[J]), "+v"(a[J]) : LANES);
+        else
+            asm volatile(FIRST : OPS : LANES);
+#undef FIRST
+#undef OPS
+    } else if constexpr (N == 4) {
+        asm volatile("s_nop 1\n" COLUMN(0, 4) COLUMN(1, 5) COLUMN(2, 6) COLUMN(3, 7)
+                     : "+v"(x[J]), "+v"(x[J + 1]), "+v"(x[J + 2]), "+v"(x[J + 3]), "+v"(a[J]), "+v"(a[J + 1]),
+                       "+v"(a[J + 2]), "+v"(a[J + 3]) : LANES);
+    } else if constexpr (N == 3) {
+        asm volatile("s_nop 1\n" COLUMN(0, 3) COLUMN(1, 4) COLUMN(2, 5)
+                     : "+v"(x[J]), "+v"(x[J + 1]), "+v"(x[J + 2]), "+v"(a[J]), "+v"(a[J + 1]), "+v"(a[J + 2])
+                     : LANES);
+    } else if constexpr (N == 2) {
+        asm volatile("s_nop 1\n" COLUMN(0, 2) COLUMN(1, 3)
+                     : "+v"(x[J]), "+v"(x[J + 1]), "+v"(a[J]), "+v"(a[J + 1]) : LANES);
+    } else if constexpr (N == 1) {
+        asm volatile("s_nop 1\n" COLUMN(0, 1) : "+v"(x[J]), "+v"(a[J]) : LANES);
     }
+#undef LANES
+    if constexpr (J + N < 16) columns_rest<T, J + N>(x, a, lx, la);
 }
+#undef COLUMN
 #undef FMAC_ROW
 #undef MOV_ROW
 
@@ -950,7 +987,7 @@ __global__ void __launch_bounds__(1024) k_band_ldl(const BlockDesc* __restrict__
             if constexpr (t < 15) {
                 const double la = a[t] * n;
                 dt = column_next<t>(x, a, x[t], la);
-                columns_rest<t, t + 2>(x, a, x[t], la);
+                columns_rest<t>(x, a, x[t], la);
             }
         });
         if (4 * part + lk < nb) {
