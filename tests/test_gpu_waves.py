@@ -272,3 +272,42 @@ def test_more_blocks_than_a_grid_takes(ca):
     for s in (slice(0, 300), slice(32000, 32300), slice(n - 300, n)):
         assert np.array_equal(v[s], c.logdetD_batch(xs[s], ms[s]))
     assert np.all(v < 0)
+
+
+def test_every_small_number_of_tile_columns(ca):
+    """k_band_ldl against the dense Gram matrix with the number of tile columns
+    looked at (from the flops that the statistics count for a band): 1 to 6,
+    where there is only the middle, 7, where one half has a column, and odd and
+    even numbers above.  Fewer than 6 come from coarse grids of the same
+    blocks; either side has the same G.  D <= 260 rows: 1e-12."""
+    import os
+    from caps_amd import autotune as at
+
+    def flops(T):
+        N, w = 16.0 * T, min(16.0 * T, 96.0)
+        return (N - w) * w * (w + 2) + w ** 3 / 3 + w * w / 2 - 5 * w / 6
+    number = {round(flops(T)): T for T in range(1, 30)}
+    seen = set()
+    try:
+        for h in ("0.45", "0.9", "1.5", "2.5", "6"):
+            os.environ["CAPS_AMD_QUAD_H"] = h
+            for rbyl, ldim in ((1, 12), (5, 40), (20, 120)):
+                c = make(ca, rbyl, ldim, 1)
+                ms = list(range(7))
+                v = []
+                for m in ms:
+                    c.stats(reset=True)
+                    v.append(c.logdetD(0.4, m))
+                    s = c.stats()
+                    assert s["blocks_factored"] == 1
+                    seen.add(number[round(s["lu_flops"])])
+                try:
+                    at.set_config(1, 1, 0, 128)
+                    w = c.logdetD_batch([0.4] * 7, ms)
+                finally:
+                    at.set_config(0)
+                assert np.max(np.abs(np.array(v) / w - 1)) < 1e-12, (h, rbyl)
+    finally:
+        os.environ.pop("CAPS_AMD_QUAD_H")
+    print("tile columns:", sorted(seen))
+    assert seen >= set(range(1, 15))
