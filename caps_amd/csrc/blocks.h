@@ -16,7 +16,6 @@ struct BlockDesc {
     double xi_;          // ξ(L+R)/c
     double alpha;        // 2 ξ(L+R)/c
     double epsm1_plate;  // ε(iξ)-1 of the plate (+inf: perfect reflector)
-    double epsm1_sphere; // ε(iξ)-1 of the sphere
     double LbyR;
     int m, lmin, ldim;      // window l in [lmin, lmin+ldim)
     int N;                  // dimension of the matrix to factor (k_wave_window

@@ -628,7 +628,7 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
         size_t operator()(const Key& k) const { return std::hash<void*>()(k.obj) * 31 + std::hash<double>()(k.xi); }
     };
     struct Tab {
-        double ep, es;
+        double ep;
         int L;
         int64_t off;
     };
@@ -655,18 +655,17 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
         d.ldim = ldim;
         const auto at = index.emplace(Key{self, xi_[b]}, (int)tabs.size());
         if (at.second) {
-            tabs.push_back({caps_epsilonm1_plate(self, xi_[b]), caps_epsilonm1_sphere(self, xi_[b]), 0, 0});
+            tabs.push_back({caps_epsilonm1_plate(self, xi_[b]), 0, 0});
             MieDesc md;
             memset(&md, 0, sizeof(md));
             md.xi_ = xi_[b];
             md.LbyR = self->LbyR;
-            md.epsm1 = tabs.back().es;
+            md.epsm1 = caps_epsilonm1_sphere(self, xi_[b]);
             mds.push_back(md);
         }
         Tab& tab = tabs[at.first->second];
         const int L0 = tab.L;   // 0: this block's own table
         d.epsm1_plate = tab.ep;
-        d.epsm1_sphere = tab.es;
         tab_of.push_back(at.first->second);
         d.n_chunks = (ldim + 15) / 16;
         if (job == JOB_TABLES) {

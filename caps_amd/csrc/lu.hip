@@ -54,9 +54,8 @@ constexpr int NB = 64;       // panel width
 template <typename T>
 __device__ __forceinline__ T* at(char* base, int64_t off) { return reinterpret_cast<T*>(base + off); }
 
-// Side buffers of the LU of one block (inside the block's arena slice):
-//   off_piv:              N ints (unused by the logdet; kept for the layout)
-// and, appended by the host after the matrix:
+// Side buffers of the LU of one block (inside the block's arena slice, after
+// the matrix):
 struct LuSide {
     int64_t off_panel;   // NPANEL x lda x NB doubles: the factored panels of a
                          // step (panel q at column k + q NB), rows relative to

@@ -59,16 +59,6 @@ __device__ __forceinline__ double wave_sum(double v)
     return (lane_d(v, 0) + lane_d(v, 16)) + (lane_d(v, 32) + lane_d(v, 48));
 }
 
-__device__ __forceinline__ int wave_max_int(int v)
-{
-    v = max(v, dpp_i<DPP_QUAD_X1>(v));
-    v = max(v, dpp_i<DPP_QUAD_X2>(v));
-    v = max(v, dpp_i<DPP_HALF_MIRROR>(v));
-    v = max(v, dpp_i<DPP_MIRROR>(v));
-    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
-}
-
 // Kahan sum of x[0..n) in index order (the recurrence of a single thread
 // running through the array), by a whole wavefront: 64 consecutive entries
 // per load (the next chunk loaded while this one is summed), each lane

@@ -51,14 +51,6 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // Exponent of what is zero whatever it is added to: 2^NO_EXP 2^E = 0.
 constexpr int NO_EXP = -(1 << 28);
 
-// x^(-1) from the hardware estimate and two Newton steps (normal x).
-__device__ __forceinline__ double rcp_nr(double x)
-{
-    double r = __builtin_amdgcn_rcp(x);
-    r = fma(fma(-x, r, 1.0), r, r);
-    return fma(fma(-x, r, 1.0), r, r);
-}
-
 // One step of S_l = √((l-m)!/(l+m)!) P_l^m upward in the degree (DLMF
 // 14.10.3), c1 = (2l+1)/√((l+1)²-m²), c2 = √(l²-m²)/√((l+1)²-m²).
 __device__ __forceinline__ void degree_step(double c1, double c2, double x, double& p, double& pp)
