@@ -210,7 +210,7 @@ def large_aspect(ca):
     xs = [r["xi_"] for r in rows]
     ms = [r["m"] for r in rows]
     t0 = time.perf_counter()
-    c.logdetD_batch(xs, ms)          # first call: the object's HBM arena (~66 GB) is allocated
+    c.logdetD_batch(xs, ms)          # first call: the object's HBM arena is allocated
     dt_first = time.perf_counter() - t0
     c.reset_stats()
     t0 = time.perf_counter()
@@ -284,7 +284,7 @@ def pfa_rule_error(M):
 
 def large_aspect_energy(ca, out, budget):
     """The T = 0 free energy of the large-aspect configuration (perfect
-    reflectors, R/L = 2000, ldim = 12000, blocks up to 24000 x 24000),
+    reflectors, R/L = 2000, ldim = 12000, matrices of up to 24000 x 24000),
     surrogate-planned, one quadrature node per batch, resumed from and
     appended to the output file `out`; stops after `budget` seconds (F is
     then NaN and a later run continues).  When complete: the rule's levels,

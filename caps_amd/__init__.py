@@ -202,14 +202,18 @@ class Caps:
         return out
 
     def last_timing(self):
+        """Stage times of the last batch in ms (caps_last_timing).  Of
+        determinants: "mie" Mie coefficients and quadrature nodes, "K" row norms,
+        trace and window, "I" rows of the wave-number factor (where M itself is formed),
+        "assemble" the band of the Gram matrix, "lu" its factorization; of a
+        block's K and I tables as the names say."""
         t = np.zeros(6)
         lib().caps_last_timing(self.ptr, _dptr(t))
         return dict(zip(["mie", "K", "I", "assemble", "lu", "total"], t))
 
     def stats(self, reset=False):
-        """Accumulated stage times and work counters of this object's batches
-        (the Mie kernel runs beside the K quadrature: "K" is the time the K
-        stage adds after the Mie kernel ends)."""
+        """Accumulated stage times (keys as in last_timing) and work counters
+        of this object's batches."""
         a = np.zeros(16)
         lib().capsx_stats(self.ptr, _dptr(a))
         if reset:

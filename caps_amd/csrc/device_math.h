@@ -145,8 +145,8 @@ __device__ inline Uniform uniform(double nu, double x)
 // there (0.6/w^6, w >= 40) times the product of the r_j^-2, at least
 // e^{-(l0² - l²)/x}, to be below 1e-16: at most 54 steps, where the continued
 // fraction took up to √(40 x) steps of three divisions (x = nχ of a metal is some 10^4:
-// 252 us for the coefficients of one ξ at R/L = 200; now all of
-// k_wave_start, whose node chains run beside them, takes 27 us).
+// 252 us for the coefficients of one ξ at R/L = 200; all of k_wave_start,
+// whose runs of degrees go beside them, takes 14 us).
 __device__ inline double ratio_half(int l, double x)
 {
     int l0 = l;

@@ -3,9 +3,9 @@
 // One device context per caps_t (stream, events, a growable HBM arena,
 // pinned staging buffers), created on the first GPU call.  A batch of
 // (ξ, m) blocks is laid out in the arena (BlockDesc offsets), the pipeline
-// Mie and nodes -> row norms -> trace and window -> rows -> Gram matrix -> LU
-// runs asynchronously on the context's stream, and only the per-block scalars
-// come back.  The
+// Mie and nodes -> row norms -> trace and window -> band of the Gram matrix ->
+// LDLᵀ (waves.hip; other forms of the matrix: enum Form) runs asynchronously on
+// the context's stream, and only the per-block scalars come back.  The
 // determinant shortcuts of the reference (src/matrix.c:78-82, 144-145,
 // 494-505) are applied to those scalars on the host.
 #include <dlfcn.h>
@@ -750,8 +750,8 @@ BatchPlan plan_batch_multi(caps_t* const* objs, Ctx* c, const double* xi_, const
     // four columns per workgroup make 1.8 times as many rows as the band has,
     // one column seven times in four times as many workgroups, which is faster
     // as long as strips of four would be fewer than CUs (R/L = 200, four columns
-    // and one: 1 block 67 and 29 us, 32 blocks 73 and 79, 40 blocks 99 and 96,
-    // 64 blocks 111 and 152)
+    // and one: 1 block 75 and 28 us, 32 blocks 104 and 77, 40 blocks 102 and 88,
+    // 64 blocks 111 and 122)
     if (strips < 256) p.gram_cols = 1;
     if (job != JOB_TABLES) {
         p.ntab = (int)tabs.size();
@@ -1547,13 +1547,12 @@ int capsx_logdetD_multi_info(caps_t* const* objs, const double* xi_, const int* 
                              int* flags)
 {
     if (n <= 0) return 0;
-    // the blocks of one caps object and m (whose I tables share the a_q,
-    // k_I) are run next to each other, so that they fall into one part of
-    // the batch and into full groups; larger blocks first (the LU's stream
-    // groups are contiguous runs of blocks, balanced by cost): ldim
-    // descending, then objects in the order of their first block, then m,
-    // then the input order.  The batch runs on objs[0]'s context (device
-    // buffers, statistics, graph setting) either way.
+    // larger blocks first, ldim descending: the LU's stream groups are
+    // contiguous runs of blocks, balanced by cost, and the longest band
+    // factorizations start first; then objects in the order of their first
+    // block, m, and the input order, so that alike batches are laid out alike.
+    // The batch runs on objs[0]'s context (device buffers, statistics, graph
+    // setting) either way.
     std::vector<int> ord(n), first(n);
     {
         std::unordered_map<caps_t*, int> seen;
@@ -3426,10 +3425,10 @@ int capsx_block_tables(caps_t* self, double xi_, int m, int* mu, int* nK, double
 // ---- the k-integrals of one block: src/include/integration.h:13-23 --------
 // The reference evaluates K_ν and I_{l1 l2} on demand by quadrature and caches
 // them; here caps_integrate_init computes the block's whole K and I tables on
-// the device (the tables caps_logdetD builds: ν from 2m, or 2 for m = 0, up
-// to 2(lmin + ldim) + 1, and l1, l2 over the block's ℓ-window with one more
-// on either side), and the functions read them.  epsrel is accepted and
-// unused (the device quadrature has a fixed accuracy, 1e-11 relative).
+// the device (ν from 2m, or 2 for m = 0, up to 2(lmin + ldim) + 1, and l1, l2
+// over the block's ℓ-window with one more on either side), and the functions
+// read them.  epsrel is accepted and unused (the device quadrature has a fixed
+// accuracy, 1e-11 relative).
 // Values outside the tables abort with a message.
 
 // Reference: src/integration.c:695-731 (NULL for xi_ < 0, m < 0 or
@@ -3575,9 +3574,10 @@ int capsx_M_copy(caps_M_t* self, double* out)
 }
 
 // Extension: accumulated statistics since the last reset: out[0..5] stage
-// milliseconds (Mie, K, I, assembly, LU, total), out[6] blocks, out[7]
-// blocks factored, out[8] algorithmic LU flops Σ(2/3 N³ - 1/2 N² + 5/6 N),
-// out[9] batches, out[10] (l1 >= l2, polarization) I integrals.
+// milliseconds (caps_last_timing), out[6] blocks, out[7]
+// blocks factored, out[8] flops of their factorizations (run_batch: band, dense
+// LDLᵀ or LU), out[9] batches, out[10] (l1 >= l2, polarization) I integrals of
+// tables.
 // With capsx_profile on: out[11] milliseconds in the LU's trailing-update
 // kernel k_lu_gemm_dma (HIP events around each launch), out[12] its
 // algorithmic flops (2 rows cols depth per updated region, over factored

@@ -748,7 +748,7 @@ void capsd_launch_fill_xi0(const BlockDesc* desc, char* arena, int64_t off_tab, 
     hipLaunchKernelGGL(k_fill_xi0, dim3((n + 63) / 64, (n + 3) / 4), dim3(256), 0, s, desc, arena, off_tab);
 }
 
-// Column dominance of the blocks' 1 - M (after their assembly): the delta
+// Column dominance of 1 - M (a caller's matrix, the ξ = 0 blocks): the delta
 // flags, and the unit diagonal written back where a block is not dominant.
 void capsd_launch_dominance(const BlockDesc* desc, char* arena, BlockOut* out, int nblocks, int maxN, int allow,
                             hipStream_t s)

@@ -15,15 +15,17 @@
 // 2 ldim.  A row of F is a ridge of a few standard deviations around the
 // degree whose saddle point is the node, so rows of distant nodes do not
 // overlap: G is banded, and each of its tiles needs a fraction of the degrees.
-// R/L = 200, ldim = 1200: 2400 rows become about 400 with a half-bandwidth
-// of 96; R/L = 2000, ldim = 12000: 24000 become about 1300.
+// R/L = 200, ldim = 1200: 2400 rows become about 460 with a half-bandwidth
+// of 96; R/L = 2000, ldim = 12000: 24000 become about 1400.
 //
 // Kernels (blockIdx.y, or .x of the last, selects the block):
 //   k_upload       the descriptors;
 //   k_wave_start   the Mie coefficients of each (object, ξ), and beside them
-//                  the nodes with the degree recurrence of P_l^m over all l,
-//                  whose state is kept at the start of every 16 degrees;
-//   k_wave_norms   the squared norms of F's rows per 16 degrees;
+//                  the nodes and, per run of 64 degrees, the matrix of the
+//                  recurrence of P_l^m in l;
+//   k_wave_prefix  the states at the runs' starts (where the runs are many);
+//   k_wave_norms   the states every 8 degrees and the squared norms of F's rows
+//                  per 16;
 //   k_wave_window  trace, trace shortcut, the nodes that matter;
 //   k_gram         the band of -G on FP64 MFMA, F's rows made on the spot;
 //   k_band_ldl     log det(1 - G): banded LDLᵀ, one workgroup per block;
@@ -117,9 +119,11 @@ __device__ __forceinline__ void next_run(double2 a, double2 b, int e, double& p,
 }
 
 // A batch's descriptors from pinned host memory.  A batch of one block is some
-// 80 us of kernels; a copy command before them, one for the results behind them (now
-// stores of k_band_ldl to pinned memory) and a timed event between every two stages
-// (now stores of the time by their first workgroups) took another 27 us (116, now 89; of an energy at T = 0, five batches: 2.20 ms, now 1.93).
+// 80 us of kernels; a copy command before them, one for the results behind them
+// (stores of k_band_ldl to pinned memory instead) and a timed event between every
+// two stages (stores of the time by their first workgroups instead) took another
+// 27 us (116 and 89; an energy at T = 0, five batches: 2.20 and 1.93 ms; measured at
+// a step of 0.5 of the grid, 91 us and 2.03 ms at the present 0.45).
 __global__ void __launch_bounds__(256) k_upload(const uint4* __restrict__ host, uint4* __restrict__ dev, int n)
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -134,8 +138,8 @@ __device__ __forceinline__ void stage_begins(int64_t* clock)
 
 // The first ntab mie_units workgroups: Mie coefficients, one lane per l.  Then
 // per block, 64 nodes per wavefront, one lane each: the degrees' recurrence as
-// a chain over all of them takes 45 cycles a step (R/L = 2000: 224 us of a
-// block's 620; 14 us and k_wave_prefix's 16 so).  Instead each run of 64
+// a chain over all of them takes 45 cycles a step (R/L = 2000: 224 us; 14 us
+// and k_wave_prefix's 16 so).  Instead each run of 64
 // degrees, from d.n_below runs below the window on (the first one shorter),
 // gives the 2 x 2 matrix that takes the state at its start to the next run's,
 // and k_wave_prefix or k_wave_norms multiply them.
@@ -497,10 +501,11 @@ __global__ void __launch_bounds__(256) k_wave_rows(const BlockDesc* __restrict__
 // the trace (together the others change the determinant by less than a few
 // 1e-17 of it; R/L = 20 .. 2000: 10-60 % of the nodes of large m).  dense:
 // the matrix dimension for the LU's kernels goes to desc[b].N.
-// NT: 1024 threads, one quarter of the runs each, or for batches that fill the GPU
-// 256 (block of R/L = 2000: 118 us with 256 threads over its chunks of 16
-// degrees, 28 so; 256 blocks of R/L = 100: 32 us with 1024, 16 with 256; below
-// that many 1024 are as fast or faster).
+// NT: 1024 threads, one quarter of the runs each (block of R/L = 2000: 118 us with
+// 256 threads over its chunks of 16 degrees, 29 so), or 256 for batches of many
+// blocks: norms and window of 4000 blocks of R/L = 20 158 us with 1024 and 118
+// with 256, of 1000 46 and 40, of 1168 of R/L = 200 400 and 394; of 300 123 and
+// 133, of 512 of R/L = 100 100 and 104.
 template <int NT>
 __global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc, char* __restrict__ arena,
                                                     BlockOut* __restrict__ out, const int* __restrict__ status,
@@ -599,24 +604,24 @@ __global__ void __launch_bounds__(NT) k_wave_window(BlockDesc* __restrict__ desc
 // makes degrees 4 w .. 4 w + 3; then the pairs are multiplied.  (Making the next
 // chunk in four more wavefronts beside the products gains nothing: FP64
 // instructions and FP64 MFMA do not overlap.  Bound by the two together:
-// 99 us without the products, 223 without the rows.)
+// at a grid of step 0.5 99 of 271 us without the products, 223 without the rows.)
 // A row's ridge covers a few chunks: a pair of tiles is multiplied over a
 // chunk only if the product of their largest chunk norms is at least 2^-60
 // tr (by Cauchy-Schwarz what is left out is smaller, below the last bit of
-// the trace; R/L = 200, NC = 4: 25 of 75 chunks per strip, 12 of 28 pairs).
+// the trace; R/L = 200, NC = 4: 24 of 75 chunks per strip, 12 of 28 pairs).
 // The pairs that count in a chunk lie next to each other, so NC = 4 deals them
 // out along the diagonals: wavefront w has tile j + r of column j = (w + r) % 4, for r = 0
 // .. 6; the busiest one then has 3.4 on average of 2.9 (whole columns: 4.8).
 // The three pairs with the strip's ninth and tenth tile are a step of their
 // own over tiles 2 .. 9, where they count at all.
 // NC = 1 for batches that would leave CUs idle: two chunks per step in twice
-// the wavefronts, a pair each (one block of R/L = 200: 27 us; 38 a chunk at a
-// time, before degrees lost their exponents).
+// the wavefronts, a pair each (one block of R/L = 200: 28 us).
 // An element sums the same products in the same order for either NC, so its
 // bits do not depend on the batch.
-// 222 blocks of R/L = 200: 271 us (309 with an exponent and a power of two per
-// degree and the states every 16 degrees); with F's rows stored by a kernel of their
-// own and read back 478 + 124 us, bound by the loads' latency.
+// 222 blocks of R/L = 200: 271 to 293 us.  (At a step of 0.5, a tenth fewer
+// nodes, 245 to 271, and 309 with an exponent and a power of two per degree and the
+// states every 16 degrees, 478 + 124 with F's rows stored by a kernel of their own
+// and read back, bound by the loads' latency.)
 template <int NC>
 __global__ void __launch_bounds__(NC == 4 ? 256 : 512, NC == 4 ? 3 : 2)
     k_gram(const BlockDesc* __restrict__ desc, char* __restrict__ arena, const BlockOut* __restrict__ out, int delta_only,
@@ -878,8 +883,9 @@ __device__ __forceinline__ double row_d(double x)
 //    a wavefront has one diagonal of tiles, and only the column in work and
 //    the next one are in LDS.
 // The pivots' FMAs and the MFMAs share the SIMDs' FP64 units, 1900 and 2800
-// cycles of the 7200 that a step takes.  26, 79 and 15 tile columns: 55, 136 and
-// 39 us; column after column from one end, through LDS, 94, 282 and 55 us.
+// cycles of the 7200 that a step takes.  16, 29 and 89 tile columns: 40, 62 and
+// 153 us; 15, 26 and 79: 39, 55 and 136 us, and column after column from one end,
+// through LDS, 55, 94 and 282 us.
 // mercator: the LU-mode rule of src/matrix.c:489-505 first (||M||_F² = tr M² =
 // Σ G_ij²; skip = 2: the host returns the two-term series).
 // host: pinned host memory for the results of all blocks, also of those that are
@@ -1273,9 +1279,10 @@ void capsd_launch_wave_start(const void* tabs, int ntab, int max_mie, const Bloc
 
 // split, pairs: the units of k_wave_norms' two forms.  Whole runs in one
 // wavefront need one of them per SIMD (16 blocks of R/L = 200, norms and
-// window: 30 us whole and 29 us split; 8: 29 and 23; 64: 49 and 61).
-// max_runs: with more than 8 runs k_wave_prefix pays for its launch (2 runs: 10
-// us with it and 6 without; 222 blocks of 19: 93 and 107; 188: 38 and 142).
+// window: 33 us whole and 30 split; 8: 30 and 26; 64: 47 and 51).
+// max_runs: with more than 8 runs k_wave_prefix pays for its launch (norms and
+// window, 2 runs: 16 us with it and 14 without; 222 blocks of 19: 104 and 116;
+// 188: 62 and 172).
 void capsd_launch_wave_norms(const BlockDesc* desc, char* arena, int nblocks, int split, int pairs, int max_runs,
                              int max_waves, int64_t* clock, hipStream_t s)
 {

@@ -269,9 +269,9 @@ int capsx_lu_grid_panel_rows(int rows);
  * gemm_kernel = the 128 x 128 trailing update (2, the default: operand
  * stages moved straight into LDS, 8 deep, three workgroups per CU; 1: 16
  * deep, two per CU; 0: stages through registers), panel_set (1, the
- * default: leaves of 8 columns; 0: leaves of 4), narrow_tiles (1, the
- * default: 128 x 64 and 64 x 128 tiles for regions one panel wide or high;
- * 0: 128 x 128 for all).  All give bit-identical factors.  Same as the
+ * default: leaves of 16 columns up to 2048 rows, then 8; 0: leaves of 4),
+ * narrow_tiles (1, the default: 128 x 64 and 64 x 128 tiles for regions one
+ * panel wide or high; 0: 128 x 128 for all).  All give bit-identical factors.  Same as the
  * CAPS_AMD_GEMM_KERNEL, CAPS_AMD_PANEL_SET and CAPS_AMD_NARROW_TILES
  * variables read at start-up.  Returns 1 for invalid values.  No
  * counterpart in the reference. */
